@@ -449,7 +449,7 @@ void xmi_detector_convolute_all_custom(xmi_inputFPtr inputFPtr, double **channel
  * the outputs: channels_conv[0..n_interactions_all] must each point to
  * nchannels doubles.  Device work runs on the null stream in a file-scope
  * device array of the library (one per device, at most 65536 channels:
- * 2.6 MB); calls that overlap on one device share it and race.  Returns 1 on
+ * 32 MB); calls that overlap on one device share it and race.  Returns 1 on
  * success, 0 with xmi_msim_last_error set (more channels than the maximum,
  * a NULL output, a device error, a pile-up train over 100 pulses). */
 int xmi_detector_convolute_all_noalloc(xmi_inputFPtr inputFPtr, double **channels_noconv, double **channels_conv,
