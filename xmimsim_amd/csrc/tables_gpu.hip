@@ -3,18 +3,18 @@
  *
  * The host generator (xmi_db.c, generator of src/xmi_data_f.F90:880-1551)
  * spends nearly all its time in four loops that are independent per output
- * value; here they run one thread per value:
- *   - angle inverse CDFs (src/xmi_data_f.F90:996-1073): one thread per
+ * value; here they run one thread per value or one workgroup per row:
+ *   - angle inverse CDFs (src/xmi_data_f.F90:996-1073): one workgroup per
  *     (element, Rayleigh|Compton, energy), the trapezoid CDF of
- *     DCS(theta) sin(theta) on 10000 points walked twice (total, inversion);
+ *     DCS(theta) sin(theta) on 10000 points in LDS, inverted by search;
  *   - total Compton-profile inverse CDF (src/xmi_data_f.F90:1131-1237): one
  *     thread per (element, random number), 100 bisection steps;
  *   - partial-profile inversions: one thread per (element, shell, point);
  *   - azimuth inverse CDF (src/xmi_data_f.F90:1483-1549): one thread per
  *     (t, random number).
- * Every thread runs the same routine of xrl_model.h as the host generator,
- * so the tables agree with the host's up to the rounding of the device's
- * math functions.  The host builds the light parts (grids, interaction
+ * The same formulas of xrl_model.h as the host generator's, so the tables
+ * agree with the host's up to the rounding of the device's math functions
+ * and of the order of the CDF's sums.  The host builds the light parts (grids, interaction
  * probabilities, yields, cascade cross sections) and allocates the arrays;
  * xmi_tables_fill_gpu fills the heavy ones.
  */
@@ -30,12 +30,83 @@
 #define TG_MAXPZ 100.0
 #define TG_CHUNK 16 /* elements per launch of the angle kernel (device memory) */
 
-__global__ void __launch_bounds__(256) k_theta_rows(const xrl_atom *atoms, int nz, const double *energies, int n_e,
-                                                    const double *rs, int n_r, double *out /* [nz][2][n_e][n_r] */) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nz * 2 * n_e) return;
-  const int z = t / (2 * n_e), kind = (t / n_e) & 1, j = t % n_e;
-  xrl_theta_icdf_row(&atoms[z], kind, energies[j], rs, n_r, TG_NTHETA_INT, out + (size_t)t * n_r, 1);
+/* cos(theta), sin(theta / 2) and sin(theta) of the CDF's points, shared by
+ * every row: [3][TG_NTHETA_INT] */
+__global__ void __launch_bounds__(256) k_theta_trig(double *trig) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= TG_NTHETA_INT) return;
+  const double th = k * (3.14159265358979323846 / (TG_NTHETA_INT - 1));
+  trig[k] = cos(th);
+  trig[TG_NTHETA_INT + k] = sin(th * 0.5);
+  trig[2 * TG_NTHETA_INT + k] = sin(th);
+}
+
+/* one workgroup per row (element, kind, energy), as xrl_theta_icdf_row: the
+ * integrand on every point into LDS, its cumulative trapezoid sums there
+ * (TG_SEG points per thread, an odd stride that keeps the threads' segments
+ * on different banks, and a scan of the segments' sums), then each random
+ * number's interval by binary search.  80 KB of LDS: two workgroups per CU.
+ * One thread per row, as before, was a chain of 2 x 10000 dependent
+ * evaluations on a few waves: 22 ms for one to sixteen elements. */
+#define TG_ROW_THREADS 512
+#define TG_SEG 21
+static_assert(TG_ROW_THREADS * TG_SEG >= TG_NTHETA_INT && TG_SEG % 2 == 1, "segments cover the row");
+__global__ void __launch_bounds__(TG_ROW_THREADS) k_theta_rows(const xrl_atom *atoms, const double *energies, int n_e,
+                                                               const double *rs, int n_r, const double *trig,
+                                                               double *out /* [nz][2][n_e][n_r] */) {
+  __shared__ double c[TG_NTHETA_INT];
+  __shared__ double wsum[TG_ROW_THREADS / 64];
+  const int row = blockIdx.x, z = row / (2 * n_e), kind = (row / n_e) & 1, tid = threadIdx.x;
+  const xrl_atom *a = &atoms[z];
+  const double E = energies[row % n_e], h = 3.14159265358979323846 / (TG_NTHETA_INT - 1);
+  for (int k = tid; k < TG_NTHETA_INT; k += TG_ROW_THREADS) {
+    const double cs = trig[k], sh = trig[TG_NTHETA_INT + k], sn = trig[2 * TG_NTHETA_INT + k];
+    c[k] = k == 0 ? 0.0 : (kind ? xrl_dcs_compt_t(a, E, cs, sh) : xrl_dcs_rayl_t(a, E, cs, sh)) * sn;
+  }
+  __syncthreads();
+  /* increments of the segment's points: 0.5 (f[k] + f[k - 1]) h */
+  const int k0 = tid * TG_SEG, k1 = min(TG_NTHETA_INT, k0 + TG_SEG);
+  const double before = k0 > 0 && k0 < TG_NTHETA_INT ? c[k0 - 1] : 0.0;
+  double own = 0.0, prev = before;
+  for (int k = k0; k < k1; k++) {
+    const double f = c[k];
+    own += k > 0 ? 0.5 * (f + prev) * h : 0.0;
+    prev = f;
+  }
+  double incl = own;
+  for (int off = 1; off < 64; off <<= 1) {
+    const double v = __shfl_up(incl, off);
+    if ((tid & 63) >= off) incl += v;
+  }
+  if ((tid & 63) == 63) wsum[tid >> 6] = incl;
+  __syncthreads(); /* and every thread has read the point before its segment */
+  double acc = incl - own;
+  for (int w = 0; w < (tid >> 6); w++) acc += wsum[w];
+  prev = before;
+  for (int k = k0; k < k1; k++) {
+    const double f = c[k];
+    acc += k > 0 ? 0.5 * (f + prev) * h : 0.0;
+    prev = f;
+    c[k] = acc;
+  }
+  __syncthreads();
+  const double total = c[TG_NTHETA_INT - 1];
+  for (int m = tid; m < n_r; m += TG_ROW_THREADS) {
+    const double target = rs[m] * total;
+    int lo = 1, hi = TG_NTHETA_INT - 1; /* first k >= 1 with c[k] >= target, the last point at most */
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (c[mid] < target) lo = mid + 1;
+      else hi = mid;
+    }
+    const double c0 = c[lo - 1], c1 = c[lo];
+    double fr = (c1 > c0) ? (target - c0) / (c1 - c0) : 0.0;
+    fr = fr < 0.0 ? 0.0 : (fr > 1.0 ? 1.0 : fr);
+    double v = ((lo - 1) + fr) * h;
+    if (m == 0) v = 0.0;
+    if (m == n_r - 1) v = 3.14159265358979323846;
+    out[(size_t)row * n_r + m] = v;
+  }
 }
 
 __global__ void __launch_bounds__(256) k_profile_total(const xrl_atom *atoms, int nz, const double *cmax,
@@ -150,13 +221,15 @@ extern "C" int xmi_tables_fill_gpu(xmi_hdf5_ZF *zs, int n, xmi_hdf5F *h) {
     {
       const int chunk = n < TG_CHUNK ? n : TG_CHUNK;
       const size_t row = (size_t)n_e * n_r;
-      DBuf d_out;
+      DBuf d_out, d_trig;
       TG_TRY(d_out.alloc(sizeof(double) * chunk * 2 * row));
+      TG_TRY(d_trig.alloc(sizeof(double) * 3 * TG_NTHETA_INT));
+      hipLaunchKernelGGL(k_theta_trig, dim3(blocks_for(TG_NTHETA_INT)), dim3(256), 0, 0, d_trig.as<double>());
+      TG_TRY(hipGetLastError());
       for (int z0 = 0; z0 < n; z0 += chunk) {
         const int nz = (n - z0) < chunk ? (n - z0) : chunk;
-        hipLaunchKernelGGL(k_theta_rows, dim3(blocks_for((size_t)nz * 2 * n_e)), dim3(256), 0, 0,
-                           d_atoms.as<xrl_atom>() + z0, nz, d_E.as<double>(), n_e, d_rs.as<double>(), n_r,
-                           d_out.as<double>());
+        hipLaunchKernelGGL(k_theta_rows, dim3(nz * 2 * n_e), dim3(TG_ROW_THREADS), 0, 0, d_atoms.as<xrl_atom>() + z0,
+                           d_E.as<double>(), n_e, d_rs.as<double>(), n_r, d_trig.as<double>(), d_out.as<double>());
         TG_TRY(hipGetLastError());
         for (int z = 0; z < nz; z++) {
           TG_TRY(hipMemcpy(zs[z0 + z].RayleighTheta_ICDF, d_out.as<double>() + (size_t)(2 * z) * row,

@@ -239,18 +239,25 @@ XRL_FN double xrl_sf_compt(const xrl_atom *a, double x) {
   return (double)a->Z * (1.0 - 1.0 / (d * d));
 }
 
-/* unpolarised differential cross sections, cm2/g/sr */
-XRL_FN double xrl_dcs_rayl(const xrl_atom *a, double E, double theta) {
-  double c = cos(theta);
-  double F = xrl_ff_rayl(a, xrl_moment_transf(E, theta));
+/* unpolarised differential cross sections, cm2/g/sr, from c = cos(theta)
+ * and sh = sin(theta / 2) */
+XRL_FN double xrl_dcs_rayl_t(const xrl_atom *a, double E, double c, double sh) {
+  double F = xrl_ff_rayl(a, E / XRL_KEV_ANGSTROM * sh);
   return XRL_RE2 * 0.5 * (1.0 + c * c) * F * F * a->barn_per_A;
 }
 
-XRL_FN double xrl_dcs_compt(const xrl_atom *a, double E, double theta) {
-  double c = cos(theta);
+XRL_FN double xrl_dcs_compt_t(const xrl_atom *a, double E, double c, double sh) {
   double k = 1.0 / (1.0 + E / XRL_MEC2 * (1.0 - c));
   double kn = XRL_RE2 * 0.5 * k * k * (k + 1.0 / k - (1.0 - c * c));
-  return kn * xrl_sf_compt(a, xrl_moment_transf(E, theta)) * a->barn_per_A;
+  return kn * xrl_sf_compt(a, E / XRL_KEV_ANGSTROM * sh) * a->barn_per_A;
+}
+
+XRL_FN double xrl_dcs_rayl(const xrl_atom *a, double E, double theta) {
+  return xrl_dcs_rayl_t(a, E, cos(theta), sin(theta * 0.5));
+}
+
+XRL_FN double xrl_dcs_compt(const xrl_atom *a, double E, double theta) {
+  return xrl_dcs_compt_t(a, E, cos(theta), sin(theta * 0.5));
 }
 
 /* linearly polarised differential cross sections (DCSP_*), cm2/g/sr.  The
