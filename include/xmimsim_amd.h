@@ -328,8 +328,8 @@ typedef struct _xmi_msim_launch {
   int batch_log2; /* histories per batch 2^batch_log2, 12..21 (default 21) */
   int use_graph;  /* 1: capture one batch's launches in a HIP graph, replayed per batch; each replay pops its
                      batch from a device batch queue */
-  int lines_kp;   /* photons per lane of the estimator's line kernel: 2..4 up to 4 layers (default 3),
-                     1..2 up to 8 (default 2), 1 beyond */
+  int lines_kp;   /* photons per lane of the estimator's line kernel: 2..4 up to 4 layers (default 4 up to 3
+                     layers, else 3), 1..3 with 5 layers (default 3), 1..2 up to 8 (default 2), 1 beyond */
   int wg_per_cu;  /* resident workgroups per CU of the estimator's grid-stride kernels (default: occupancy) */
 } xmi_msim_launch;
 int xmi_msim_set_launch(const xmi_msim_launch *launch); /* 0 and an error message for a shape out of range */

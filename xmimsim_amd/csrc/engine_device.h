@@ -63,7 +63,7 @@ struct VrSoA {
   double *theta, *phi;          /* scattering angle to the detector point, azimuth to the polarisation */
   double *omega;                /* solid angle of the detector */
   double *pesc;                 /* escape probability at the photon energy */
-  double *dist;                 /* [NL][cap] path in the k-th layer crossed (k = 0: own layer) */
+  double *dist;                 /* [NL][cap] path by layer, 0 where not crossed */
   double *sar, *sat;            /* off-grid point (r, theta) for the cone estimate */
   int *info;                    /* bit 0 active, bit 1 upwards, bits 8.. layers crossed */
   unsigned int *blk;            /* estimator stream position (Philox block) after the solid angle */
@@ -163,7 +163,8 @@ struct EngineParams {
   int fl_off[ENG_MAX_LAYERS + 1];
   const int4 *fl_info;          /* {u, q, shell, compact bin} */
   const double *fl_wf;          /* weight fraction of u in the layer * yield * rate */
-  const double *fl_mr;          /* [entry][layer bound of the kernels] mu*rho of the line per layer, 0 past the stack */
+  const double *fl_ent;         /* [entry][layer bound of the kernels + 1]: {element, shell} in one word, then -mu*rho of
+                                   the line per layer in units of ENG_EXP_UNIT, 0 past the stack */
   const int *lbin_g;            /* compact bin -> u * ENG_MAX_ACT + q */
   int n_lbins;
   /* azimuth and solid angle */
@@ -208,7 +209,7 @@ struct EngineParams {
   int *lay_list;                /* [n_layers][cap] */
   int *lay_woff;                /* [n_layers][n_waves]: per-wave counts, then exclusive offsets */
   int *lay_total;               /* [n_layers] entries of each list */
-  int *lay_segbase;             /* [16][32] segment totals, then offsets of the per-wave scan */
+  int *lay_segbase;             /* [16][ENG_SCAN_NSEG] segment totals, then offsets of the per-wave scan */
   int n_waves;                  /* row length of lay_woff: waves of a one-thread-per-slot launch over cap */
   int cap;
 };

@@ -270,7 +270,7 @@ struct Engine {
   int sa_nr = 0, sa_nt = 0;
   /* per-call buffers (grow only) */
   DevBuf el_Z, el_w, el_u, precalc_mu, act_n, act_line, act_shell, act_factor, act_E, act_ch, act_murho;
-  DevBuf fl_info, fl_wf, fl_mr, lbin_g;
+  DevBuf fl_info, fl_wf, fl_ent, lbin_g;
   DevBuf lay_rc, lay_edge, lay_pb, lay_kstart, lay_cell, el_cell;
   DevBuf src_desc, src_line_mus, exc_layers, exc_atoms;
   DevBuf state, vr, tallies, counters, queue, lay_list, lay_woff, lay_total, lay_segbase, cone_acc, esc_tally;
@@ -791,8 +791,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
   P.n_lbins = act_base[nZ];
   std::vector<int4> fl_info;
   std::vector<double> fl_wf;
-  std::vector<double> fl_mr;
-  const int fl_stride = NL <= 1 ? 1 : NL <= 2 ? 2 : NL <= 4 ? 4 : NL <= 8 ? 8 : 16;
+  std::vector<double> fl_ent;
+  const int fl_stride = eng_layer_bound(NL);
   for (int l = 0; l < NL; l++) {
     P.fl_off[l] = (int)fl_info.size();
     for (int k = 0; k < P.layer_nel[l]; k++) {
@@ -801,17 +801,25 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
         size_t o = (size_t)u * ENG_MAX_ACT + q;
         fl_info.push_back(make_int4(u, q, acts[o], act_base[u] + q));
         fl_wf.push_back(elW[(size_t)P.layer_off[l] + k] * actf[o]);
-        /* padded to the kernels' layer bound, zeros past the stack */
+        /* {element, shell} in one word, then the attenuation padded to the
+         * kernels' layer bound, zeros past the stack; in units of the line
+         * kernel's table exponential */
+        const uint64_t uz = (uint64_t)(uint32_t)u | ((uint64_t)(uint32_t)acts[o] << 32);
+        double word;
+        memcpy(&word, &uz, sizeof(word));
+        fl_ent.push_back(word);
         for (int l2 = 0; l2 < fl_stride; l2++)
-          fl_mr.push_back(l2 < NL ? actm[((size_t)l2 * nZ + u) * ENG_MAX_ACT + q] : 0.0);
+          fl_ent.push_back(l2 < NL ? -ENG_EXP_UNIT * actm[((size_t)l2 * nZ + u) * ENG_MAX_ACT + q] : 0.0);
       }
     }
   }
   P.fl_off[NL] = (int)fl_info.size();
-  /* one zero entry past the end: the walk reads entry t + 1 ahead of use */
-  fl_info.push_back(make_int4(0, 0, 0, 0));
-  fl_wf.push_back(0.0);
-  for (int l2 = 0; l2 < fl_stride; l2++) fl_mr.push_back(0.0);
+  /* two zero entries past the end: the walk reads entry t + 2 ahead of use */
+  for (int k = 0; k < 2; k++) {
+    fl_info.push_back(make_int4(0, 0, 0, 0));
+    fl_wf.push_back(0.0);
+    for (int l2 = 0; l2 <= fl_stride; l2++) fl_ent.push_back(0.0);
+  }
 
   /* sources: continuous intervals, then discrete lines */
   std::vector<SourceDesc> src;
@@ -933,7 +941,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       d.run0 = (uint64_t)total_hist;
       total_hist += (d.valid && d.count > 0) ? d.count : 0;
     }
-    const int cap_max = 1 << (g_launch.batch_log2 ? g_launch.batch_log2 : 21);
+    const int cap_max = 1 << (g_launch.batch_log2 ? g_launch.batch_log2 : ENG_BATCH_LOG2);
     int cap = (int)(total_hist < cap_max ? (total_hist > 0 ? total_hist : 1) : cap_max);
     /* a brute-force run with cascades keeps a second slot per primary for
      * the offspring photon of its cascade */
@@ -942,7 +950,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.off_half = (brute && P.casc) ? cap : 0;
     size_t per = (size_t)slots;
     /* the kernels' layer-count bound (estimator records hold nl_bound paths) */
-    const int nl_bound = NL <= 1 ? 1 : NL <= 2 ? 2 : NL <= 4 ? 4 : NL <= 8 ? 8 : 16;
+    const int nl_bound = eng_layer_bound(NL);
     size_t state_bytes = per * (15 * sizeof(double) + (size_t)NL * sizeof(double) + 5 * sizeof(int) + sizeof(uint64_t));
     size_t vr_bytes = per * ((6 + (size_t)nl_bound) * sizeof(double) + 2 * sizeof(int));
     size_t n_ch2 = (size_t)n_int * nch * 2, n_line2 = (size_t)n_int * nZ * ENG_MAX_ACT * 2, n_rc2 = (size_t)n_int * nZ * 4;
@@ -982,14 +990,15 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     /* layer lists: a row of cap slots per layer; per-wave offsets of the
      * k_step launch (ceil(cap / ENG_BLOCK) workgroups of ENG_BLOCK / 64 waves) */
     P.n_waves = step_waves;
-    if (!brute && step_waves > 32 * 1024) {
-      xmi_set_error("xmi_main_msim: %d waves per batch exceed the layer scan's 32768", step_waves);
+    if (!brute && step_waves > ENG_SCAN_SEG * ENG_SCAN_NSEG) {
+      xmi_set_error("xmi_main_msim: %d waves per batch exceed the layer scan's %d", step_waves,
+                    ENG_SCAN_SEG * ENG_SCAN_NSEG);
       return 0;
     }
     HIP_TRY(G.lay_list.ensure((size_t)NL * cap * sizeof(int)));
     HIP_TRY(G.lay_woff.ensure((size_t)NL * step_waves * sizeof(int)));
     HIP_TRY(G.lay_total.ensure((size_t)ENG_MAX_LAYERS * sizeof(int)));
-    HIP_TRY(G.lay_segbase.ensure((size_t)ENG_MAX_LAYERS * 32 * sizeof(int)));
+    HIP_TRY(G.lay_segbase.ensure((size_t)ENG_MAX_LAYERS * ENG_SCAN_NSEG * sizeof(int)));
     /* off-grid cone accumulators: zero here, and cleared again by the
      * kernel after each photon's estimate */
     {
@@ -1013,7 +1022,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       up.add(G.act_murho, actm.data(), actm.size());
       up.add(G.fl_info, fl_info.data(), fl_info.size());
       up.add(G.fl_wf, fl_wf.data(), fl_wf.size());
-      up.add(G.fl_mr, fl_mr.data(), fl_mr.size());
+      up.add(G.fl_ent, fl_ent.data(), fl_ent.size());
       up.add(G.lbin_g, lbin_g.data(), lbin_g.size());
       up.add(G.lay_rc, lay_rc.data(), lay_rc.size());
       up.add(G.lay_edge, lay_edge.data(), lay_edge.size());
@@ -1078,7 +1087,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.act_murho = G.act_murho.as<double>();
     P.fl_info = G.fl_info.as<int4>();
     P.fl_wf = G.fl_wf.as<double>();
-    P.fl_mr = G.fl_mr.as<double>();
+    P.fl_ent = G.fl_ent.as<double>();
     P.lbin_g = G.lbin_g.as<int>();
     P.lay_rc = G.lay_rc.as<double>();
     P.lay_edge = G.lay_edge.as<double>();

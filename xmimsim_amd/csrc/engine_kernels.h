@@ -33,12 +33,31 @@
 #define ENG_CNT_HITS (ENG_CNT_ERR_SOURCE + 4)     /* brute force: photons that reached the detector */
 #define ENG_NCOUNTERS (ENG_CNT_ERR_SOURCE + 5)
 
+/* histories per batch unless the launch shape says otherwise: every kernel of
+ * an order ends with a part-filled round of workgroups, and the scan, list
+ * and reset launches cost the same for any size, so the batch is as large as
+ * 0.6 GB of photon records (three layers) make it */
+#define ENG_BATCH_LOG2 21
+/* segments of the per-wave layer-count scan (k_layer_scan, d_layer_list):
+ * the waves of the largest batch, one thread per slot */
+#define ENG_SCAN_SEG 1024
+#define ENG_SCAN_NSEG 128
+static_assert((1 << ENG_BATCH_LOG2) / 64 <= ENG_SCAN_SEG * ENG_SCAN_NSEG, "the layer scan covers a batch");
+
+/* the line kernel's exponential: table entries, and units of its exponents
+ * (512 / ln 2 per unit of attenuation) */
+#define ENG_EXP_N 512
+#define ENG_EXP_UNIT 738.6598609351493
+
 /* events recorded per order when profiling: start, after the step, after
  * each of the four estimator kernels, after the interactions */
 #define ENG_ORDER_EVENTS 7
 
 /* m_e c^2 in keV as the reference computes it (src/xmi_main.F90:48-55) */
 #define ENG_MEC2 (9.10938188e-31 * 2.99792458e8 * 2.99792458e8 / 1.602176487e-19 / 1000.0)
+
+/* the kernels' layer-count bound: the smallest instance that holds n layers */
+static inline int eng_layer_bound(int n) { return n <= 5 ? (n < 1 ? 1 : n) : n <= 8 ? 8 : 16; }
 
 struct SourceDesc {
   int kind;               /* 0 = continuous interval, 1 = discrete line */

@@ -32,9 +32,6 @@
 
 #include "engine_kernels.h"
 
-/* segments of the per-wave layer-count scan (k_layer_scan, d_layer_list) */
-#define ENG_SCAN_SEG 1024
-#define ENG_SCAN_NSEG 32
 
 /* ------------------------------------------------------------------------ */
 /* physics helpers on the device */
@@ -719,32 +716,37 @@ __device__ __forceinline__ int d_vr_geom(const EngineParams &P, const PhotonSoA 
     const int up = d_dot(nd, P.n_sample) > 0.0;
     const int dir = up ? 1 : -1;
     const int ncross = up ? P.n_layers - cur + 1 : cur;
-    /* path to the detector through the layers, in crossing order; the
-     * layer holding the detector point ends the walk */
+    /* path to the detector through the layers, by layer (0 where not
+     * crossed); the layer holding the detector point ends the walk */
     double tc[3] = {coords[0], coords[1], coords[2]};
     int done = 0, nc = 0;
     double murhod = 0.0;
 #pragma unroll
     for (int k = 0; k < NL; k++) {
+      const int l0 = cur - 1 + k * dir, back = cur - 2 - k;
       double dd = 0.0;
-      if (k < ncross && !done) {
-        const int l0 = cur - 1 + k * dir;
-        double pp[3] = {0.0, 0.0, up ? P.layer_ze[l0] : P.layer_zb[l0]}, ip[3];
-        d_intersect(pp, P.n_sample, tc, nd, ip);
-        dd = d_distance(tc, ip);
-        if (dd > total_distance) {
-          dd = total_distance;
-          done = 1;
-        } else {
-          tc[0] = ip[0];
-          tc[1] = ip[1];
-          tc[2] = ip[2];
-          total_distance -= dd;
+      if (k < ncross) {
+        if (!done) {
+          double pp[3] = {0.0, 0.0, up ? P.layer_ze[l0] : P.layer_zb[l0]}, ip[3];
+          d_intersect(pp, P.n_sample, tc, nd, ip);
+          dd = d_distance(tc, ip);
+          if (!(dd <= total_distance)) {
+            dd = total_distance;
+            done = 1;
+          } else {
+            tc[0] = ip[0];
+            tc[1] = ip[1];
+            tc[2] = ip[2];
+            total_distance -= dd;
+          }
+          murhod += S.mus[(size_t)l0 * cap + i] * P.layer_density[l0] * dd;
+          nc = k + 1;
         }
-        murhod += S.mus[(size_t)l0 * cap + i] * P.layer_density[l0] * dd;
-        nc = k + 1;
+        V.dist[(size_t)l0 * cap + i] = dd;
       }
-      V.dist[(size_t)k * cap + i] = dd;
+      /* the layers on the other side of the point's own */
+      const int other = up ? back : cur + k;
+      if (up ? back >= 0 : other < P.n_layers) V.dist[(size_t)other * cap + i] = 0.0;
     }
     /* solid angle, src/xmi_solid_angle_f.F90:712-801 */
     double omega = 0.0;
@@ -919,18 +921,24 @@ __global__ void __launch_bounds__(ENG_SCAN_SEG) k_layer_scan(EngineParams P, int
   if (threadIdx.x == ENG_SCAN_SEG - 1) P.lay_segbase[L0 * ENG_SCAN_NSEG + seg] = base + incl;
 }
 
-/* segment totals -> segment offsets, and each layer's total (one lane per
- * layer) */
-__global__ void k_layer_base(EngineParams P, int nseg) {
-  const int L0 = threadIdx.x;
-  if (L0 >= P.n_layers) return;
-  int run = 0;
-  for (int s = 0; s < nseg; s++) {
-    const int t = P.lay_segbase[L0 * ENG_SCAN_NSEG + s];
-    P.lay_segbase[L0 * ENG_SCAN_NSEG + s] = run;
-    run += t;
+/* segment totals -> segment offsets, and each layer's total: one workgroup
+ * of ENG_SCAN_NSEG threads per layer */
+__global__ void __launch_bounds__(ENG_SCAN_NSEG) k_layer_base(EngineParams P, int nseg) {
+  __shared__ int first;
+  const int L0 = blockIdx.x, s = threadIdx.x, lane = s & 63;
+  int *seg = P.lay_segbase + L0 * ENG_SCAN_NSEG;
+  const int v = s < nseg ? seg[s] : 0;
+  int incl = v;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(incl, off);
+    if (lane >= off) incl += t;
   }
-  P.lay_total[L0] = run;
+  if (s == 63) first = incl;
+  __syncthreads();
+  if (s >= 64) incl += first;
+  if (s < nseg) seg[s] = incl - v;
+  if (s == ENG_SCAN_NSEG - 1) P.lay_total[L0] = incl;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -952,9 +960,8 @@ __global__ void k_layer_base(EngineParams P, int nseg) {
  *                 (element, fluorescence line) entries with the line data in
  *                 scalar registers and sums each line's terms over its photons
  *
- * Path lengths are kept in crossing order (k = 0: the photon's own layer) so
- * that register arrays have compile-time indices only (NL bounds the layer
- * count).  Tallies are 128-bit fixed point, privatised in LDS when they fit;
+ * Path lengths are kept by layer, 0 where the path does not cross it, so that
+ * register arrays have compile-time indices only (NL bounds the layer count).  Tallies are 128-bit fixed point, privatised in LDS when they fit;
  * integer adds commute, so totals do not depend on the order of the adds. */
 
 __device__ __forceinline__ double d_wave_sum(double v) {
@@ -1024,6 +1031,37 @@ __device__ __forceinline__ double d_exp_neg(double x, const double *tab) {
   return ldexp(fma(T, p, T), ni >> 6);
 }
 
+
+/* reciprocal square root of x > 0 far from the ends of the range: the
+ * hardware's estimate (2^-24 or better) and one third-order step */
+__device__ __forceinline__ double d_rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+/* E^-p of the photo-ionisation cross sections (p = 11/4) for an energy in the
+ * provider's range: E^(-1/2) cubed twice times E^(1/4), from two reciprocal
+ * square roots; 0 for E <= 0, as xrl_energy */
+static_assert(XRL_PHOTO_EXPONENT == 2.75, "d_photo_pe forms E^-11/4");
+__device__ __forceinline__ double d_photo_pe(double E) {
+  const double a = d_rsqrt_pos(E), a2 = a * a;
+  return E > 0.0 ? a2 * a2 * (a2 * d_rsqrt_pos(a)) : 0.0;
+}
+
+/* e^-m from t = -m ENG_EXP_UNIT, for a factor that tables and coefficients
+ * hold in these units: t = 512 k + j + f with |f| <= 1/2, so the value is
+ * 2^k * tab[j] * 2^(f/512), tab[j] = 2^(j/512) in LDS (4 KB) and the last
+ * factor minus 1 its Taylor polynomial of degree 4 (1.2e-18); two
+ * instructions fewer than the 64-entry table's reduction and degree 5, and
+ * the unit saves the scaling and the clamp: ldexp underflows to 0 by itself */
+__device__ __forceinline__ double d_exp_unit_poly(double f) {
+  constexpr double h = 0.6931471805599453 / ENG_EXP_N;
+  double p = fma(f, h * h * h * h / 24.0, h * h * h / 6.0);
+  p = fma(f, p, h * h / 2.0);
+  p = fma(f, p, h);
+  return f * p;
+}
 
 /* persistent: the off-grid queue's photons (entries flattened over the
  * ENG_SPREAD sub-queues) times ENG_CONE_SEGS(hits) segments of
@@ -1285,9 +1323,9 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
     /* per-photon factors, shared by every element of the layer */
     double E = 0.0, wo = 0.0, pesc = 0.0, inv_mu = 0.0, c_lamb0 = 1.0, A0 = 0.0, A1 = 0.0, th_e = 0.0;
     phx_stream sd; /* advanced model: uniforms from the same stream position */
-    /* rho * path in the k-th layer crossed: in registers for up to four
+    /* rho * path by layer (0 where not crossed): in registers for up to five
      * layers, read from the records beyond (register budget) */
-    constexpr int NR = NL <= 4 ? NL : 1;
+    constexpr int NR = NL <= 5 ? NL : 1;
     double rd[NR];
     xrl_dcsp_ctx dc = {0.0, 0.0, 0.0};
     int dir = 1, nc = 0, ch_r = -1;
@@ -1302,10 +1340,10 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
       inv_mu = 1.0 / S.mus[(size_t)(L - 1) * cap + i];
       dir = (info & VR_UP) ? 1 : -1;
       nc = info >> VR_NC_SHIFT;
-      if (NL <= 4) {
+      if (NL <= 5) {
 #pragma unroll
-        for (int k = 0; k < NR; k++)
-          if (k < nc) rd[k] = P.layer_density[L - 1 + k * dir] * V.dist[(size_t)k * cap + i];
+        for (int l = 0; l < NR; l++)
+          if (l < P.n_layers) rd[l] = P.layer_density[l] * V.dist[(size_t)l * cap + i];
       }
       /* the estimator stream from the block after the geometry and cone
        * draws, as words */
@@ -1386,10 +1424,16 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
           if (!(energy > 0.0)) continue;
           const xrl_ectx ce = xrl_energy(energy);
           double m2 = 0.0;
+          if (NL <= 5) {
+#pragma unroll
+            for (int l = 0; l < NR; l++)
+              if (rd[l] > 0.0) m2 += d_layer_mu_tab(P, l, &ce) * rd[l];
+          } else {
 #pragma unroll 1
-          for (int kk = 0; kk < nc; kk++) {
-            const int l0 = L - 1 + kk * dir;
-            m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)kk * cap + i]);
+            for (int kk = 0; kk < nc; kk++) {
+              const int l0 = L - 1 + kk * dir;
+              m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)l0 * cap + i]);
+            }
           }
           const double tw = dcw * d_exp_neg(-m2, exp_tab) * sw;
           twc += tw;
@@ -1428,15 +1472,15 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
         {
           const xrl_ectx ce = xrl_energy(energy);
           double m2 = 0.0;
-          if (NL <= 4) {
+          if (NL <= 5) {
 #pragma unroll
-            for (int kk = 0; kk < NR; kk++)
-              if (kk < nc) m2 += d_layer_mu_tab(P, L - 1 + kk * dir, &ce) * rd[kk];
+            for (int l = 0; l < NR; l++)
+              if (rd[l] > 0.0) m2 += d_layer_mu_tab(P, l, &ce) * rd[l];
           } else {
 #pragma unroll 1
             for (int kk = 0; kk < nc; kk++) {
               const int l0 = L - 1 + kk * dir;
-              m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)kk * cap + i]);
+              m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)l0 * cap + i]);
             }
           }
           twc = Pconv * (xrl_dcsp_compt_c(a, &dc) * wo) * d_exp_neg(-m2, exp_tab);
@@ -1469,7 +1513,14 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
   }
 }
 
-/* lines phase: KP photons per lane, a chunk of 64 KP photons (all in layer
+/* Bound by vector issue of the pairs (line, photon): 15 instructions each
+ * with three layers (three for the attenuation, rint, difference, conversion,
+ * two for the table's index, four for the polynomial, one each for the table,
+ * the exponent and the sum).  2^21 histories of the three-layer tube run took
+ * 250 us with the 64-entry table, four-layer rows and one entry loaded ahead
+ * of its use, 230 now.
+ *
+ * lines phase: KP photons per lane, a chunk of 64 KP photons (all in layer
  * L); the wavefront walks the layer's (element, line) entries.  Per (line t,
  * photon) term
  *   wf_t * P_shell(t, photon) * g * exp(-sum_l mu_rho(t, l) * d_l)
@@ -1490,14 +1541,14 @@ template <int NL, int KP, bool use_lds>
 __global__ void __launch_bounds__(ENG_BLOCK) k_vr_lines(EngineParams P, PhotonSoA S, VrSoA V, int n) {
   /* LDS tallies (when they fit): compact line bins [n_lbins][2] */
   extern __shared__ unsigned long long lds[];
-  __shared__ double exp_tab[64];
+  __shared__ double exp_tab[ENG_EXP_N];
   /* per wavefront: the lanes' terms of 8 lines, row j = line j of the group */
   __shared__ double lred[ENG_BLOCK / 64][8 * ENG_LRED_STRIDE];
   const size_t n_line2 = (size_t)P.n_lbins * 2;
   const size_t cap = (size_t)P.cap;
   unsigned long long *gline = P.t_line + (size_t)(n - 1) * P.nZ * ENG_MAX_ACT * 2;
   unsigned long long *tline = gline;
-  if (threadIdx.x < 64) exp_tab[threadIdx.x] = exp2((double)threadIdx.x / 64.0);
+  for (int k = threadIdx.x; k < ENG_EXP_N; k += ENG_BLOCK) exp_tab[k] = exp2((double)k / ENG_EXP_N);
   if (use_lds) {
     tline = lds;
     for (size_t k = threadIdx.x; k < n_line2; k += blockDim.x) lds[k] = 0ull;
@@ -1514,40 +1565,36 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_vr_lines(EngineParams P, PhotonSo
     const int L = lc.L;
     /* the lane's KP photons: list entries e0, e0 + 64, ... of layer L */
     const int e0 = (int)((c - lc.c_begin) * (64 * KP)) + __lane_id();
-    double E[KP], pe[KP], g[KP], x[KP];
+    double E[KP], g[KP], x[KP];
     /* path length per layer, by layer index (0 where not crossed) */
     double dl[KP][NL];
-    int act[KP], fo[KP], pl[KP], pu[KP], kE[KP];
+    int fo[KP], px[KP], kE[KP];
     int any_act = 0;
 #pragma unroll
     for (int k = 0; k < KP; k++) {
       const int e = e0 + 64 * k;
       const int i = e < lc.tot ? P.lay_list[(size_t)(L - 1) * cap + e] : 0;
       const int info = e < lc.tot ? V.info[i] : 0;
-      act[k] = info & VR_ACTIVE;
-      any_act |= act[k];
+      const int act = info & VR_ACTIVE;
+      any_act |= act;
       E[k] = 2.0;
-      pe[k] = g[k] = x[k] = 0.0;
+      g[k] = x[k] = 0.0;
       fo[k] = 1;
-      pl[k] = pu[k] = kE[k] = 0;
+      px[k] = kE[k] = 0;
 #pragma unroll
       for (int l = 0; l < NL; l++) dl[k][l] = 0.0;
-      if (act[k]) {
+      if (act) {
         E[k] = S.energy[i];
-        pe[k] = xrl_energy(E[k]).pe;
         g[k] = V.omega[i] / 4.0 / ENG_PI * S.weight[i] / S.mus[(size_t)(L - 1) * cap + i];
-        pl[k] = S.prev_line[i];
-        pu[k] = S.prev_u[i];
-        fo[k] = !(n > 1 && pl[k] > 0);
-        const int nc = info >> VR_NC_SHIFT, dir = (info & VR_UP) ? 1 : -1;
+        const int pl = S.prev_line[i];
+        fo[k] = !(n > 1 && pl > 0);
+        /* E^-p goes with the weight factor; a fluorescence photon has its
+         * place in the rows of the cascade table instead */
+        if (fo[k]) g[k] *= d_photo_pe(E[k]);
+        else px[k] = S.prev_u[i] * XMI_NLINES_VR_DEV + (pl - 1);
 #pragma unroll
-        for (int q = 0; q < NL; q++) {
-          const double d = q < nc ? V.dist[(size_t)q * cap + i] : 0.0;
-          const int l0 = L - 1 + q * dir;
-#pragma unroll
-          for (int l = 0; l < NL; l++)
-            if (q < nc && l == l0) dl[k][l] = d;
-        }
+        for (int l = 0; l < NL; l++)
+          if (l < P.n_layers) dl[k][l] = V.dist[(size_t)l * cap + i];
       }
     }
     if (__ballot(any_act) == 0ull) continue;
@@ -1555,28 +1602,30 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_vr_lines(EngineParams P, PhotonSo
     int u_cur = -1, z_cur = -1, any = 0;
     double *wred = lred[threadIdx.x >> 6];
     const int lane = __lane_id();
-    const auto *fl_info = d_const((const int *)P.fl_info);
-    const auto *fl_wf = d_const(P.fl_wf);
-    const auto *fl_mr = d_const(P.fl_mr);
-    /* the next entry's scalars are loaded one iteration ahead (the tables
-     * end with a zero entry), so that their latency overlaps this entry's
-     * arithmetic */
-    int nx_u = fl_info[4 * t0], nx_z = fl_info[4 * t0 + 2];
-    double nx_wf = fl_wf[t0], nx_mr[NL];
+    /* the entries' scalars come two ahead, in two buffers by the entry's
+     * parity (the tables end with two zero entries; one rotated buffer would
+     * copy, and so wait for, what was just asked for).  Scalar and LDS loads
+     * complete out of order with each other, so a wait for an LDS value waits
+     * for every scalar load under way: they are issued behind an entry's LDS
+     * reads, where the next wait is a whole entry's arithmetic away.  Two
+     * buffers of more than four layers would not fit the scalar registers:
+     * there the next entry's are issued first */
+    constexpr int AH = NL <= 4 ? 2 : 1;
+    const auto *ent = d_const(P.fl_ent) + (size_t)t0 * (NL + 1);
+    double nx[AH][NL + 1]; /* {element, shell} packed, attenuation by layer */
+    auto fetch = [&](double *to, int t) {
 #pragma unroll
-    for (int l = 0; l < NL; l++) nx_mr[l] = fl_mr[(size_t)t0 * NL + l];
-    for (int t = t0; t < t1; t++) {
-      /* {element, active line, shell, compact bin} */
-      const int2 it = make_int2(nx_u, nx_z);
-      const double wf = nx_wf;
+      for (int l = 0; l <= NL; l++) to[l] = ent[(t - t0) * (NL + 1) + l];
+    };
+#pragma unroll
+    for (int a = 0; a < AH; a++) fetch(nx[a], t0 + a);
+    auto entry = [&](double *buf, int t) {
+      const long long uz = __double_as_longlong(buf[0]);
+      const int2 it = make_int2((int)uz, (int)(uz >> 32));
       double mr[NL];
 #pragma unroll
-      for (int l = 0; l < NL; l++) mr[l] = nx_mr[l];
-      nx_u = fl_info[4 * (t + 1)];
-      nx_z = fl_info[4 * (t + 1) + 2];
-      nx_wf = fl_wf[t + 1];
-#pragma unroll
-      for (int l = 0; l < NL; l++) nx_mr[l] = fl_mr[(size_t)(t + 1) * NL + l];
+      for (int l = 0; l < NL; l++) mr[l] = buf[l + 1];
+      if (AH == 1) fetch(buf, t + 1);
       if (it.x != u_cur) {
         /* edges of the element above each photon's energy */
         const auto *a = d_const(&P.atoms[it.x]);
@@ -1592,39 +1641,46 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_vr_lines(EngineParams P, PhotonSo
       if (it.y != z_cur) {
         z_cur = it.y;
         int nz = 0;
+        const double *sc = &P.atoms[u_cur].shell_C[P.cascade - 1][0][z_cur];
+        const double *pc = P.precalc_xrf + ((size_t)u_cur * 9 + z_cur) * P.nZ * XMI_NLINES_VR_DEV;
 #pragma unroll
         for (int k = 0; k < KP; k++) {
           double v;
-          if (fo[k]) {
-            v = (!P.use_M_lines && z_cur >= 4) ? 0.0 : pe[k] * P.atoms[u_cur].shell_C[P.cascade - 1][kE[k]][z_cur];
-          } else {
-            v = z_cur <= smax ? P.precalc_xrf[(((size_t)u_cur * 9 + z_cur) * P.nZ + pu[k]) * XMI_NLINES_VR_DEV +
-                                              (pl[k] - 1)]
-                              : 0.0;
-          }
+          if (fo[k]) v = (!P.use_M_lines && z_cur >= 4) ? 0.0 : sc[9 * kE[k]];
+          else v = z_cur <= smax ? pc[px[k]] : 0.0;
           /* shell factor times the photon's weight factor; 0 for lanes
            * without a photon, so that their terms vanish */
-          x[k] = act[k] ? v * g[k] : 0.0;
+          x[k] = v * g[k];
           nz |= x[k] != 0.0;
         }
         any = __ballot(nz) != 0ull;
       }
       const int j = (t - t0) & 7;
-      double part = 0.0;
+      double acc = 0.0;
       if (any) {
-        /* attenuation rows are padded to NL entries (zeros past the stack);
-         * the lane's photons are summed before the wavefront sum */
-        double acc = 0.0;
+        /* attenuation rows are padded to NL entries (zeros past the stack),
+         * in units of the table exponential; the lane's photons are summed
+         * before the wavefront sum */
+        double T[KP], p[KP];
+        int ni[KP];
 #pragma unroll
         for (int k = 0; k < KP; k++) {
-          double m2 = 0.0;
+          double m = mr[0] * dl[k][0];
 #pragma unroll
-          for (int l = 0; l < NL; l++) m2 += mr[l] * dl[k][l];
-          acc = fma(x[k], d_exp_neg(-m2, exp_tab), acc);
+          for (int l = 1; l < NL; l++) m = fma(mr[l], dl[k][l], m);
+          const double r = rint(m);
+          ni[k] = (int)r;
+          T[k] = exp_tab[ni[k] & (ENG_EXP_N - 1)];
+          p[k] = d_exp_unit_poly(m - r);
         }
-        part = acc * wf;
+#pragma unroll
+        for (int k = 0; k < KP; k++) acc = fma(x[k], ldexp(fma(T[k], p[k], T[k]), ni[k] >> 9), acc);
       }
-      wred[j * ENG_LRED_STRIDE + lane] = part;
+      wred[j * ENG_LRED_STRIDE + lane] = acc;
+      if (AH == 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(buf, t + 2);
+      }
       if (j == 7 || t == t1 - 1) {
         /* line m of the group (m <= j): lane 8m + q adds the terms of lanes
          * 8r + q (r = 0..7), then the eight lanes of m are summed (xor 1,
@@ -1645,9 +1701,13 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_vr_lines(EngineParams P, PhotonSo
           const int4 il = P.fl_info[tl];
           unsigned long long *bin =
               use_lds ? &tline[(size_t)il.w * 2] : &tline[((size_t)il.x * ENG_MAX_ACT + il.y) * 2];
-          fx_add_global(bin, sum, shift);
+          fx_add_global(bin, sum * P.fl_wf[tl], shift);
         }
       }
+    };
+    for (int t = t0; t < t1; t += 2) {
+      entry(nx[0], t);
+      if (t + 1 < t1) entry(nx[AH - 1], t + 1);
     }
   }
   if (use_lds) {
@@ -2569,18 +2629,23 @@ static void launch_lines_kp(const EngineParams *P, const PhotonSoA *S, const VrS
   }
 }
 
-/* photons per lane of k_vr_lines (P->lines_kp, 0: the default): each
- * line's wavefront sum then serves 64 KP photons; fewer where the
- * per-photon path lengths take more registers.  Three rather than four up
- * to four layers by default: 126 VGPRs give four waves per SIMD instead of
- * three (3 % faster) */
+/* photons per lane of k_vr_lines (P->lines_kp, 0: the default): an entry's
+ * loads, staging and reduction then serve 64 KP photons; fewer where the
+ * per-photon path lengths take more registers.  Four up to three layers
+ * (107 VGPRs, four waves per SIMD; three photons run 3 % slower on the
+ * three-layer tube run, 10 % on one layer), three up to five (three against
+ * four on four layers: 2 % faster), two up to eight */
 template <int NL>
 static void launch_lines(const EngineParams *P, const PhotonSoA *S, const VrSoA *V, int n, int n_cu, int blocks,
                          hipStream_t st) {
   const int kp = P->lines_kp;
   if constexpr (NL <= 4) {
     if (kp == 2) launch_lines_kp<NL, 2>(P, S, V, n, n_cu, blocks, st);
-    else if (kp == 4) launch_lines_kp<NL, 4>(P, S, V, n, n_cu, blocks, st);
+    else if (kp == 3 || (kp != 4 && NL == 4)) launch_lines_kp<NL, 3>(P, S, V, n, n_cu, blocks, st);
+    else launch_lines_kp<NL, 4>(P, S, V, n, n_cu, blocks, st);
+  } else if constexpr (NL <= 5) {
+    if (kp == 1) launch_lines_kp<NL, 1>(P, S, V, n, n_cu, blocks, st);
+    else if (kp == 2) launch_lines_kp<NL, 2>(P, S, V, n, n_cu, blocks, st);
     else launch_lines_kp<NL, 3>(P, S, V, n, n_cu, blocks, st);
   } else if constexpr (NL <= 8) {
     if (kp == 1) launch_lines_kp<NL, 1>(P, S, V, n, n_cu, blocks, st);
@@ -2631,13 +2696,15 @@ static void launch_estimator_nl(const EngineParams *P, const PhotonSoA *S, const
 }
 
 /* NL, the layer-count bound of the estimator and the step: the smallest of
- * 1, 2, 4, 8, 16 that holds n_layers */
+ * 1 to 5, 8, 16 that holds n_layers */
 static void launch_estimator(const EngineParams *P, const PhotonSoA *S, const VrSoA *V, int n, int count, int n_cu,
                              int blocks, hipStream_t st, hipEvent_t *ev) {
   const int nl = P->n_layers;
   if (nl <= 1) launch_estimator_nl<1>(P, S, V, n, count, n_cu, blocks, st, ev);
   else if (nl <= 2) launch_estimator_nl<2>(P, S, V, n, count, n_cu, blocks, st, ev);
+  else if (nl <= 3) launch_estimator_nl<3>(P, S, V, n, count, n_cu, blocks, st, ev);
   else if (nl <= 4) launch_estimator_nl<4>(P, S, V, n, count, n_cu, blocks, st, ev);
+  else if (nl <= 5) launch_estimator_nl<5>(P, S, V, n, count, n_cu, blocks, st, ev);
   else if (nl <= 8) launch_estimator_nl<8>(P, S, V, n, count, n_cu, blocks, st, ev);
   else launch_estimator_nl<16>(P, S, V, n, count, n_cu, blocks, st, ev);
 }
@@ -2727,14 +2794,16 @@ hipError_t eng_launch_order(const EngineParams *P, const PhotonSoA *S, const VrS
     const int nl = P->n_layers;
     if (nl <= 1) hipLaunchKernelGGL((k_step<1, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
     else if (nl <= 2) hipLaunchKernelGGL((k_step<2, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
+    else if (nl <= 3) hipLaunchKernelGGL((k_step<3, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
     else if (nl <= 4) hipLaunchKernelGGL((k_step<4, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
+    else if (nl <= 5) hipLaunchKernelGGL((k_step<5, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
     else if (nl <= 8) hipLaunchKernelGGL((k_step<8, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
     else hipLaunchKernelGGL((k_step<16, true>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, n, count);
   }
   {
     const int nw = blocks * (ENG_BLOCK / 64), nseg = (nw + ENG_SCAN_SEG - 1) / ENG_SCAN_SEG;
     hipLaunchKernelGGL(k_layer_scan, dim3(nseg, P->n_layers), dim3(ENG_SCAN_SEG), 0, st, *P, nw);
-    hipLaunchKernelGGL(k_layer_base, dim3(1), dim3(64), 0, st, *P, nseg);
+    hipLaunchKernelGGL(k_layer_base, dim3(P->n_layers), dim3(ENG_SCAN_NSEG), 0, st, *P, nseg);
   }
   if (ev) (void)hipEventRecord(ev[1], st);
   launch_estimator(P, S, V, n, count, n_cu, blocks, st, ev ? ev + 2 : nullptr);
