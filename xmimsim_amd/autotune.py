@@ -115,7 +115,7 @@ def tune(prep: "api.Prepared", sample_histories: int = 1 << 23, seed: int = 1,
     """The fastest launch shape for prep's workload and the table of timed
     shapes ({"launch": shape, "ms": device time}); (shape, []) when the
     cache holds the signature.  Candidates are tried besides the defaults
-    (2^21 histories per batch, kernel by kernel, the default photons per lane
+    (2^23 histories per batch, kernel by kernel, the default photons per lane
     and the occupancy's workgroups).  The engine's launch shape in force
     before the call is restored; apply the result with
     api.set_launch(**shape).  timer(shape) -> ms replaces the timed runs

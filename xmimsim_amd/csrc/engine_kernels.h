@@ -36,8 +36,8 @@
 /* histories per batch unless the launch shape says otherwise: every kernel of
  * an order ends with a part-filled round of workgroups, and the scan, list
  * and reset launches cost the same for any size, so the batch is as large as
- * 0.6 GB of photon records (three layers) make it */
-#define ENG_BATCH_LOG2 21
+ * 2.3 GB of photon records (three layers) make it */
+#define ENG_BATCH_LOG2 23
 /* segments of the per-wave layer-count scan (k_layer_scan, d_layer_list):
  * the waves of the largest batch, one thread per slot */
 #define ENG_SCAN_SEG 1024
