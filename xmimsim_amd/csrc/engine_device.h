@@ -36,7 +36,6 @@ struct PhotonSoA {
   double *x, *y, *z;
   double *dx, *dy, *dz;
   double *ex, *ey, *ez;
-  double *theta, *phi;
   double *energy, *weight;
   double *mus;                  /* [n_layers][cap] */
   int *layer;                   /* 1-based, 0 = dead */
@@ -86,7 +85,7 @@ struct EngineParams {
   int brute;
   int casc;                     /* cascades of a primary: bit 0 Auger, bit 1 radiative */
   int off_half;
-  double slit_x, slit_y, d_source_slit;
+  double slit_ax, slit_ay, d_source_slit; /* half opening angles of the slit */
   int n_layers;
   int n_int;
   int nch;
@@ -127,6 +126,7 @@ struct EngineParams {
   const double *tab_R;          /* [n_r] */
   int n_e, n_r;
   double tab_E0, tab_Einv, tab_R0, tab_Rinv;
+  int tab_uniform;              /* the angle and azimuth tables' grids are uniform (d_table) */
   const double *fycorr;         /* [nZ][9] */
   const double *ip_E;           /* concatenated */
   const double *ip_r;
@@ -149,6 +149,7 @@ struct EngineParams {
   const double *cp_pcdf, *cp_qinv, *cp_Qs, *cp_inv;
   const double *precalc_xrf;    /* [nZ][9][nZ][219] */
   const double *line_E;         /* [nZ][219] */
+  const double *rate_cum;       /* [nZ][220] radiative rates summed along each shell's lines, index |line| */
   const double *precalc_mu;     /* [n_layers][nZ][219] */
   /* detection tables */
   const int *act_n;             /* [nZ] */

@@ -237,7 +237,7 @@ struct DeviceTables {
   const xmi_hdf5F *owner = nullptr;
   int nZ = 0;
   int Zs[XMI_MAXZ + 1];
-  DevBuf atoms, ray, comp, tabE, tabR, fycorr, ipE, ipr, iprc, ipoff, ipacc, cp_icdf, cp_rn, precalc_xrf, lineE;
+  DevBuf atoms, ray, comp, tabE, tabR, fycorr, ipE, ipr, iprc, ipoff, ipacc, cp_icdf, cp_rn, precalc_xrf, lineE, rate_cum;
   DevBuf cp_cdfg, cp_gscale;
   DevBuf phi, phiT, phiR;
   /* the advanced Compton model's subshell profiles, uploaded on first use */
@@ -247,6 +247,7 @@ struct DeviceTables {
   int n_e = 0, n_r = 0, cp_len = 0, phi_nt = 0, phi_nr = 0;
   double tab_E0 = 0, tab_Einv = 0, tab_R0 = 0, tab_Rinv = 0, phi_T0 = 0, phi_Tinv = 0, phi_R0 = 0, phi_Rinv = 0;
   double ip_acc_E0 = 0, ip_acc_inv = 0;
+  int tab_uniform = 0; /* the angle and azimuth tables' grids are uniform */
 };
 
 /* device copies of the tables of each xmi_hdf5F handle, shared by all engines */
@@ -272,7 +273,7 @@ struct Engine {
   DevBuf el_Z, el_w, el_u, precalc_mu, act_n, act_line, act_shell, act_factor, act_E, act_ch, act_murho;
   DevBuf fl_info, fl_wf, fl_ent, lbin_g;
   DevBuf lay_rc, lay_edge, lay_pb, lay_kstart, lay_cell, el_cell;
-  DevBuf src_desc, src_line_mus, exc_layers, exc_atoms;
+  DevBuf src_desc, src_run0, src_line_mus, exc_layers, exc_atoms;
   DevBuf state, vr, tallies, counters, queue, lay_list, lay_woff, lay_total, lay_segbase, cone_acc, esc_tally;
   DevBuf queue2, qcount2, olist;
   DevBuf batch_queue;
@@ -295,6 +296,15 @@ static int engine_init(Engine &E) {
   return 1;
 }
 static int engine_init() { return engine_init(g_engine); }
+
+/* whether a grid's points lie at a[0] + k h to rounding (1e-13 of its range) */
+static int grid_uniform(const double *a, int n) {
+  if (n < 2) return 0;
+  const double h = (a[n - 1] - a[0]) / (double)(n - 1);
+  for (int k = 0; k < n; k++)
+    if (!(fabs(a[k] - (a[0] + (double)k * h)) <= 1e-13 * fabs(a[n - 1] - a[0]))) return 0;
+  return a[n - 1] > a[0];
+}
 
 static double uniform_inv(const double *a, int n) { return (double)(n - 1) / (a[n - 1] - a[0]); }
 
@@ -325,7 +335,8 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
   std::vector<double> cdfg((size_t)XMI_CP_GRID * nZ), gscale(nZ);
   std::vector<double> ipE, ipr, iprc;
   std::vector<int> ipoff(nZ + 1), ipacc((size_t)nZ * ENG_IP_ACC);
-  std::vector<double> pxrf((size_t)nZ * 9 * nZ * XMI_NLINES_VR, 0.0), lineE((size_t)nZ * XMI_NLINES_VR, 0.0);
+  std::vector<double> pxrf((size_t)nZ * 9 * nZ * XMI_NLINES_VR, 0.0), lineE((size_t)nZ * XMI_NLINES_VR, 0.0),
+      rcum((size_t)nZ * (XMI_NLINES_VR + 1), 0.0);
   t->ip_acc_E0 = z0->ip_energies[0];
   double Emax = z0->ip_energies[z0->ip_len - 1];
   t->ip_acc_inv = (double)ENG_IP_ACC / (Emax - t->ip_acc_E0);
@@ -361,6 +372,12 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
     else
       t->has_precalc = false;
     for (int l = 1; l <= XMI_NLINES_VR; l++) lineE[(size_t)i * XMI_NLINES_VR + l - 1] = atoms[i].line_energy[l];
+    for (int sh = 0; sh < 9; sh++) {
+      int first, last;
+      xrl_shell_lines(sh, &first, &last);
+      double sum = 0.0;
+      for (int l = first; l <= last; l++) rcum[(size_t)i * (XMI_NLINES_VR + 1) + l] = sum += atoms[i].rad_rate[l];
+    }
   }
   ipoff[nZ] = (int)ipE.size();
   t->tab_E0 = z0->Energies[0];
@@ -373,8 +390,11 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
   t->phi_Tinv = uniform_inv(h->Thetas, h->phi_n_theta);
   t->phi_R0 = h->RandomNumbers[0];
   t->phi_Rinv = uniform_inv(h->RandomNumbers, h->phi_n_r);
+  t->tab_uniform = grid_uniform(z0->Energies, t->n_e) && grid_uniform(z0->RandomNumbers, t->n_r) &&
+                   grid_uniform(h->Thetas, h->phi_n_theta) && grid_uniform(h->RandomNumbers, h->phi_n_r);
   hipError_t e = hipSuccess;
   e = upload(t->atoms, atoms.data(), atoms.size(), st, sg);
+  if (e == hipSuccess) e = upload(t->rate_cum, rcum.data(), rcum.size(), st, sg);
   if (e == hipSuccess) e = upload(t->ray, ray.data(), ray.size(), st, sg);
   if (e == hipSuccess) e = upload(t->comp, comp.data(), comp.size(), st, sg);
   if (e == hipSuccess) e = upload(t->tabE, z0->Energies, (size_t)t->n_e, st, sg);
@@ -521,8 +541,8 @@ static void fill_geometry(EngineParams &P, const xmi_inputF *in) {
     const double c = cos(in->half_apex);
     P.det_cos2 = c * c;
   }
-  P.slit_x = in->geometry.slit_size_x;
-  P.slit_y = in->geometry.slit_size_y;
+  P.slit_ax = atan(in->geometry.slit_size_x / in->geometry.d_source_slit / 2.0);
+  P.slit_ay = atan(in->geometry.slit_size_y / in->geometry.d_source_slit / 2.0);
   P.d_source_slit = in->geometry.d_source_slit;
 }
 
@@ -941,6 +961,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       d.run0 = (uint64_t)total_hist;
       total_hist += (d.valid && d.count > 0) ? d.count : 0;
     }
+    std::vector<uint64_t> run0;
+    for (const auto &d : src) run0.push_back(d.run0);
     const int cap_max = 1 << (g_launch.batch_log2 ? g_launch.batch_log2 : ENG_BATCH_LOG2);
     int cap = (int)(total_hist < cap_max ? (total_hist > 0 ? total_hist : 1) : cap_max);
     /* a brute-force run with cascades keeps a second slot per primary for
@@ -951,7 +973,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     size_t per = (size_t)slots;
     /* the kernels' layer-count bound (estimator records hold nl_bound paths) */
     const int nl_bound = eng_layer_bound(NL);
-    size_t state_bytes = per * (15 * sizeof(double) + (size_t)NL * sizeof(double) + 5 * sizeof(int) + sizeof(uint64_t));
+    size_t state_bytes = per * (11 * sizeof(double) + (size_t)NL * sizeof(double) + 5 * sizeof(int) + sizeof(uint64_t));
     size_t vr_bytes = per * ((6 + (size_t)nl_bound) * sizeof(double) + 2 * sizeof(int));
     size_t n_ch2 = (size_t)n_int * nch * 2, n_line2 = (size_t)n_int * nZ * ENG_MAX_ACT * 2, n_rc2 = (size_t)n_int * nZ * 4;
     /* brute force: hits by interactions so far, and by the last interaction */
@@ -1031,6 +1053,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       up.add(G.lay_cell, lay_cell.data(), lay_cell.size());
       up.add(G.el_cell, el_cell.data(), el_cell.size());
       up.add(G.src_desc, src.data(), src.size());
+      up.add(G.src_run0, run0.data(), run0.size());
       up.add(G.src_line_mus, src_mus.data(), src_mus.size());
       up.add(G.exc_layers, exc_flat.data(), exc_flat.size());
       up.add(G.exc_atoms, exc_atoms.data(), exc_atoms.size());
@@ -1077,6 +1100,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     }
     P.precalc_xrf = T->precalc_xrf.as<double>();
     P.line_E = T->lineE.as<double>();
+    P.rate_cum = T->rate_cum.as<double>();
+    P.tab_uniform = T->tab_uniform;
     P.precalc_mu = G.precalc_mu.as<double>();
     P.act_n = G.act_n.as<int>();
     P.act_line = G.act_line.as<int>();
@@ -1156,12 +1181,11 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
 
     PhotonSoA S;
     char *sp = G.state.as<char>();
-    double **dfields[] = {&S.x, &S.y, &S.z, &S.dx, &S.dy, &S.dz, &S.ex, &S.ey, &S.ez, &S.theta, &S.phi, &S.energy, &S.weight};
+    double **dfields[] = {&S.x, &S.y, &S.z, &S.dx, &S.dy, &S.dz, &S.ex, &S.ey, &S.ez, &S.energy, &S.weight};
     for (double **f : dfields) {
       *f = (double *)sp;
       sp += per * sizeof(double);
     }
-    sp += 2 * per * sizeof(double);
     S.mus = (double *)sp;
     sp += per * NL * sizeof(double);
     S.hid = (uint64_t *)sp;
@@ -1191,6 +1215,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
 
     SourceTable ST;
     ST.d = G.src_desc.as<SourceDesc>();
+    ST.run0 = G.src_run0.as<uint64_t>();
     ST.n = (int)src.size();
     ST.line_mus = G.src_line_mus.as<double>();
     ST.exc_layers = G.exc_layers.as<double>();

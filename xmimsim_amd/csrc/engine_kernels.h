@@ -80,6 +80,7 @@ struct SourceDesc {
 
 struct SourceTable {
   const SourceDesc *d;
+  const uint64_t *run0;       /* [n] the descriptors' run0, for the search */
   int n;
   const double *line_mus;     /* [n_sources][n_layers] mus at the line energy */
   const double *exc_layers;   /* per absorber: density, thickness, n_el, Z[n_el], w[n_el] */

@@ -33,6 +33,171 @@
 #include "engine_kernels.h"
 
 
+/* read-only tables through the constant address space: wave-uniform reads
+ * become scalar loads (the tables are not written while a kernel runs) */
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(4))) T *d_const(const T *p) {
+  return (const __attribute__((address_space(4))) T *)p;
+}
+
+/* ------------------------------------------------------------------------ */
+/* elementary functions on the ranges the kernels use */
+
+/* square root of x > 0 (no scaling: x far from the ends of the range): the
+ * hardware's reciprocal root, one coupled Newton step and a residual
+ * correction; NaN at 0 */
+__device__ __forceinline__ double d_sqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
+/* sin(pi w) for |w| <= 1/2: w times the polynomial in w^2 that interpolates
+ * sin(pi w) / w at the Chebyshev nodes of the interval (relative error below
+ * 4e-19 before rounding) */
+__device__ __forceinline__ double d_sinpi_core(double w) {
+  const double z = w * w;
+  double p = fma(z, 0x1.9d462020fcc78p-21, -0x1.6f7acdb8f6580p-16);
+  p = fma(z, p, 0x1.e8f3675ee37ddp-12);
+  p = fma(z, p, -0x1.e3074dfaf87afp-8);
+  p = fma(z, p, 0x1.5078348551854p-4);
+  p = fma(z, p, -0x1.32d2cce627c86p-1);
+  p = fma(z, p, 0x1.466bc6775aa7dp+1);
+  p = fma(z, p, -0x1.4abbce625be52p+2);
+  p = fma(z, p, 0x1.921fb54442d18p+1);
+  return w * p;
+}
+
+/* sin(pi t) and cos(pi t) for |t| <= 1: the sine folded to [0, 1/2], the
+ * cosine as the sine of 1/2 - |t| (both differences exact) */
+__device__ __forceinline__ double d_sinpi1(double t) {
+  const double w = fabs(t);
+  return copysign(d_sinpi_core(fmin(w, 1.0 - w)), t);
+}
+__device__ __forceinline__ double d_cospi1(double t) { return d_sinpi_core(0.5 - fabs(t)); }
+
+/* reciprocal square root of x > 0 far from the ends of the range: the
+ * hardware's estimate (2^-24 or better) and one third-order step */
+__device__ __forceinline__ double d_rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+/* E^-p of the photo-ionisation cross sections (p = 11/4) for an energy in the
+ * provider's range: E^(-1/2) cubed twice times E^(1/4), from two reciprocal
+ * square roots; 0 for E <= 0, as xrl_energy */
+static_assert(XRL_PHOTO_EXPONENT == 2.75, "d_photo_pe forms E^-11/4");
+__device__ __forceinline__ double d_photo_pe(double E) {
+  const double a = d_rsqrt_pos(E), a2 = a * a;
+  return E > 0.0 ? a2 * a2 * (a2 * d_rsqrt_pos(a)) : 0.0;
+}
+
+/* the provider's energy context (xrl_energy) with E^-p as d_photo_pe */
+__device__ __forceinline__ xrl_ectx d_energy(double E) {
+  xrl_ectx c;
+  c.E = E;
+  c.pe = c.cf = 0.0;
+  c.ci = 0;
+  if (!(E > 0.0)) return c;
+  const double inv_h = (double)(XRL_NCS - 1) / (XRL_CS_LNE1 - XRL_CS_LNE0);
+  const double x = (log(E) - XRL_CS_LNE0) * inv_h;
+  int i = (int)floor(x);
+  i = i < 0 ? 0 : (i > XRL_NCS - 2 ? XRL_NCS - 2 : i);
+  c.ci = i;
+  c.cf = x - (double)i;
+  c.pe = d_photo_pe(E);
+  return c;
+}
+
+/* ---- directions ----------------------------------------------------------
+ * A photon's frame is e_theta = (ct cp, ct sp, -st), e_phi = (-sp, cp, 0) and
+ * its direction d = (st cp, st sp, ct).  The reference keeps the angles and
+ * takes their sines and cosines back; here they are read off d itself: ct =
+ * dz, st = sqrt(1 - dz^2) (what sin(acos(dz)) gives: beside the axis it
+ * carries dz's rounding, as the reference's does), cp and sp from (dx, dy)
+ * (cp = 1, sp = 0 on the axis, as atan2(0, 0) = 0).  A turn takes two square
+ * roots where it took six sines and cosines, an acos and an atan2, and two
+ * words of photon state less: k_interact 193 -> 135 us for 2^21 slots. */
+struct DFrame {
+  double et[3], ep0, ep1;
+  double d[3];
+};
+
+/* sqrt(1 - c^2), 0 where rounding has taken |c| to 1 or beyond */
+__device__ __forceinline__ double d_sin_of(double c) {
+  const double x = (1.0 - c) * (1.0 + c);
+  return x > 0.0 ? d_sqrt_pos(x) : 0.0;
+}
+
+__device__ __forceinline__ DFrame d_frame(const double *d) {
+  const double s2 = fma(d[0], d[0], d[1] * d[1]);
+  const double is = d_rsqrt_pos(s2), st = d_sin_of(d[2]);
+  const int axis = !(s2 > 0.0);
+  const double cp = axis ? 1.0 : d[0] * is, sp = axis ? 0.0 : d[1] * is;
+  DFrame f;
+  f.et[0] = d[2] * cp;
+  f.et[1] = d[2] * sp;
+  f.et[2] = -st;
+  f.ep0 = -sp;
+  f.ep1 = cp;
+  f.d[0] = st * cp;
+  f.d[1] = st * sp;
+  f.d[2] = d[2];
+  return f;
+}
+
+/* the direction of a frame turned by the polar angle (cosine c, sine s) with
+ * the azimuth (cosine ca, sine sa), of unit length again: the length is 1 up
+ * to rounding, so one linear step restores it */
+__device__ __forceinline__ void d_turn(double *d, const DFrame &f, double c, double s, double ca, double sa) {
+  const double v0 = s * ca, v1 = s * sa;
+  const double n0 = fma(v0, f.et[0], fma(v1, f.ep0, c * f.d[0]));
+  const double n1 = fma(v0, f.et[1], fma(v1, f.ep1, c * f.d[1]));
+  const double n2 = fma(v0, f.et[2], c * f.d[2]);
+  const double k = fma(-0.5, fma(n0, n0, fma(n1, n1, n2 * n2)), 1.5);
+  d[0] = n0 * k;
+  d[1] = n1 * k;
+  d[2] = n2 * k;
+}
+
+/* the polarisation after a turn: its part normal to the new direction */
+__device__ __forceinline__ void d_update_elecv(const double *d, double *e) {
+  const double c = d_dot(d, e);
+  for (int i = 0; i < 3; i++) e[i] = fma(-c, d[i], e[i]);
+  const double k = d_rsqrt_pos(d_dot(e, e));
+  for (int i = 0; i < 3; i++) e[i] *= k;
+}
+
+/* azimuth (cosine, sine) of phi, measured from the polarisation e, in the
+ * frame of the direction (src/xmi_main.F90:2034-2060: phi0 + phi, phi0 the
+ * arc cosine of e . e_theta with the sign of e . e_phi) */
+__device__ __forceinline__ void d_from_polarisation(const DFrame &f, const double *e, double *ca, double *sa) {
+  double c0 = e[0] * f.et[0] + e[1] * f.et[1] + e[2] * f.et[2];
+  c0 = fmin(fmax(c0, -1.0), 1.0);
+  const double s0 = e[0] * f.ep0 + e[1] * f.ep1 < 0.0 ? -d_sin_of(c0) : d_sin_of(c0);
+  const double c = *ca, s = *sa;
+  *ca = c * c0 - s * s0;
+  *sa = s * c0 + c * s0;
+}
+
+/* cosine and sine of an azimuth table's angle in [0, 2 pi] */
+__device__ __forceinline__ void d_azimuth(double phi, double *c, double *s) {
+  const double t = fma(phi, 1.0 / ENG_PI, -1.0);
+  *c = -d_cospi1(t);
+  *s = -d_sinpi1(t);
+}
+
+/* cosine and sine of 2 pi u, u in [0, 1) (2 u - 1 is exact) */
+__device__ __forceinline__ void d_turns(double u, double *c, double *s) {
+  const double t = fma(2.0, u, -1.0);
+  *c = -d_cospi1(t);
+  *s = -d_sinpi1(t);
+}
+
 /* ------------------------------------------------------------------------ */
 /* physics helpers on the device */
 
@@ -54,7 +219,7 @@ __device__ __forceinline__ double d_layer_mu_tab(const EngineParams &P, int laye
 }
 
 __device__ __forceinline__ void d_mu_all(const EngineParams &P, double E, double *mus, size_t stride, size_t idx) {
-  xrl_ectx c = xrl_energy(E);
+  xrl_ectx c = d_energy(E);
   for (int l = 0; l < P.n_layers; l++) mus[(size_t)l * stride + idx] = d_layer_mu_tab(P, l, &c);
 }
 
@@ -70,45 +235,22 @@ __device__ __forceinline__ void d_wave_count(unsigned long long *ctr, int pred) 
   if (m != 0ull && __lane_id() == 0) atomicAdd(ctr, (unsigned long long)__popcll(m));
 }
 
-__device__ __forceinline__ void d_update_dirv(double *dirv, double *theta, double *phi, double theta_i, double phi_i) {
-  double phi_new = phi_i;
-  if (phi_i > 2.0 * ENG_PI) phi_new = phi_i - 2.0 * ENG_PI;
-  else if (phi_i < 0.0) phi_new = phi_i + 2.0 * ENG_PI;
-  double cp = cos(*phi), sp = sin(*phi), ct = cos(*theta), st = sin(*theta);
-  double ts = sin(theta_i);
-  double v0 = ts * cos(phi_new), v1 = ts * sin(phi_new), v2 = cos(theta_i);
-  double d0 = ct * cp * v0 + (-sp) * v1 + st * cp * v2;
-  double d1 = ct * sp * v0 + cp * v1 + st * sp * v2;
-  double d2 = (-st) * v0 + 0.0 * v1 + ct * v2;
-  double n = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-  dirv[0] = d0 / n;
-  dirv[1] = d1 / n;
-  dirv[2] = d2 / n;
-  *theta = acos(dirv[2]);
-  double ph = atan2(dirv[1], dirv[0]);
-  if (ph > 2.0 * ENG_PI) ph -= 2.0 * ENG_PI;
-  else if (ph < 0.0) ph += 2.0 * ENG_PI;
-  *phi = ph;
-}
-
-__device__ __forceinline__ void d_update_elecv(const double *dirv, double *elecv) {
-  double cosalfa = d_dot(dirv, elecv);
-  double c_alfa = acos(cosalfa);
-  double sinalfa = sin(c_alfa);
-  double c_ae = 1.0 / sinalfa;
-  double c_be = -c_ae * cosalfa;
-  for (int i = 0; i < 3; i++) elecv[i] = c_ae * elecv[i] + c_be * dirv[i];
-  d_normalize(elecv);
-}
-
-__device__ __forceinline__ double d_phi0(double theta, double phi, const double *elecv) {
-  double cp = cos(phi), sp = sin(phi), ct = cos(theta), st = sin(theta);
-  double cosphi0 = elecv[0] * (cp * ct) + elecv[1] * (ct * sp) + elecv[2] * (-st);
-  double sinphi0 = elecv[0] * sp + elecv[1] * (-cp) + elecv[2] * 0.0;
-  if (fabs(cosphi0) > 1.0) cosphi0 = cosphi0 > 0 ? 1.0 : -1.0;
-  double phi0 = acos(cosphi0);
-  if (sinphi0 > 0.0) phi0 = -phi0;
-  return phi0;
+/* table value at (x1, x2), rows along x1: on the uniform grids of the
+ * generator the cell and the fraction come from the coordinate itself (its
+ * rounding, 2e-13 of a cell, is far below the table's), without reading the
+ * grids; other grids (a table file may hold any) take d_bilinear */
+__device__ __forceinline__ double d_table(int uniform, const double *arr, const double *a1, int n1, double a10,
+                                          double a1inv, const double *a2, int n2, double a20, double a2inv, double x1,
+                                          double x2) {
+  if (!uniform) return d_bilinear(arr, a1, n1, a10, a1inv, a2, n2, a20, a2inv, x1, x2);
+  const double t1 = (x1 - a10) * a1inv, t2 = (x2 - a20) * a2inv;
+  int p1 = (int)floor(t1), p2 = (int)floor(t2);
+  p1 = p1 < 0 ? 0 : (p1 > n1 - 2 ? n1 - 2 : p1);
+  p2 = p2 < 0 ? 0 : (p2 > n2 - 2 ? n2 - 2 : p2);
+  const double f1 = t1 - (double)p1, f2 = t2 - (double)p2;
+  const double *r0 = arr + (size_t)p1 * n2 + p2, *r1 = r0 + n2;
+  const double v0 = fma(f2, r0[1] - r0[0], r0[0]), v1 = fma(f2, r1[1] - r1[0], r1[0]);
+  return fma(f1, v1 - v0, v0);
 }
 
 /* cone-sampling estimate of the detector solid angle seen from (r1, theta1),
@@ -203,36 +345,6 @@ __device__ __forceinline__ int d_sa_setup(const SaGeom g, double r1, double thet
   return 1;
 }
 
-/* square root of x > 0 (no scaling: x far from the ends of the range): the
- * hardware's reciprocal root, one coupled Newton step and a residual
- * correction; NaN at 0 */
-__device__ __forceinline__ double d_sqrt_pos(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  return fma(fma(-g, g, x), h, g);
-}
-
-/* sin(pi t) for |t| <= 1: folded to [0, 1/2] (exact), then w times the
- * polynomial in w^2 that interpolates sin(pi w) / w at the Chebyshev nodes of
- * the interval (relative error below 4e-19 before rounding) */
-__device__ __forceinline__ double d_sinpi1(double t) {
-  double w = fabs(t);
-  w = fmin(w, 1.0 - w);
-  const double z = w * w;
-  double p = fma(z, 0x1.9d462020fcc78p-21, -0x1.6f7acdb8f6580p-16);
-  p = fma(z, p, 0x1.e8f3675ee37ddp-12);
-  p = fma(z, p, -0x1.e3074dfaf87afp-8);
-  p = fma(z, p, 0x1.5078348551854p-4);
-  p = fma(z, p, -0x1.32d2cce627c86p-1);
-  p = fma(z, p, 0x1.466bc6775aa7dp+1);
-  p = fma(z, p, -0x1.4abbce625be52p+2);
-  p = fma(z, p, 0x1.921fb54442d18p+1);
-  return copysign(w * p, t);
-}
-
 /* one cone direction from two words at their midpoints, u1 = 1 - cos theta
  * over 1 - cos apex and u2 = phi over 2 pi; 1 if it reaches the window */
 __device__ __forceinline__ int d_sa_trial(const SaCone &c, uint32_t w1, uint32_t w2) {
@@ -295,7 +407,7 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_solid_angle_grid(EngineParams P, 
 
 __device__ double d_gauss(phx_stream *s, double sigma) {
   double u1 = phx_uniform(s), u2 = phx_uniform(s);
-  return sigma * sqrt(-2.0 * log(1.0 - u1)) * cos(2.0 * ENG_PI * u2);
+  return sigma * sqrt(-2.0 * log(1.0 - u1)) * -d_cospi1(fma(2.0, u2, -1.0));
 }
 
 __device__ double d_exc_corr(const SourceTable &S, double E) {
@@ -351,20 +463,24 @@ __device__ int d_ran_trap(double x1, double x2, double y1, double y2, double u, 
 __device__ int d_source_one(const EngineParams &P, const PhotonSoA &S, const SourceTable &T, uint64_t batch_start,
                             int i) {
   const uint64_t run = batch_start + (uint64_t)i;
+  /* last source with run0 <= run (empty sources share their successor's run0
+   * and are skipped): a wave's photons are neighbours in the run order, so the
+   * search for its first photon is scalar and the others walk on from there */
+  const auto *run0 = d_const(T.run0);
+  const uint64_t run_w = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)run) |
+                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(run >> 32)) << 32);
   int lo = 0, hi = T.n - 1;
-  while (lo < hi) { /* last descriptor with run0 <= run: empty sources share
-                       their successor's run0 and are skipped */
-    int mid = (lo + hi + 1) >> 1;
-    if (T.d[mid].run0 <= run) lo = mid;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (run0[mid] <= run_w) lo = mid;
     else hi = mid - 1;
   }
+  while (lo + 1 < T.n && T.run0[lo + 1] <= run) lo++;
   const SourceDesc &d = T.d[lo];
   const uint64_t hid = d.hid0 + (run - d.run0);
   const size_t cap = (size_t)P.cap;
   S.layer[i] = 0;
-  S.hid[i] = hid;
-  S.prev_line[i] = 0;
-  S.prev_u[i] = -1;
+  S.hid[i] = hid; /* the last interaction's line and element are written by the interactions */
   if (P.brute) {
     S.cflags[i] = P.casc;
     if (P.off_half) S.layer[i + P.off_half] = 0; /* no offspring yet */
@@ -403,10 +519,8 @@ __device__ int d_source_one(const EngineParams &P, const PhotonSoA &S, const Sou
   /* xmi_coords_dir, src/xmi_main.F90:957-1136 */
   double dirv[3], coords[3], x1, y1;
   if (fabs(d.sx * d.sy) < 1.0e-20) {
-    double x1m = atan(P.slit_x / P.d_source_slit / 2.0);
-    double y1m = atan(P.slit_y / P.d_source_slit / 2.0);
-    x1 = x1m * (-1.0 + 2.0 * phx_uniform(&s));
-    y1 = y1m * (-1.0 + 2.0 * phx_uniform(&s));
+    x1 = P.slit_ax * (-1.0 + 2.0 * phx_uniform(&s));
+    y1 = P.slit_ay * (-1.0 + 2.0 * phx_uniform(&s));
     coords[0] = coords[1] = coords[2] = 0.0;
   } else {
     x1 = d_gauss(&s, d.sxp);
@@ -415,17 +529,21 @@ __device__ int d_source_one(const EngineParams &P, const PhotonSoA &S, const Sou
     coords[1] = d_gauss(&s, d.sy) - P.d_source_slit * sin(y1);
     coords[2] = 0.0;
   }
-  dirv[0] = tan(x1);
-  dirv[1] = tan(y1);
+  if (fabs(x1) < 0.5 * ENG_PI && fabs(y1) < 0.5 * ENG_PI) {
+    const double tx = x1 * (1.0 / ENG_PI), ty = y1 * (1.0 / ENG_PI);
+    dirv[0] = d_sinpi_core(tx) / d_cospi1(tx);
+    dirv[1] = d_sinpi_core(ty) / d_cospi1(ty);
+  } else {
+    dirv[0] = tan(x1);
+    dirv[1] = tan(y1);
+  }
   dirv[2] = 1.0;
-  d_normalize(dirv);
+  d_normalize(dirv); /* rounded as the reference's: the frame of a beam along z hangs on the last bit of dz */
 
   double ev[3];
   if (d.pol == 1) {
     /* escape-ratio runs: a random polarisation azimuth in the x-y plane */
-    const double te = phx_uniform(&s) * ENG_PI * 2.0;
-    ev[0] = cos(te);
-    ev[1] = sin(te);
+    d_turns(phx_uniform(&s), &ev[0], &ev[1]);
     ev[2] = 0.0;
   } else {
     int horizontal;
@@ -441,10 +559,8 @@ __device__ int d_source_one(const EngineParams &P, const PhotonSoA &S, const Sou
       atomicAdd(d_ctr(P, ENG_CNT_ERR_SOURCE), 1ull);
     return 0;
   }
-  double c_alfa = acos(cosalfa);
-  double c_ae = 1.0 / sin(c_alfa);
-  double c_be = -c_ae * cosalfa;
-  for (int k = 0; k < 3; k++) ev[k] = c_ae * ev[k] + c_be * dirv[k];
+  const double c_ae = d_rsqrt_pos((1.0 - cosalfa) * (1.0 + cosalfa));
+  for (int k = 0; k < 3; k++) ev[k] = c_ae * fma(-cosalfa, dirv[k], ev[k]);
 
   /* xmi_photon_shift_first_layer */
   int layer = 0;
@@ -480,8 +596,6 @@ __device__ int d_source_one(const EngineParams &P, const PhotonSoA &S, const Sou
   S.ex[i] = ev[0];
   S.ey[i] = ev[1];
   S.ez[i] = ev[2];
-  S.theta[i] = acos(dirv[2]);
-  S.phi[i] = atan2(dirv[1], dirv[0]);
   S.energy[i] = E;
   S.weight[i] = w;
   S.layer[i] = layer;
@@ -981,13 +1095,6 @@ __device__ __forceinline__ double d_readlane(double v, int lane) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-/* read-only tables through the constant address space: wave-uniform reads
- * become scalar loads (the tables are not written while a kernel runs) */
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T *d_const(const T *p) {
-  return (const __attribute__((address_space(4))) T *)p;
-}
-
 /* one DPP lane move of a double (two 32-bit moves); lanes the row mask
  * leaves out, or whose source lane lies outside the row, read 0 */
 template <int CTRL, int ROW_MASK>
@@ -1031,23 +1138,6 @@ __device__ __forceinline__ double d_exp_neg(double x, const double *tab) {
   return ldexp(fma(T, p, T), ni >> 6);
 }
 
-
-/* reciprocal square root of x > 0 far from the ends of the range: the
- * hardware's estimate (2^-24 or better) and one third-order step */
-__device__ __forceinline__ double d_rsqrt_pos(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-(x * y), y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-/* E^-p of the photo-ionisation cross sections (p = 11/4) for an energy in the
- * provider's range: E^(-1/2) cubed twice times E^(1/4), from two reciprocal
- * square roots; 0 for E <= 0, as xrl_energy */
-static_assert(XRL_PHOTO_EXPONENT == 2.75, "d_photo_pe forms E^-11/4");
-__device__ __forceinline__ double d_photo_pe(double E) {
-  const double a = d_rsqrt_pos(E), a2 = a * a;
-  return E > 0.0 ? a2 * a2 * (a2 * d_rsqrt_pos(a)) : 0.0;
-}
 
 /* e^-m from t = -m ENG_EXP_UNIT, for a factor that tables and coefficients
  * hold in these units: t = 512 k + j + f with |f| <= 1/2, so the value is
@@ -1740,19 +1830,18 @@ __device__ __forceinline__ void d_rayleigh_one(const EngineParams &P, const Phot
   d_stream_seek(&s, 3u);
   double E = S.energy[i];
   double r = phx_uniform(&s);
-  double theta_i = d_bilinear(P.ray_icdf + (size_t)u * P.n_e * P.n_r, P.tab_E, P.n_e, P.tab_E0, P.tab_Einv, P.tab_R,
-                              P.n_r, P.tab_R0, P.tab_Rinv, E, r);
-  double tt = sin(theta_i);
-  tt = tt * tt;
-  tt = tt / (4.0 - 2.0 * tt);
-  double r2 = phx_uniform(&s);
-  double phi_i = d_bilinear(P.phi_icdf, P.phi_T, P.phi_nt, P.phi_T0, P.phi_Tinv, P.phi_R, P.phi_nr, P.phi_R0,
-                            P.phi_Rinv, tt, r2);
-  double th = S.theta[i], ph = S.phi[i];
-  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]};
-  double phi0 = d_phi0(th, ph, ev);
-  double dirv[3];
-  d_update_dirv(dirv, &th, &ph, theta_i, phi0 + phi_i);
+  const double h = d_table(P.tab_uniform, P.ray_icdf + (size_t)u * P.n_e * P.n_r, P.tab_E, P.n_e, P.tab_E0, P.tab_Einv,
+                           P.tab_R, P.n_r, P.tab_R0, P.tab_Rinv, E, r) * (0.5 / ENG_PI);
+  /* half the scattering angle, over pi */
+  const double sh = d_sinpi_core(h), ct = fma(-2.0 * sh, sh, 1.0), st = 2.0 * sh * d_cospi1(h);
+  const double s2 = st * st, tt = s2 / (4.0 - 2.0 * s2);
+  const double phi_i = d_table(P.tab_uniform, P.phi_icdf, P.phi_T, P.phi_nt, P.phi_T0, P.phi_Tinv, P.phi_R, P.phi_nr,
+                               P.phi_R0, P.phi_Rinv, tt, phx_uniform(&s));
+  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]}, dirv[3] = {S.dx[i], S.dy[i], S.dz[i]}, ca, sa;
+  const DFrame f = d_frame(dirv);
+  d_azimuth(phi_i, &ca, &sa);
+  d_from_polarisation(f, ev, &ca, &sa);
+  d_turn(dirv, f, ct, st, ca, sa);
   d_update_elecv(dirv, ev);
   S.dx[i] = dirv[0];
   S.dy[i] = dirv[1];
@@ -1760,8 +1849,6 @@ __device__ __forceinline__ void d_rayleigh_one(const EngineParams &P, const Phot
   S.ex[i] = ev[0];
   S.ey[i] = ev[1];
   S.ez[i] = ev[2];
-  S.theta[i] = th;
-  S.phi[i] = ph;
   /* brute force: the history row of the last interaction, and its element */
   S.prev_line[i] = BRUTE ? 384 : 0;
   if (BRUTE) S.prev_u[i] = u;
@@ -1777,17 +1864,15 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   phx_stream_init(&s, P.seed, P.sample, (uint32_t)n, BRUTE ? d_tr_sub(P, i) : PHX_SUB_TRANSPORT, S.hid[i]);
   d_stream_seek(&s, 3u);
   double E = S.energy[i];
-  double theta_i = d_bilinear(P.comp_icdf + (size_t)u * P.n_e * P.n_r, P.tab_E, P.n_e, P.tab_E0, P.tab_Einv, P.tab_R,
-                              P.n_r, P.tab_R0, P.tab_Rinv, E, phx_uniform(&s));
-  double K0K = 1.0 + E * (1.0 - cos(theta_i)) / ENG_MEC2;
-  double tt = sin(theta_i);
-  tt = tt * tt;
-  tt = tt / (K0K + (1.0 / K0K) - tt) / 2.0;
-  double phi_i = d_bilinear(P.phi_icdf, P.phi_T, P.phi_nt, P.phi_T0, P.phi_Tinv, P.phi_R, P.phi_nr, P.phi_R0,
-                            P.phi_Rinv, tt, phx_uniform(&s));
-  double th = S.theta[i], ph = S.phi[i];
-  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]};
-  double phi0 = d_phi0(th, ph, ev);
+  const double theta_i = d_table(P.tab_uniform, P.comp_icdf + (size_t)u * P.n_e * P.n_r, P.tab_E, P.n_e, P.tab_E0,
+                                 P.tab_Einv, P.tab_R, P.n_r, P.tab_R0, P.tab_Rinv, E, phx_uniform(&s));
+  /* half the scattering angle, over pi */
+  const double h = theta_i * (0.5 / ENG_PI), sth2 = d_sinpi_core(h), mct = 2.0 * sth2 * sth2; /* 1 - cos theta */
+  const double ct = 1.0 - mct, st = 2.0 * sth2 * d_cospi1(h);
+  const double K0K = 1.0 + E * mct / ENG_MEC2, st2 = st * st;
+  const double tt = st2 / (K0K + (1.0 / K0K) - st2) / 2.0;
+  const double phi_i = d_table(P.tab_uniform, P.phi_icdf, P.phi_T, P.phi_nt, P.phi_T0, P.phi_Tinv, P.phi_R, P.phi_nr,
+                               P.phi_R0, P.phi_Rinv, tt, phx_uniform(&s));
   if (ADV) {
     /* xmi_update_photon_energy_compton: the subshell by count * CDF(Qimax),
      * Q from its profile below Qimax, the energy from Q; 0 ends the photon */
@@ -1826,10 +1911,9 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   const double cc = (double)1.2399e-6f, c0 = (double)4.85e-12f, c1 = (double)1.456e-2f;
   double energy = E * 1000.0;
   double c_lamb0 = cc / energy;
-  double sth2 = sin(theta_i / 2.0);
   const double *rn = P.cp_rn;
   const double *icdf = P.cp_icdf + (size_t)u * P.cp_len;
-  const double drn = rn[1] - rn[0];
+  const double drn = rn[1] - rn[0], inv_drn = 1.0 / drn;
   /* the reference loops until acceptance; every draw with pz <= 0 is accepted,
    * so the bound below is never reached by valid data and only turns a
    * corrupted table into a counted error instead of a hung wave */
@@ -1837,7 +1921,7 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   for (int it = 0; it < 4096; it++) {
     double r = phx_uniform(&s);
     int pos = (int)(r / drn);
-    double pz = d_interp(rn[pos], icdf[pos], rn[pos + 1], icdf[pos + 1], r);
+    double pz = fma((icdf[pos + 1] - icdf[pos]) * inv_drn, r - rn[pos], icdf[pos]);
     if (phx_uniform(&s) < 0.5) pz = -pz;
     double dlamb = c0 * sth2 * sth2 - c1 * c_lamb0 * sth2 * pz;
     energy = cc / (c_lamb0 + dlamb) / 1000.0;
@@ -1857,12 +1941,18 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   d_mu_all(P, E, S.mus, cap, i);
   if (E == 0.0) return;
   }
-  double dirv[3];
-  d_update_dirv(dirv, &th, &ph, theta_i, phi_i + phi0);
+  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]}, dirv[3] = {S.dx[i], S.dy[i], S.dz[i]};
+  double cph, sph;
+  d_azimuth(phi_i, &cph, &sph);
+  {
+    const DFrame f = d_frame(dirv);
+    double ca = cph, sa = sph;
+    d_from_polarisation(f, ev, &ca, &sa);
+    d_turn(dirv, f, ct, st, ca, sa);
+  }
   d_update_elecv(dirv, ev);
-  double ct = cos(theta_i), cph = cos(phi_i), sph = sin(phi_i);
   double pp = 2.0 * ((ct * cph) * (ct * cph) + sph * sph);
-  double rat = 1.0 / (1.0 + (1.0 - ct) * E / (double)510.998910f);
+  double rat = 1.0 / (1.0 + mct * E / (double)510.998910f);
   double rk = rat - 2.0 + 1.0 / rat;
   pp = pp / (rk + pp);
   double r = phx_uniform(&s);
@@ -1881,8 +1971,6 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   S.ex[i] = ev[0];
   S.ey[i] = ev[1];
   S.ez[i] = ev[2];
-  S.theta[i] = th;
-  S.phi[i] = ph;
   S.prev_line[i] = BRUTE ? 385 : 0;
   if (BRUTE) S.prev_u[i] = u;
 }
@@ -1956,6 +2044,36 @@ __device__ int d_coster_kronig(const xrl_atom *a, phx_stream *s, int shell) {
   return shell;
 }
 
+/* first and last line of a vacancy's shell 0 (K) .. 8 (M5), one byte each
+ * (xrl_shell_lines: a shell's last line precedes the next one's first) */
+__device__ __forceinline__ int d_shell_first(int shell) {
+  constexpr unsigned long long f = (unsigned long long)XRL_KL1 | (unsigned long long)XRL_L1_FIRST << 8 |
+                                   (unsigned long long)XRL_L2_FIRST << 16 | (unsigned long long)XRL_L3_FIRST << 24 |
+                                   (unsigned long long)XRL_M1_FIRST << 32 | (unsigned long long)XRL_M2_FIRST << 40 |
+                                   (unsigned long long)XRL_M3_FIRST << 48 | (unsigned long long)XRL_M4_FIRST << 56;
+  return shell < 8 ? (int)((f >> (8 * shell)) & 0xffull) : (shell == 8 ? XRL_M5_FIRST : XRL_M5_LAST + 1);
+}
+static_assert(XRL_KP5 + 1 == XRL_L1_FIRST && XRL_L1_LAST + 1 == XRL_L2_FIRST && XRL_L2_LAST + 1 == XRL_L3_FIRST &&
+              XRL_L3_LAST + 1 == XRL_M1_FIRST && XRL_M1_LAST + 1 == XRL_M2_FIRST && XRL_M2_LAST + 1 == XRL_M3_FIRST &&
+              XRL_M3_LAST + 1 == XRL_M4_FIRST && XRL_M4_LAST + 1 == XRL_M5_FIRST && XRL_M5_LAST < 255,
+              "the shells' lines are consecutive");
+
+/* the line that the number r selects among a shell's by the radiative rates
+ * (first whose cumulative rate exceeds r), 0 for none; rate_cum holds each
+ * shell's running sums, so five probes replace up to 29 dependent ones */
+__device__ __forceinline__ int d_pick_line(const EngineParams &P, int u, int shell, double r) {
+  if (shell < 0 || shell > 8) return 0;
+  int lo = d_shell_first(shell), hi = d_shell_first(shell + 1);
+  const double *cum = P.rate_cum + (size_t)u * (XMI_NLINES_VR_DEV + 1);
+  const int end = hi;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (r < cum[mid]) hi = mid;
+    else lo = mid + 1;
+  }
+  return lo < end ? lo : 0;
+}
+
 /* ------------------------------------------------------------------------ */
 /* cascades of brute-force runs, src/xmi_main.F90:2413-4783 */
 
@@ -1971,22 +2089,9 @@ __device__ __forceinline__ int d_yield_check(const EngineParams &P, int u, int s
 
 /* xmi_fluorescence_line_check (src/xmi_main.F90:5352-5437): the line of a
  * vacancy by the radiative rates, its energy, or 0 and line 0 */
-__device__ double d_line_check(const EngineParams &P, const xrl_atom *a, int u, int shell, phx_stream *s,
-                               int *line) {
-  const double r = phx_uniform(s);
-  *line = 0;
-  if (shell < 0 || shell > 8) return 0.0;
-  int first, last;
-  xrl_shell_lines(shell, &first, &last);
-  double sumz = 0.0;
-  for (int l = first; l <= last; l++) {
-    sumz += a->rad_rate[l];
-    if (r < sumz) {
-      *line = l;
-      return P.line_E[(size_t)u * XMI_NLINES_VR_DEV + (l - 1)];
-    }
-  }
-  return 0.0;
+__device__ double d_line_check(const EngineParams &P, int u, int shell, phx_stream *s, int *line) {
+  *line = d_pick_line(P, u, shell, phx_uniform(s));
+  return *line ? P.line_E[(size_t)u * XMI_NLINES_VR_DEV + (*line - 1)] : 0.0;
 }
 
 /* a cascade's photon in slot j: energy and attenuation, isotropic direction,
@@ -1997,23 +2102,18 @@ __device__ void d_cascade_emit(const EngineParams &P, const PhotonSoA &S, int j,
   S.energy[j] = E;
   d_mu_all(P, E, S.mus, (size_t)P.cap, j);
   S.cflags[j] = 0;
-  const double th = acos(2.0 * phx_uniform(s) - 1.0);
-  const double ph = 2.0 * ENG_PI * phx_uniform(s);
-  const double dirv[3] = {sin(th) * cos(ph), sin(th) * sin(ph), cos(th)};
-  const double r = 2.0 * ENG_PI * phx_uniform(s);
-  double ev[3] = {cos(r), sin(r), 0.0};
-  const double cosalfa = d_dot(ev, dirv);
-  const double c_alfa = acos(cosalfa);
-  const double c_ae = 1.0 / sin(c_alfa), c_be = -c_ae * cosalfa;
-  for (int k = 0; k < 3; k++) ev[k] = c_ae * ev[k] + c_be * dirv[k];
+  const double ct = 2.0 * phx_uniform(s) - 1.0, st = sqrt((1.0 - ct) * (1.0 + ct));
+  double cp, sp, ev[3] = {0.0, 0.0, 0.0};
+  d_turns(phx_uniform(s), &cp, &sp);
+  const double dirv[3] = {st * cp, st * sp, ct};
+  d_turns(phx_uniform(s), &ev[0], &ev[1]);
+  d_update_elecv(dirv, ev);
   S.dx[j] = dirv[0];
   S.dy[j] = dirv[1];
   S.dz[j] = dirv[2];
   S.ex[j] = ev[0];
   S.ey[j] = ev[1];
   S.ez[j] = ev[2];
-  S.theta[j] = th;
-  S.phi[j] = ph;
   S.prev_line[j] = line;
   S.prev_u[j] = u;
 }
@@ -2058,7 +2158,7 @@ __device__ int d_cascade_auger(const EngineParams &P, const PhotonSoA &S, int i,
     if ((m_shell && !P.use_M_lines) || !d_yield_check(P, u, sh[k], s)) continue;
     const int v = d_coster_kronig(a, s, sh[k]);
     int line;
-    const double e = d_line_check(P, a, u, v, s, &line);
+    const double e = d_line_check(P, u, v, s, &line);
     if (e <= 1.0) continue;
     d_cascade_emit(P, S, k == 0 ? i : d_offspring(P, S, i), e, line, u, s);
     spawned = k == 1;
@@ -2086,7 +2186,7 @@ __device__ int d_cascade_radiative(const EngineParams &P, const PhotonSoA &S, in
   if (!d_yield_check(P, u, sn, s)) return 0;
   sn = d_coster_kronig(a, s, sn);
   int ln;
-  const double e = d_line_check(P, a, u, sn, s, &ln);
+  const double e = d_line_check(P, u, sn, s, &ln);
   if (e <= 1.0) return 0;
   S.cflags[i] = 0;
   d_cascade_emit(P, S, d_offspring(P, S, i), e, ln, u, s);
@@ -2104,17 +2204,22 @@ __device__ __forceinline__ int d_photo_one(const EngineParams &P, const PhotonSo
   phx_stream_init(&s, P.seed, P.sample, (uint32_t)n, BRUTE ? d_tr_sub(P, i) : PHX_SUB_TRANSPORT, S.hid[i]);
   d_stream_seek(&s, 3u);
   double E = S.energy[i];
-  xrl_ectx ec = xrl_energy(E);
-  double photo_total = xrl_cs_photo_total_c(a, &ec);
-  double sumz = 0.0;
-  double r = phx_uniform(&s);
-  int max_shell = P.use_M_lines ? 8 : 3;
+  /* the shell by its share of the photo-ionisation: the cross sections are
+   * E^-p times the shells' constants, so E^-p cancels */
+  const double r_sh = phx_uniform(&s);
+  const int max_shell = P.use_M_lines ? 8 : 3;
   int shell = -1;
-  for (int sh = 0; sh <= max_shell; sh++) {
-    sumz += xrl_cs_photo_partial_c(a, sh, &ec) / photo_total;
-    if (r < sumz) {
-      shell = sh;
-      break;
+  {
+    int k = 0;
+#pragma unroll
+    for (int sh = 0; sh < 9; sh++) k += a->edge[sh] > E ? 1 : 0;
+    const double target = r_sh * a->photo_Bsum[k];
+    double sum = 0.0;
+#pragma unroll
+    for (int sh = 0; sh < 9; sh++) {
+      const double e = a->edge[sh];
+      if (sh <= max_shell && e > 0.0 && E >= e) sum += a->photo_B[sh];
+      if (shell < 0 && target < sum) shell = sh;
     }
   }
   S.prev_line[i] = 0;
@@ -2133,17 +2238,7 @@ __device__ __forceinline__ int d_photo_one(const EngineParams &P, const PhotonSo
     S.weight[i] *= P.fycorr[(size_t)u * 9 + shell];
   }
   shell = d_coster_kronig(a, &s, shell);
-  r = phx_uniform(&s);
-  sumz = 0.0;
-  int first, lastl, line = 0;
-  xrl_shell_lines(shell, &first, &lastl);
-  for (int l = first; l <= lastl; l++) {
-    sumz += a->rad_rate[l];
-    if (r < sumz) {
-      line = l;
-      break;
-    }
-  }
+  const int line = d_pick_line(P, u, shell, phx_uniform(&s));
   if (line == 0) {
     S.energy[i] = 0.0;
     return 0;
@@ -2152,12 +2247,12 @@ __device__ __forceinline__ int d_photo_one(const EngineParams &P, const PhotonSo
   S.energy[i] = E;
   for (int l = 0; l < P.n_layers; l++)
     S.mus[(size_t)l * cap + i] = P.precalc_mu[((size_t)l * P.nZ + u) * XMI_NLINES_VR_DEV + (line - 1)];
-  double theta_i = acos(-2.0 * phx_uniform(&s) + 1.0);
-  double phi_i = 2.0 * ENG_PI * phx_uniform(&s);
-  double th = S.theta[i], ph = S.phi[i];
-  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]};
-  double dirv[3];
-  d_update_dirv(dirv, &th, &ph, theta_i, phi_i);
+  /* isotropic: cos theta = 1 - 2 u */
+  const double ui = phx_uniform(&s), ct = fma(-2.0, ui, 1.0), st = 2.0 * sqrt(ui * (1.0 - ui));
+  double ca, sa;
+  d_turns(phx_uniform(&s), &ca, &sa);
+  double ev[3] = {S.ex[i], S.ey[i], S.ez[i]}, dirv[3] = {S.dx[i], S.dy[i], S.dz[i]};
+  d_turn(dirv, d_frame(dirv), ct, st, ca, sa);
   d_update_elecv(dirv, ev);
   S.dx[i] = dirv[0];
   S.dy[i] = dirv[1];
@@ -2165,8 +2260,6 @@ __device__ __forceinline__ int d_photo_one(const EngineParams &P, const PhotonSo
   S.ex[i] = ev[0];
   S.ey[i] = ev[1];
   S.ez[i] = ev[2];
-  S.theta[i] = th;
-  S.phi[i] = ph;
   S.prev_line[i] = line;
   S.prev_u[i] = u;
   if (BRUTE && (S.cflags[i] & 2)) return d_cascade_radiative(P, S, i, u, a, shell, line, &s);
@@ -2234,9 +2327,8 @@ __device__ __forceinline__ int d_interact_entry(const EngineParams &P, const Pho
  * photons that interact at this order, and a wavefront straddles two queues
  * at two places at most.  Each photon is one thread's, with its own random
  * stream, so results do not depend on the assignment. */
-/* occupancy: five waves per SIMD (96 VGPRs, a few spilled; 6 % faster than four).
- * ADV: the advanced Compton model, compiled apart so that the default
- * instance spills less (10 VGPRs instead of 28) */
+/* 72 VGPRs leave seven waves per SIMD.  ADV: the advanced Compton model,
+ * compiled apart */
 template <bool ADV>
 __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
 k_interact(EngineParams P, PhotonSoA S, int n) {
