@@ -49,3 +49,35 @@ def test_lookups_on_moved_grids_match_the_oracle(orc, moved):
     assert np.all(np.abs(vr - ovr) <= 1e-9 * np.maximum(np.abs(ovr), 1e-6 * scale))
     assert np.abs(ch - och).max() <= 1e-9 * och.max()
     prep.close()
+
+
+@pytest.mark.parametrize("moved,n_layers", [(False, 4), (False, 5), (False, 7), (True, 2), (True, 5)])
+def test_estimator_geometry_of_layer_stacks_matches_the_oracle(orc, moved, n_layers):
+    """Every unrolled layer count of the step and its estimator geometry, with
+    the solid angle from a uniform grid and from one that is not."""
+    inp = workloads.single_layer_steel(n_photons_line=20000, n_interactions=3)
+    layer = api.Layer([8, 20, 26], [0.5, 0.3, 0.2], 1.5, 0.05)
+    inp.layers = [api.Layer(list(layer.Z), [0.5 + 0.02 * k, 0.3 - 0.02 * k, 0.2], 1.5 + 0.1 * k, 0.05 + 0.01 * k)
+                  for k in range(n_layers)]
+    inp.reference_layer = (n_layers + 1) // 2
+    inp.discrete[0].energy = 30.0
+    inp.discrete[0].vertical_intensity = 1e9
+    prep = api.Prepared(inp)
+    prep.compute_solid_angle(hits_per_single=200, seed=3)
+    if moved:
+        sa = prep.solid_angle.contents
+        rng = np.random.default_rng(5)
+        for p, n in ((sa.grid_dims_r_vals, sa.grid_dims_r_n), (sa.grid_dims_theta_vals, sa.grid_dims_theta_n)):
+            a = np.ctypeslib.as_array(p, (n,))
+            a[1:-1] += (a[1] - a[0]) * rng.uniform(-0.3, 0.3, n - 2)
+            assert np.all(np.diff(a) > 0)
+    print("stack", n_layers, "grid", "moved" if moved else "uniform", flush=True)
+    ch, vr, _, st = prep.run(seed=9)
+    och, ovr, _, ost = orc.run(prep, seed=9, rng_mode=orc.RNG_PER_HISTORY)
+    assert st.histories == ost.histories and vr.sum() > 0
+    scale = ovr.max()
+    # as above: the photons start in dense layers whose depths, about 0.1 cm
+    # at z = 100 cm +- 1e-14, are given to 1e-13
+    assert np.all(np.abs(vr - ovr) <= 1e-9 * np.maximum(np.abs(ovr), 1e-6 * scale))
+    assert np.abs(ch - och).max() <= 1e-9 * och.max()
+    prep.close()

@@ -59,7 +59,8 @@ struct LayCell {
 };
 
 struct VrSoA {
-  double *theta, *phi;          /* scattering angle to the detector point, azimuth to the polarisation */
+  double *ct, *q;               /* cosine of the scattering angle to the detector point; its sine squared times
+                                   the squared cosine of the azimuth to the polarisation */
   double *omega;                /* solid angle of the detector */
   double *pesc;                 /* escape probability at the photon energy */
   double *dist;                 /* [NL][cap] path by layer, 0 where not crossed */
@@ -179,6 +180,7 @@ struct EngineParams {
   const double *sa_t;
   int sa_nr, sa_nt;
   double sa_r0, sa_rinv, sa_t0, sa_tinv;
+  int sa_uniform;               /* both axes of the solid-angle grid are uniform (d_table) */
   /* tallies */
   unsigned long long *t_ch;     /* [n_int][nch][2] */
   unsigned long long *t_line;   /* [n_int][nZ][ENG_MAX_ACT][2] */

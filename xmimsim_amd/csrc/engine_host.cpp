@@ -1139,6 +1139,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       P.sa_rinv = uniform_inv(solid_angles->grid_dims_r_vals, (int)solid_angles->grid_dims_r_n);
       P.sa_t0 = solid_angles->grid_dims_theta_vals[0];
       P.sa_tinv = uniform_inv(solid_angles->grid_dims_theta_vals, (int)solid_angles->grid_dims_theta_n);
+      P.sa_uniform = grid_uniform(solid_angles->grid_dims_r_vals, (int)solid_angles->grid_dims_r_n) &&
+                     grid_uniform(solid_angles->grid_dims_theta_vals, (int)solid_angles->grid_dims_theta_n);
     }
     /* escape tallies: fluorescence, Compton, normalisation */
     EscParams Q;
@@ -1202,7 +1204,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
 
     VrSoA V;
     char *vp = G.vr.as<char>();
-    double **vfields[] = {&V.theta, &V.phi, &V.omega, &V.pesc, &V.sar, &V.sat};
+    double **vfields[] = {&V.ct, &V.q, &V.omega, &V.pesc, &V.sar, &V.sat};
     for (double **f : vfields) {
       *f = (double *)vp;
       vp += per * sizeof(double);

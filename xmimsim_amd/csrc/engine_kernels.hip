@@ -726,20 +726,20 @@ __device__ __forceinline__ double d_elem_cs_total(const EngineParams &P, int j, 
   return c->pe * pb + (r.T0 + c->cf * r.dT);
 }
 
-/* atom selection and interaction type of the photon in slot i (energy E,
- * now in layer my), from its transport stream after the step's number:
- * S.elem set, the type returned (0 Rayleigh, 1 Compton, 2 photo-absorption) */
+/* atom selection and interaction type of the photon in slot i (energy E, now
+ * in layer my, whose mass attenuation is mu_cur), from its transport stream
+ * after the step's number: S.elem set, the type returned (0 Rayleigh, 1
+ * Compton, 2 photo-absorption).  Both choices compare products instead of
+ * quotients: one division in all */
 __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &S, int i, double E, int my,
-                                        phx_stream *sp) {
+                                        double mu_cur, phx_stream *sp) {
   phx_stream &s = *sp;
-  const size_t cap = (size_t)P.cap;
   /* atom selection, src/xmi_main.F90:1558-1572 */
-  double R2 = phx_uniform(&s);
+  const double target = phx_uniform(&s) * mu_cur;
   int off = P.layer_off[my - 1], nel = P.layer_nel[my - 1];
-  double mu_cur = S.mus[(size_t)(my - 1) * cap + i];
   double thr = 0.0;
   int sel = nel - 1;
-  xrl_ectx ec = xrl_energy(E);
+  xrl_ectx ec = d_energy(E);
   {
     /* the next element's record is loaded before this one's test */
     const size_t ci = (size_t)ec.ci;
@@ -752,8 +752,8 @@ __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &
         rn = P.el_cell[(size_t)(off + k + 1) * XRL_NCS + ci];
         wn = P.el_w[off + k + 1];
       }
-      thr += w * d_elem_cs_total(P, off + k, r, &ec) / mu_cur;
-      if (R2 < thr) {
+      thr = fma(w, d_elem_cs_total(P, off + k, r, &ec), thr);
+      if (target < thr) {
         sel = k;
         break;
       }
@@ -775,8 +775,9 @@ __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &
     while (pos + 2 < len && ie[pos + 1] < E) pos++;
   }
   const double *ir = P.ip_r + P.ip_off[u], *irc = P.ip_rc + P.ip_off[u];
-  double pr = d_interp(ie[pos], ir[pos], ie[pos + 1], ir[pos + 1], E);
-  double pc = d_interp(ie[pos], irc[pos], ie[pos + 1], irc[pos + 1], E);
+  const double f = (E - ie[pos]) / (ie[pos + 1] - ie[pos]);
+  const double pr = fma(ir[pos + 1] - ir[pos], f, ir[pos]);
+  const double pc = fma(irc[pos + 1] - irc[pos], f, irc[pos]);
   return (R3 < pr) ? 0 : ((R3 < pc) ? 1 : 2);
 }
 
@@ -784,118 +785,118 @@ __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &
 #define VR_UP 2
 #define VR_NC_SHIFT 8
 
+/* path lengths through the layers from a point of layer cur along the unit
+ * direction d, itn = d . n_sample, in travel order: entry k is layer k upwards
+ * and layer NL - 1 - k downwards (planes and predicate are then selects of
+ * wave-uniform values), 0 where not crossed.  From plane to plane through the
+ * rounded points, with the reference's divisions: with z about 100 cm the
+ * points carry 1e-14 cm, and a photon that leaves a dense layer from 1e-7 cm
+ * below its surface shows another rounding of them at 1e-7 */
+template <int NL>
+__device__ __forceinline__ void d_layer_walk(const EngineParams &P, const double *from, const double *d, double itn,
+                                             int up, int cur, double *dist) {
+  double lp[3] = {from[0], from[1], from[2]};
+#pragma unroll
+  for (int k = 0; k < NL; k++) {
+    const double z = up ? P.layer_ze[k] : P.layer_zb[NL - 1 - k];
+    const int crossed = up ? k >= cur - 1 && k < P.n_layers : NL - 1 - k <= cur - 1;
+    const double diff[3] = {0.0 - lp[0], 0.0 - lp[1], z - lp[2]};
+    const double t = d_dot(diff, P.n_sample) / itn;
+    const double p[3] = {t * d[0] + lp[0], t * d[1] + lp[1], t * d[2] + lp[2]};
+    dist[k] = crossed ? d_distance(lp, p) : 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) lp[j] = crossed ? p[j] : lp[j];
+  }
+}
+
 /* the geometry of the detection-weight estimator for the photon of slot i,
  * at its interaction point coords (lab frame) with direction dirv_l in layer
  * cur (src/xmi_variance_reduction.F90:29-330): a point of the detector
  * window, the scattering angle and polarisation azimuth towards it, the path
  * through the layers and its escape probability, the solid angle from the
- * grid (or the slot queued for a cone estimate: *need_sa).  Writes the
- * photon's estimator record; returns 1 when there is an event (*info set),
- * 0 for a point behind the window plane. */
+ * grid (or the slot queued for a cone estimate: *need_sa).  mus: the layers'
+ * mass attenuation at the photon's energy.  Writes the photon's estimator
+ * record; returns 1 when there is an event (*info set), 0 for a point behind
+ * the window plane.
+ *
+ * The scattering angle enters the cross sections through its cosine c (the
+ * half angle's sine is sqrt((1 - c) / 2)) and the azimuth through sin^2 theta
+ * cos^2 phi: those two are stored and no angle is formed.  The detector frame
+ * is orthonormal, so c and the distance to the window's centre are taken in
+ * the lab frame. */
 template <int NL>
 __device__ __forceinline__ int d_vr_geom(const EngineParams &P, const PhotonSoA &S, const VrSoA &V, int n, int i,
-                                         const double *coords, const double *dirv_l, int cur, int *need_sa,
-                                         int *info) {
+                                         const double *coords, const double *dirv_l, int cur, const double *mus,
+                                         int *need_sa, int *info) {
   const size_t cap = (size_t)P.cap;
   phx_stream s;
   phx_stream_init(&s, P.seed, P.sample, (uint32_t)n, PHX_SUB_VARRED, S.hid[i]);
-  double radius = sqrt(phx_uniform(&s)) * P.det_radius;
-  double th = 2.0 * ENG_PI * phx_uniform(&s);
-  double dp[3] = {0.0, cos(th) * radius, sin(th) * radius};
-  double rel[3] = {coords[0] - P.p_det[0], coords[1] - P.p_det[1], coords[2] - P.p_det[2]};
-  double lpnt[3], dirv[3], ld[3];
+  const double radius = sqrt(phx_uniform(&s)) * P.det_radius;
+  double ca, sa;
+  d_turns(phx_uniform(&s), &ca, &sa);
+  const double rel[3] = {coords[0] - P.p_det[0], coords[1] - P.p_det[1], coords[2] - P.p_det[2]};
+  double lpnt[3];
   d_matvec(P.det_inv, rel, lpnt);
-  d_matvec(P.det_inv, dirv_l, dirv);
-  for (int k = 0; k < 3; k++) ld[k] = dp[k] - lpnt[k];
-  if (ld[0] >= 0.0) {
-    return 0;
-  } else {
-    double total_distance = d_distance(dp, lpnt);
-    d_normalize(dirv);
-    d_normalize(ld);
-    double nd[3];
-    d_matvec(P.det_new, ld, nd);
-    double c = d_dot(dirv, ld);
-    c = c > 1.0 ? 1.0 : (c < -1.0 ? -1.0 : c);
-    const double theta = acos(c);
-    double proj[3], ndd = d_dot(nd, dirv_l);
-    for (int k = 0; k < 3; k++) proj[k] = nd[k] - ndd * dirv_l[k];
-    d_normalize(proj);
-    double ev[3] = {S.ex[i], S.ey[i], S.ez[i]};
-    double en = d_norm(ev);
-    double evn[3] = {ev[0] / en, ev[1] / en, ev[2] / en};
-    c = d_dot(proj, evn);
-    c = c > 1.0 ? 1.0 : (c < -1.0 ? -1.0 : c);
-    const double phi = acos(c);
-    const int up = d_dot(nd, P.n_sample) > 0.0;
-    const int dir = up ? 1 : -1;
-    const int ncross = up ? P.n_layers - cur + 1 : cur;
-    /* path to the detector through the layers, by layer (0 where not
-     * crossed); the layer holding the detector point ends the walk */
-    double tc[3] = {coords[0], coords[1], coords[2]};
-    int done = 0, nc = 0;
-    double murhod = 0.0;
+  double ld[3] = {-lpnt[0], ca * radius - lpnt[1], sa * radius - lpnt[2]};
+  if (ld[0] >= 0.0) return 0;
+  const double d2 = d_dot(ld, ld), id = d_rsqrt_pos(d2);
+  for (int k = 0; k < 3; k++) ld[k] *= id;
+  double nd[3];
+  d_matvec(P.det_new, ld, nd);
+  const double c0 = d_dot(dirv_l, nd);
+  const double c = c0 > 1.0 ? 1.0 : (c0 < -1.0 ? -1.0 : c0);
+  /* cosine of the angle between the polarisation and the part of nd normal
+   * to the direction, times sin theta, squared */
+  double q;
+  {
+    double proj[3];
+    for (int k = 0; k < 3; k++) proj[k] = fma(-c0, dirv_l[k], nd[k]);
+    const double ev[3] = {S.ex[i], S.ey[i], S.ez[i]};
+    const double pe = d_dot(proj, ev), pp = d_dot(proj, proj) * d_dot(ev, ev);
+    double cf = pp > 0.0 ? pe * d_rsqrt_pos(pp) : 0.0;
+    cf = cf > 1.0 ? 1.0 : (cf < -1.0 ? -1.0 : cf);
+    q = (1.0 - c) * (1.0 + c) * cf * cf;
+  }
+  const double itn = d_dot(nd, P.n_sample);
+  const int up = itn > 0.0;
+  /* path to the detector through the layers (0 where not crossed); the layer
+   * holding the detector point ends the walk */
+  double murhod = 0.0;
+  {
+    double dd[NL], rest = d2 * id;
+    d_layer_walk<NL>(P, coords, nd, itn, up, cur, dd);
 #pragma unroll
     for (int k = 0; k < NL; k++) {
-      const int l0 = cur - 1 + k * dir, back = cur - 2 - k;
-      double dd = 0.0;
-      if (k < ncross) {
-        if (!done) {
-          double pp[3] = {0.0, 0.0, up ? P.layer_ze[l0] : P.layer_zb[l0]}, ip[3];
-          d_intersect(pp, P.n_sample, tc, nd, ip);
-          dd = d_distance(tc, ip);
-          if (!(dd <= total_distance)) {
-            dd = total_distance;
-            done = 1;
-          } else {
-            tc[0] = ip[0];
-            tc[1] = ip[1];
-            tc[2] = ip[2];
-            total_distance -= dd;
-          }
-          murhod += S.mus[(size_t)l0 * cap + i] * P.layer_density[l0] * dd;
-          nc = k + 1;
-        }
-        V.dist[(size_t)l0 * cap + i] = dd;
-      }
-      /* the layers on the other side of the point's own */
-      const int other = up ? back : cur + k;
-      if (up ? back >= 0 : other < P.n_layers) V.dist[(size_t)other * cap + i] = 0.0;
+      dd[k] = dd[k] <= rest ? dd[k] : rest;
+      rest -= dd[k];
+      murhod = fma(up ? mus[k] * P.layer_density[k] : mus[NL - 1 - k] * P.layer_density[NL - 1 - k], dd[k], murhod);
     }
-    /* solid angle, src/xmi_solid_angle_f.F90:712-801 */
-    double omega = 0.0;
-    double r = d_distance(P.p_det, coords);
-    double dv[3] = {coords[0] - P.p_det[0], coords[1] - P.p_det[1], coords[2] - P.p_det[2]};
-    d_normalize(dv);
-    double tt = acos(d_dot(dv, P.n_det));
-    if (tt > ENG_PI / 2.0) tt = ENG_PI - tt;
-    double sth = ENG_PI / 2.0 - tt;
-    if (sth >= P.sa_t[0]) {
-      int p1 = d_findpos_uniform(P.sa_r, P.sa_nr, P.sa_r0, P.sa_rinv, r);
-      int p2 = d_findpos_uniform(P.sa_t, P.sa_nt, P.sa_t0, P.sa_tinv, sth);
-      if (p1 < 0 || p2 < 0) {
-        *need_sa = 1;
-        V.sar[i] = r;
-        V.sat[i] = sth;
-      } else {
-        const double *a1 = P.sa_r, *a2 = P.sa_t;
-        double denom = (a1[p1 + 1] - a1[p1]) * (a2[p2 + 1] - a2[p2]);
-        double c1 = (a1[p1 + 1] - r) * (a2[p2 + 1] - sth) / denom;
-        double c2 = (r - a1[p1]) * (a2[p2 + 1] - sth) / denom;
-        double c3 = (a1[p1 + 1] - r) * (sth - a2[p2]) / denom;
-        double c4 = (r - a1[p1]) * (sth - a2[p2]) / denom;
-        const double *g0 = P.sa_grid + (size_t)p2 * P.sa_nr + p1;
-        const double *g1 = P.sa_grid + (size_t)(p2 + 1) * P.sa_nr + p1;
-        omega = c1 * g0[0] + c2 * g0[1] + c3 * g1[0] + c4 * g1[1];
-      }
-    }
-    V.theta[i] = theta;
-    V.phi[i] = phi;
-    V.omega[i] = omega;
-    V.pesc[i] = exp(-murhod);
-    V.blk[i] = s.ctr[0]; /* two uniforms drawn: block 1, nothing buffered */
-    *info = VR_ACTIVE | (up ? VR_UP : 0) | (nc << VR_NC_SHIFT);
+#pragma unroll
+    for (int l = 0; l < NL; l++)
+      if (l < P.n_layers) V.dist[(size_t)l * cap + i] = up ? dd[l] : dd[NL - 1 - l];
   }
+  /* solid angle, src/xmi_solid_angle_f.F90:712-801 */
+  double omega = 0.0;
+  const double r = sqrt(d_dot(rel, rel));
+  double tt = acos(fmin(fmax(d_dot(rel, P.n_det) / r, -1.0), 1.0));
+  if (tt > ENG_PI / 2.0) tt = ENG_PI - tt;
+  const double sth = ENG_PI / 2.0 - tt;
+  if (sth >= P.sa_t[0]) {
+    if (r > P.sa_r[P.sa_nr - 1] || sth > P.sa_t[P.sa_nt - 1]) {
+      *need_sa = 1;
+      V.sar[i] = r;
+      V.sat[i] = sth;
+    } else {
+      omega = d_table(P.sa_uniform, P.sa_grid, P.sa_t, P.sa_nt, P.sa_t0, P.sa_tinv, P.sa_r, P.sa_nr, P.sa_r0, P.sa_rinv,
+                      sth, r);
+    }
+  }
+  V.ct[i] = c;
+  V.q[i] = q;
+  V.omega[i] = omega;
+  V.pesc[i] = exp(-murhod);
+  V.blk[i] = s.ctr[0]; /* two uniforms drawn: block 1, nothing buffered */
+  *info = VR_ACTIVE | (up ? VR_UP : 0) | ((up ? P.n_layers - cur + 1 : cur) << VR_NC_SHIFT);
   return 1;
 }
 
@@ -909,94 +910,85 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_vr_list(EngineParams P, PhotonSoA
   d_layer_list(P, ev_layer, i);
 }
 
-/* NL bounds the layer count; path lengths and mu*rho are kept in crossing
- * order (k = 0: the photon's layer) so that register arrays are only indexed
- * by compile-time indices */
-/* occupancy: six waves per SIMD up to four layers (80 VGPRs, two spilled;
- * measured 2 % faster than five waves); more layers keep their natural budget */
-/* EST: the estimator's geometry of the new interaction point follows in the
- * same thread (d_vr_geom), while the photon's record is in registers */
+/* NL bounds the layer count; the layers' attenuation is kept by layer and the
+ * path lengths in travel order (d_layer_walk), so that register arrays have
+ * compile-time indices and the layers' constants are wave-uniform; layers
+ * the path does not cross add nothing.
+ * EST: the estimator's geometry of the new interaction point follows in the
+ * same thread (d_vr_geom), while the photon's record is in registers.
+ * Occupancy: as many waves as the registers allow without spills (80 VGPRs up
+ * to three layers, 96 for four, 115 for five, 161 for eight).
+ * Bound by double-precision issue: 1768 vector instructions at three layers
+ * (2487 with angles, a division per layer and choice): 40.9 -> 31.7 ms of the
+ * 1e8-history tube run on three layers */
 template <int NL, bool EST>
-__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(NL <= 4 ? 6 : 1)))
+__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(NL <= 3 ? 6 : NL <= 4 ? 5 : NL <= 5 ? 4 : 1)))
 k_step(EngineParams P, PhotonSoA S, VrSoA V, int n, int count) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   int type = -1, ev_layer = 0, need_sa = 0, info = 0, vr_active = 0;
   const size_t cap = (size_t)P.cap;
-  if (i < count && S.layer[i] > 0) {
-    double E = S.energy[i];
+  const int cur = i < count ? S.layer[i] : 0;
+  if (cur > 0) {
+    const double E = S.energy[i];
     if (E < 1.0) {
       S.layer[i] = 0;
     } else {
       phx_stream s;
       phx_stream_init(&s, P.seed, P.sample, (uint32_t)n, PHX_SUB_TRANSPORT, S.hid[i]);
-      double R = phx_uniform(&s);
-      double dirv[3] = {S.dx[i], S.dy[i], S.dz[i]};
-      double coords[3] = {S.x[i], S.y[i], S.z[i]};
-      double w = S.weight[i];
-      const int cur = S.layer[i];
-      const int up = d_dot(dirv, P.n_sample) > 0.0;
-      const int dir = up ? 1 : -1;
-      const int nc = up ? P.n_layers - cur + 1 : cur; /* layers up to the stack's edge */
-      double dist[NL], md[NL];
-      double lp[3] = {coords[0], coords[1], coords[2]};
+      const double R = phx_uniform(&s);
+      const double dirv[3] = {S.dx[i], S.dy[i], S.dz[i]};
+      const double coords[3] = {S.x[i], S.y[i], S.z[i]};
+      const double itn = d_dot(dirv, P.n_sample);
+      const int up = itn > 0.0;
+      double mus[NL], md[NL], dist[NL]; /* md: by travel order, as dist */
 #pragma unroll
-      for (int k = 0; k < NL; k++) {
-        dist[k] = 0.0;
-        md[k] = 0.0;
-        if (k < nc) {
-          const int l0 = cur - 1 + k * dir;
-          double pp[3] = {0.0, 0.0, up ? P.layer_ze[l0] : P.layer_zb[l0]}, ip[3];
-          d_intersect(pp, P.n_sample, lp, dirv, ip);
-          dist[k] = d_distance(lp, ip);
-          lp[0] = ip[0];
-          lp[1] = ip[1];
-          lp[2] = ip[2];
-          md[k] = S.mus[(size_t)l0 * cap + i] * P.layer_density[l0];
-        }
-      }
+      for (int l = 0; l < NL; l++) mus[l] = l < P.n_layers ? S.mus[(size_t)l * cap + i] : 0.0;
+      d_layer_walk<NL>(P, coords, dirv, itn, up, cur, dist);
       double Pabs = 0.0;
 #pragma unroll
-      for (int k = 0; k < NL; k++)
-        if (k < nc) Pabs += md[k] * dist[k];
-      double Pabs2 = -1.0 * expm1(-1.0 * Pabs);
-      w *= Pabs2;
-      double negln = -1.0 * log1p(-1.0 * R * Pabs2);
-      /* layer of the interaction: first where the optical depth exceeds negln */
-      int kmy = 0, found = 0;
+      for (int k = 0; k < NL; k++) {
+        md[k] = up ? mus[k] * P.layer_density[k] : mus[NL - 1 - k] * P.layer_density[NL - 1 - k];
+        Pabs = fma(md[k], dist[k], Pabs);
+      }
+      const double Pabs2 = -expm1(-Pabs);
+      const double negln = -log1p(-1.0 * R * Pabs2);
+      /* layer of the interaction: first where the optical depth exceeds negln
+       * (rounding may leave none: then the own layer) */
+      int km = up ? cur - 1 : NL - cur, found = 0;
       double sum = 0.0;
 #pragma unroll
       for (int k = 0; k < NL; k++) {
-        if (k < nc && !found) {
-          sum += md[k] * dist[k];
-          if (sum > negln) {
-            kmy = k;
-            found = 1;
-          }
+        sum = fma(md[k], dist[k], sum);
+        if (!found && sum > negln) {
+          km = k;
+          found = 1;
         }
       }
-      double mrm = md[0];
+      const int my = up ? km + 1 : NL - km;
+      double mu_my = mus[0], mrm = md[0];
 #pragma unroll
-      for (int k = 1; k < NL; k++)
-        if (k == kmy) mrm = md[k];
+      for (int l = 1; l < NL; l++) {
+        if (l == my - 1) mu_my = mus[l];
+        if (l == km) mrm = md[l];
+      }
       double tsum = 0.0;
 #pragma unroll
       for (int k = 0; k < NL; k++)
-        if (k <= kmy) tsum += (1.0 - (md[k] / mrm)) * dist[k];
-      tsum = tsum - 1.0 * log1p(-1.0 * R * Pabs2) / mrm;
-      const int my = cur + kmy * dir;
+        if (k < km) tsum += (1.0 - (md[k] / mrm)) * dist[k];
+      tsum = tsum + negln / mrm;
       const double pt[3] = {coords[0] + tsum * dirv[0], coords[1] + tsum * dirv[1], coords[2] + tsum * dirv[2]};
       S.x[i] = pt[0];
       S.y[i] = pt[1];
       S.z[i] = pt[2];
-      S.weight[i] = w;
+      S.weight[i] *= Pabs2;
       S.layer[i] = my;
       /* an estimator event of this order */
       ev_layer = E > 1.0 ? my : 0;
 
       /* atom and type serve the interaction, which the last order of the
        * estimator path does not launch */
-      if (!EST || n < P.n_int) type = d_select(P, S, i, E, my, &s);
-      if (EST && ev_layer) vr_active = d_vr_geom<NL>(P, S, V, n, i, pt, dirv, my, &need_sa, &info);
+      if (!EST || n < P.n_int) type = d_select(P, S, i, E, my, mu_my, &s);
+      if (EST && ev_layer) vr_active = d_vr_geom<NL>(P, S, V, n, i, pt, dirv, my, mus, &need_sa, &info);
     }
   }
   d_enqueue(P, type, i);
@@ -1302,16 +1294,15 @@ __device__ __forceinline__ double d_profile_cdf_eval(const double v[2], double g
  * 752-947 (estimator) with src/xmi_aux_f.F90:1951-2057 (kinematics) */
 
 /* the largest projected momentum an electron of binding energy Ii can carry
- * for scattering by theta (xmi_get_qimax) */
-__device__ __forceinline__ double d_qimax(double energy, double Ii, double theta) {
+ * for scattering by the angle of cosine ct (xmi_get_qimax) */
+__device__ __forceinline__ double d_qimax(double energy, double Ii, double ct) {
   if (Ii != 0.0 && energy < Ii) return 0.0;
-  const double EminIi = energy - Ii, ct = cos(theta);
+  const double EminIi = energy - Ii;
   const double Q = 137.0 * (EminIi * energy * (1.0 - ct) / ENG_MEC2 - Ii);
   return Q / sqrt(EminIi * EminIi + energy * energy - 2.0 * EminIi * energy * ct);
 }
 
-__device__ __forceinline__ double d_q_from_energy(double E0, double E1, double theta) {
-  const double ct = cos(theta);
+__device__ __forceinline__ double d_q_from_energy(double E0, double E1, double ct) {
   const double Q = 137.0 * (E1 - E0 + (1.0 - ct) * E0 * E1 / ENG_MEC2);
   return Q / sqrt(E1 * E1 + E0 * E0 - 2.0 * E0 * E1 * ct);
 }
@@ -1319,8 +1310,7 @@ __device__ __forceinline__ double d_q_from_energy(double E0, double E1, double t
 /* xmi_get_energy_from_q: the root of the quadratic whose momentum has Q's
  * sign; 0 in the reference's exceptions, -1 when no root has it (the
  * reference stops there) */
-__device__ double d_energy_from_q(double E0, double Q, double theta) {
-  const double c = cos(theta);
+__device__ double d_energy_from_q(double E0, double Q, double c) {
   if (fabs(c - 1.0) < 1e-8) return 0.0;
   if (fabs(Q) < 1e-4) return E0 / (1.0 + E0 * (1.0 - c) / ENG_MEC2);
   const double d = 1.0 + E0 / ENG_MEC2 - E0 * c / ENG_MEC2;
@@ -1343,7 +1333,7 @@ __device__ double d_energy_from_q(double E0, double Q, double theta) {
       E2 = t1 < t2 ? t2 : t1;
     }
   }
-  const double Q1 = d_q_from_energy(E0, E1, theta), Q2 = d_q_from_energy(E0, E2, theta);
+  const double Q1 = d_q_from_energy(E0, E1, c), Q2 = d_q_from_energy(E0, E2, c);
   if (Q * Q1 > 0.0) return E1;
   if (Q * Q2 > 0.0) return E2;
   if (fabs(E1 - E2) < 1e-10 || fabs(Q1 - Q2) < 1e-10) return E1;
@@ -1352,8 +1342,8 @@ __device__ double d_energy_from_q(double E0, double Q, double theta) {
 
 /* subshell g's two-sided partial-profile CDF at its Qimax */
 __device__ __forceinline__ double d_adv_cdf(const EngineParams &P, const xrl_atom *a, int g, double energy,
-                                            double theta) {
-  const double q = d_qimax(energy, a->edge[P.cp_sh_idx[g]], theta);
+                                            double ct) {
+  const double q = d_qimax(energy, a->edge[P.cp_sh_idx[g]], ct);
   if (q < -100.0) return 0.0;
   if (q > 100.0) return 1.0;
   const double qp = fabs(q);
@@ -1411,7 +1401,7 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
     const int info = e < lc.tot ? V.info[i] : 0;
     const int mine = info & VR_ACTIVE;
     /* per-photon factors, shared by every element of the layer */
-    double E = 0.0, wo = 0.0, pesc = 0.0, inv_mu = 0.0, c_lamb0 = 1.0, A0 = 0.0, A1 = 0.0, th_e = 0.0;
+    double E = 0.0, wo = 0.0, pesc = 0.0, inv_mu = 0.0, c_lamb0 = 1.0, A0 = 0.0, A1 = 0.0, ct_e = 0.0;
     phx_stream sd; /* advanced model: uniforms from the same stream position */
     /* rho * path by layer (0 where not crossed): in registers for up to five
      * layers, read from the records beyond (register budget) */
@@ -1424,7 +1414,7 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
     for (int k = 0; k < NR; k++) rd[k] = 0.0;
     if (mine) {
       E = S.energy[i];
-      const double theta = V.theta[i], phi = V.phi[i];
+      const double ct = V.ct[i], q = V.q[i], mct = 1.0 - ct;
       wo = V.omega[i] * S.weight[i];
       pesc = V.pesc[i];
       inv_mu = 1.0 / S.mus[(size_t)(L - 1) * cap + i];
@@ -1453,9 +1443,12 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
           sd.ctr[0] = V.blk[i];
         }
       }
-      th_e = theta;
-      dc = xrl_dcsp_setup(E, theta, phi);
-      const double sth2 = sin(theta / 2.0);
+      ct_e = ct;
+      /* xrl_dcsp_setup from cos theta and sin^2 theta cos^2 phi */
+      const double sth2 = sqrt(0.5 * mct), kk = 1.0 / (1.0 + E / XRL_MEC2 * mct);
+      dc.x = E / XRL_KEV_ANGSTROM * sth2;
+      dc.thomson = XRL_RE2 * (1.0 - q);
+      dc.kn = XRL_RE2 * 0.5 * kk * kk * (kk + 1.0 / kk - 2.0 * q);
       c_lamb0 = cc / (E * 1000.0);
       A0 = c0 * sth2 * sth2;
       A1 = c1 * c_lamb0 * sth2;
@@ -1504,13 +1497,13 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
          * uniform each (xmi_compton_varred) */
         const int g0 = P.cp_sh_off[u], g1 = P.cp_sh_off[u + 1];
         double csum = 0.0;
-        for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, th_e);
+        for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct_e);
         const double dcw = Pconv * (xrl_dcsp_compt_c(a, &dc) * wo);
         for (int g = g0; csum != 0.0 && g < g1; g++) {
-          const double cdf = d_adv_cdf(P, a, g, E, th_e);
+          const double cdf = d_adv_cdf(P, a, g, E, ct_e);
           const double sw = a->occupancy[P.cp_sh_idx[g]] * cdf / csum;
           if (sw == 0.0) continue;
-          const double energy = d_energy_from_q(E, d_adv_q(P, g, phx_uniform(&sd) * cdf), th_e);
+          const double energy = d_energy_from_q(E, d_adv_q(P, g, phx_uniform(&sd) * cdf), ct_e);
           if (!(energy > 0.0)) continue;
           const xrl_ectx ce = xrl_energy(energy);
           double m2 = 0.0;
@@ -1879,7 +1872,7 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
     const xrl_atom *a = &P.atoms[u];
     const int g0 = P.cp_sh_off[u], g1 = P.cp_sh_off[u + 1];
     double csum = 0.0;
-    for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, theta_i);
+    for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct);
     if (csum == 0.0) {
       S.energy[i] = 0.0;
       return;
@@ -1888,7 +1881,7 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
     double ts = 0.0, cdf_sel = 0.0;
     int sel = -1, last = g0;
     for (int g = g0; g < g1; g++) {
-      const double w = a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, theta_i);
+      const double w = a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct);
       if (w > 0.0) last = g;
       ts += w / csum;
       if (r <= ts) {
@@ -1897,8 +1890,8 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
       }
     }
     if (sel < 0) sel = last; /* rounding left the running sum just below r */
-    cdf_sel = d_adv_cdf(P, a, sel, E, theta_i);
-    const double e = d_energy_from_q(E, d_adv_q(P, sel, phx_uniform(&s) * cdf_sel), theta_i);
+    cdf_sel = d_adv_cdf(P, a, sel, E, ct);
+    const double e = d_energy_from_q(E, d_adv_q(P, sel, phx_uniform(&s) * cdf_sel), ct);
     if (!(e > 0.0)) {
       S.energy[i] = 0.0;
       return;
@@ -2646,7 +2639,7 @@ __device__ __forceinline__ void d_brute_step(const EngineParams &P, const Photon
     S.y[i] = c[1];
     S.z[i] = c[2];
     S.layer[i] = inside;
-    *type = d_select(P, S, i, E, inside, &s);
+    *type = d_select(P, S, i, E, inside, S.mus[(size_t)(inside - 1) * cap + i], &s);
   }
 }
 
