@@ -81,3 +81,38 @@ def test_estimator_geometry_of_layer_stacks_matches_the_oracle(orc, moved, n_lay
     assert np.all(np.abs(vr - ovr) <= 1e-9 * np.maximum(np.abs(ovr), 1e-6 * scale))
     assert np.abs(ch - och).max() <= 1e-9 * och.max()
     prep.close()
+
+
+@pytest.mark.parametrize("advanced", [False, True])
+def test_compton_profiles_on_moved_grids_match_the_oracle(orc, advanced):
+    """The Doppler draws take cell and fraction from the number on the uniform
+    grids and read the nodes otherwise."""
+    inp = workloads.single_layer_steel(n_photons_line=20000, n_interactions=2)
+    inp.layers[0].Z, inp.layers[0].weight = [6, 8, 26], [0.6, 0.3, 0.1]
+    inp.layers[0].density, inp.layers[0].thickness = 1.5, 1.0
+    inp.discrete[0].energy = 30.0
+    inp.discrete[0].vertical_intensity = 1e9
+    prep = api.Prepared(inp, options=api.default_options(use_advanced_compton=int(advanced)))
+    h = C.cast(prep.hdf5F, C.POINTER(lines.HDF5)).contents
+    rng = np.random.default_rng(6)
+    n = h.Zs[0].cp_len
+    d = rng.uniform(-0.3, 0.3, (3, n))
+    d[:, :2] = d[:, -2:] = 0.0  # the first cell's width places a number in its cell
+    seen = set()
+    for k in range(h.n_Z):
+        z = h.Zs[k]
+        for p, dk in ((z.cp_random_numbers, d[0]),) + (((z.cp_Qs, d[1]), (z.cp_partial_cdf_inv, d[2])) if advanced else ()):
+            if C.addressof(p.contents) in seen:
+                continue
+            seen.add(C.addressof(p.contents))
+            a = np.ctypeslib.as_array(p, (n,))
+            a += (a[1] - a[0]) * dk
+            assert np.all(np.diff(a) > 0)
+    prep.compute_solid_angle(hits_per_single=200, seed=3)
+    print("Compton grids moved", "advanced" if advanced else "", flush=True)
+    ch, vr, _, st = prep.run(seed=9)
+    och, ovr, _, ost = orc.run(prep, seed=9, rng_mode=orc.RNG_PER_HISTORY)
+    assert st.histories == ost.histories and vr.sum() > 0
+    assert np.all(np.abs(vr - ovr) <= 1e-9 * np.maximum(np.abs(ovr), 1e-6 * ovr.max()))
+    assert np.abs(ch - och).max() <= 1e-9 * och.max()
+    prep.close()

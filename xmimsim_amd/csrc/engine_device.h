@@ -115,9 +115,10 @@ struct EngineParams {
   const double *lay_edge;       /* [lay_eoff[l] .. lay_eoff[l+1]) */
   const double *lay_pb;         /* [lay_eoff[l] + l .. lay_eoff[l+1] + l] */
   const int *lay_kstart;        /* [n_layers][XRL_NCS] */
-  const struct LayCell *lay_cell; /* [n_layers][XRL_NCS] */
-  const struct LayCell *el_cell;  /* [elements of the layers, layer_off order][XRL_NCS]: each element's own
-                                     total cross section (K counts its own edges) */
+  const struct LayCell *lay_cell; /* [XRL_NCS][n_layers]: an energy's layers side by side */
+  const struct LayCell *el_cell;  /* [XRL_NCS][n_lay_el], elements of the layers in layer_off order: each element's
+                                     own total cross section (K counts its own edges) */
+  int n_lay_el;
   int lay_eoff[ENG_MAX_LAYERS + 1];
   /* per element */
   const xrl_atom *atoms;        /* [nZ] */
@@ -137,6 +138,8 @@ struct EngineParams {
   double ip_acc_E0, ip_acc_inv;
   const double *cp_icdf;        /* [nZ][cp_len] */
   const double *cp_rn;          /* [cp_len] shared */
+  double cp_rn_inv;             /* nodes per unit of cp_rn */
+  int cp_rn_uniform;            /* cp_rn starts at 0 in equal steps */
   int cp_len;
   const double *cp_cdfg;        /* [nZ][XMI_CP_GRID] profile CDF on a uniform momentum grid */
   const double *cp_gscale;      /* [nZ] grid points per unit momentum */
@@ -148,6 +151,8 @@ struct EngineParams {
   int adv_compton;
   const int *cp_sh_off, *cp_sh_idx;
   const double *cp_pcdf, *cp_qinv, *cp_Qs, *cp_inv;
+  double cp_Qs_rcp, cp_inv_rcp; /* their nodes per unit */
+  int cp_adv_uniform;           /* both start at 0 in equal steps */
   const double *precalc_xrf;    /* [nZ][9][nZ][219] */
   const double *line_E;         /* [nZ][219] */
   const double *rate_cum;       /* [nZ][220] radiative rates summed along each shell's lines, index |line| */
@@ -226,10 +231,18 @@ __device__ __forceinline__ void fx_split(double v, int shift, unsigned long long
     *hi = 0ull;
     return;
   }
-  double t = ldexp(v, shift - 64);
-  double th = trunc(t);
-  *hi = (unsigned long long)th;
-  *lo = (unsigned long long)ldexp(t - th, 64);
+  /* v = m 2^e with the 53-bit integer m: v 2^shift is m shifted by sh = e +
+   * shift, truncated */
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned long long m = (b & 0x000fffffffffffffull) | 0x0010000000000000ull;
+  const int sh = (int)(b >> 52) - 1075 + shift;
+  if (sh >= 0) {
+    *lo = sh < 64 ? m << sh : 0ull;
+    *hi = sh > 75 ? ~0ull : (sh < 64 ? (m >> 1) >> (63 - sh) : m << (sh - 64));
+  } else {
+    *lo = sh > -64 ? m >> -sh : 0ull;
+    *hi = 0ull;
+  }
 }
 
 __device__ __forceinline__ void fx_add_global(unsigned long long *bin, double v, int shift) {

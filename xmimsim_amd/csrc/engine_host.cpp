@@ -248,6 +248,10 @@ struct DeviceTables {
   double tab_E0 = 0, tab_Einv = 0, tab_R0 = 0, tab_Rinv = 0, phi_T0 = 0, phi_Tinv = 0, phi_R0 = 0, phi_Rinv = 0;
   double ip_acc_E0 = 0, ip_acc_inv = 0;
   int tab_uniform = 0; /* the angle and azimuth tables' grids are uniform */
+  int cp_rn_uniform = 0;  /* the Compton profiles' random numbers start at 0 in equal steps */
+  double cp_rn_inv = 0.0; /* and their nodes per unit */
+  int cp_adv_uniform = 0; /* so do the subshell profiles' two grids */
+  double cp_Qs_rcp = 0.0, cp_inv_rcp = 0.0;
 };
 
 /* device copies of the tables of each xmi_hdf5F handle, shared by all engines */
@@ -392,6 +396,9 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
   t->phi_Rinv = uniform_inv(h->RandomNumbers, h->phi_n_r);
   t->tab_uniform = grid_uniform(z0->Energies, t->n_e) && grid_uniform(z0->RandomNumbers, t->n_r) &&
                    grid_uniform(h->Thetas, h->phi_n_theta) && grid_uniform(h->RandomNumbers, h->phi_n_r);
+  t->cp_rn_uniform = z0->cp_random_numbers[0] == 0.0 && grid_uniform(z0->cp_random_numbers, t->cp_len);
+  t->cp_rn_inv = t->cp_rn_uniform ? uniform_inv(z0->cp_random_numbers, t->cp_len)
+                                  : 1.0 / (z0->cp_random_numbers[1] - z0->cp_random_numbers[0]);
   hipError_t e = hipSuccess;
   e = upload(t->atoms, atoms.data(), atoms.size(), st, sg);
   if (e == hipSuccess) e = upload(t->rate_cum, rcum.data(), rcum.size(), st, sg);
@@ -445,6 +452,10 @@ static int ensure_adv_tables(DeviceTables *t, const xmi_hdf5F *h, hipStream_t st
   off[nZ] = (int)idx.size();
   hipError_t e = upload(t->cp_shoff, off.data(), off.size(), st, sg);
   if (e == hipSuccess) e = upload(t->cp_shidx, idx.data(), idx.size(), st, sg);
+  const double *Qs = h->Zs[0].cp_Qs, *ci = h->Zs[0].cp_partial_cdf_inv;
+  t->cp_adv_uniform = Qs[0] == 0.0 && ci[0] == 0.0 && grid_uniform(Qs, N) && grid_uniform(ci, N);
+  t->cp_Qs_rcp = t->cp_adv_uniform ? uniform_inv(Qs, N) : 1.0 / (Qs[1] - Qs[0]);
+  t->cp_inv_rcp = t->cp_adv_uniform ? uniform_inv(ci, N) : 1.0 / (ci[1] - ci[0]);
   if (e == hipSuccess) e = upload(t->cp_pcdf, pcdf.data(), pcdf.size(), st, sg);
   if (e == hipSuccess) e = upload(t->cp_qinv, qinv.data(), qinv.size(), st, sg);
   if (e == hipSuccess) e = upload(t->cp_Qs, h->Zs[0].cp_Qs, (size_t)N, st, sg);
@@ -706,7 +717,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     for (int l = 0; l < NL; l++) {
       const int eo = P.lay_eoff[l], ne = P.lay_eoff[l + 1] - eo;
       for (int c = 0; c < XRL_NCS; c++) {
-        LayCell &r = lay_cell[(size_t)l * XRL_NCS + c];
+        LayCell &r = lay_cell[(size_t)c * NL + l];
         const double *T = &lay_rc[(size_t)l * XRL_NCS];
         r.T0 = T[c];
         r.dT = c + 1 < XRL_NCS ? T[c + 1] - T[c] : 0.0;
@@ -733,7 +744,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       std::sort(ed.begin(), ed.end(), [](double x, double y) { return x > y; });
       const int ne = (int)ed.size();
       for (int c = 0; c < XRL_NCS; c++) {
-        LayCell &r = el_cell[j * XRL_NCS + c];
+        LayCell &r = el_cell[c * elZ.size() + j];
         r.T0 = a->cs_rc[c];
         r.dT = c + 1 < XRL_NCS ? a->cs_rc[c + 1] - a->cs_rc[c] : 0.0;
         const double e_hi = g_cells.hi[c], e_lo = g_cells.lo[c];
@@ -1086,6 +1097,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.ip_acc_inv = T->ip_acc_inv;
     P.cp_icdf = T->cp_icdf.as<double>();
     P.cp_rn = T->cp_rn.as<double>();
+    P.cp_rn_inv = T->cp_rn_inv;
+    P.cp_rn_uniform = T->cp_rn_uniform;
     P.cp_len = T->cp_len;
     P.cp_cdfg = T->cp_cdfg.as<double>();
     P.cp_gscale = T->cp_gscale.as<double>();
@@ -1097,6 +1110,9 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       P.cp_qinv = T->cp_qinv.as<double>();
       P.cp_Qs = T->cp_Qs.as<double>();
       P.cp_inv = T->cp_inv.as<double>();
+      P.cp_Qs_rcp = T->cp_Qs_rcp;
+      P.cp_inv_rcp = T->cp_inv_rcp;
+      P.cp_adv_uniform = T->cp_adv_uniform;
     }
     P.precalc_xrf = T->precalc_xrf.as<double>();
     P.line_E = T->lineE.as<double>();
@@ -1120,6 +1136,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.lay_kstart = G.lay_kstart.as<int>();
     P.lay_cell = G.lay_cell.as<LayCell>();
     P.el_cell = G.el_cell.as<LayCell>();
+    P.n_lay_el = (int)elZ.size();
     P.phi_icdf = T->phi.as<double>();
     P.phi_T = T->phiT.as<double>();
     P.phi_R = T->phiR.as<double>();

@@ -87,6 +87,14 @@ __device__ __forceinline__ double d_rsqrt_pos(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+/* 1 / x for normal x away from the range's ends: the instruction's seed and
+ * one cubic step, a third of an IEEE division's issue */
+__device__ __forceinline__ double d_rcp(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+
 /* E^-p of the photo-ionisation cross sections (p = 11/4) for an energy in the
  * provider's range: E^(-1/2) cubed twice times E^(1/4), from two reciprocal
  * square roots; 0 for E <= 0, as xrl_energy */
@@ -204,18 +212,21 @@ __device__ __forceinline__ void d_turns(double u, double *c, double *s) {
 /* mass attenuation of a layer, sum_i w_i CS_Total(Z_i, E) (src/xmi_aux_f.F90:1109-1141),
  * from the per-layer tables: equal to the element sum up to rounding, since
  * the layer sums are formed once on the host */
-__device__ __forceinline__ double d_layer_mu_tab(const EngineParams &P, int layer0, const xrl_ectx *c) {
-  if (!(c->E > 0.0)) return 0.0;
-  const LayCell r = P.lay_cell[(size_t)layer0 * XRL_NCS + c->ci];
+__device__ __forceinline__ double d_cell_mu(const EngineParams &P, int layer0, const LayCell &r, const xrl_ectx &c) {
   double pb = r.pb;
   if (!r.edge_free) {
     /* an edge inside the cell: count the edges above E */
     const int eo = P.lay_eoff[layer0], ne = P.lay_eoff[layer0 + 1] - eo;
     int K = r.K;
-    while (K < ne && P.lay_edge[eo + K] > c->E) K++;
+    while (K < ne && P.lay_edge[eo + K] > c.E) K++;
     pb = P.lay_pb[eo + layer0 + K];
   }
-  return c->pe * pb + (r.T0 + c->cf * r.dT);
+  return fma(c.pe, pb, fma(c.cf, r.dT, r.T0));
+}
+
+__device__ __forceinline__ double d_layer_mu_tab(const EngineParams &P, int layer0, const xrl_ectx *c) {
+  if (!(c->E > 0.0)) return 0.0;
+  return d_cell_mu(P, layer0, P.lay_cell[(size_t)c->ci * P.n_layers + layer0], *c);
 }
 
 __device__ __forceinline__ void d_mu_all(const EngineParams &P, double E, double *mus, size_t stride, size_t idx) {
@@ -742,14 +753,14 @@ __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &
   xrl_ectx ec = d_energy(E);
   {
     /* the next element's record is loaded before this one's test */
-    const size_t ci = (size_t)ec.ci;
-    LayCell rn = P.el_cell[(size_t)off * XRL_NCS + ci];
+    const LayCell *cell = P.el_cell + (size_t)ec.ci * P.n_lay_el + off;
+    LayCell rn = cell[0];
     double wn = P.el_w[off];
     for (int k = 0; k < nel; k++) {
       const LayCell r = rn;
       const double w = wn;
       if (k + 1 < nel) {
-        rn = P.el_cell[(size_t)(off + k + 1) * XRL_NCS + ci];
+        rn = cell[k + 1];
         wn = P.el_w[off + k + 1];
       }
       thr = fma(w, d_elem_cs_total(P, off + k, r, &ec), thr);
@@ -783,7 +794,6 @@ __device__ __forceinline__ int d_select(const EngineParams &P, const PhotonSoA &
 
 #define VR_ACTIVE 1
 #define VR_UP 2
-#define VR_NC_SHIFT 8
 
 /* path lengths through the layers from a point of layer cur along the unit
  * direction d, itn = d . n_sample, in travel order: entry k is layer k upwards
@@ -896,7 +906,7 @@ __device__ __forceinline__ int d_vr_geom(const EngineParams &P, const PhotonSoA 
   V.omega[i] = omega;
   V.pesc[i] = exp(-murhod);
   V.blk[i] = s.ctr[0]; /* two uniforms drawn: block 1, nothing buffered */
-  *info = VR_ACTIVE | (up ? VR_UP : 0) | ((up ? P.n_layers - cur + 1 : cur) << VR_NC_SHIFT);
+  *info = VR_ACTIVE | (up ? VR_UP : 0);
   return 1;
 }
 
@@ -1110,26 +1120,107 @@ __device__ __forceinline__ double d_wave_total(double v) {
   return d_readlane(v, 63);
 }
 
-/* e^x for x <= 0, table-driven (P. T. P. Tang, "Table-driven implementation
- * of the exponential function in IEEE floating-point arithmetic", ACM TOMS
- * 15(2), 1989): x = (64 m + j) ln2/64 + r with |r| <= ln2/128, so
- * e^x = 2^m * 2^(j/64) * e^r; e^r - 1 is its Taylor polynomial of degree 5
- * (truncation below 4e-17 relative).  tab[j] = 2^(j/64), j = 0..63.
- * Arguments below -746 give 0, as e^x underflows there. */
-__device__ __forceinline__ double d_exp_neg(double x, const double *tab) {
-  x = fmax(x, -746.0);
-  const double n = rint(x * 92.33248261689366);          /* 64 / ln 2 */
-  double r = fma(-n, 0.010830424696249145, x);           /* ln2/64, leading part */
-  r = fma(-n, 3.623510646634843e-19, r);                 /* ln2/64, trailing part */
-  const int ni = (int)n;
-  double q = fma(r, 1.0 / 120.0, 1.0 / 24.0);
-  q = fma(r, q, 1.0 / 6.0);
-  q = fma(r, q, 0.5);
-  const double p = fma(r * r, q, r);
-  const double T = tab[ni & 63];
-  return ldexp(fma(T, p, T), ni >> 6);
+/* the wavefront's sums of a and of b, in a fixed order: the halves exchanged
+ * first (a's sums then live in lanes 0 to 31, b's in 32 to 63), so that one
+ * row reduction serves both */
+__device__ __forceinline__ void d_wave_total2(double a, double b, double *ta, double *tb) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  double v = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+             __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+  v += d_dpp0<0x111, 0xf>(v); /* row_shr:1 */
+  v += d_dpp0<0x112, 0xf>(v); /* row_shr:2 */
+  v += d_dpp0<0x114, 0xf>(v); /* row_shr:4 */
+  v += d_dpp0<0x118, 0xf>(v); /* row_shr:8: lane 15 of a row holds its sum */
+  v += d_dpp0<0x142, 0xa>(v); /* row_bcast:15 into rows 1 and 3 */
+  *ta = d_readlane(v, 31);
+  *tb = d_readlane(v, 63);
 }
 
+/* The scattering kernel's tables in LDS: 2^(j/64) for the exponential and,
+ * for a mantissa m in [1 + j/128, 1 + (j+1)/128), the rounded reciprocal of
+ * the interval's middle with its logarithm in cells of the ln E grid (from
+ * the grid's first node) and its power 11/4. */
+#define ENG_LOG_LOG2 7
+#define ENG_LOG_N (1 << ENG_LOG_LOG2)
+struct ScatterTab {
+  double exp2t[64];
+  double inv[ENG_LOG_N], cell[ENG_LOG_N], pw[ENG_LOG_N];
+};
+
+__device__ __forceinline__ void d_scatter_tab(ScatterTab *t) {
+  const int j = threadIdx.x;
+  if (j < 64) t->exp2t[j] = exp2((double)j / 64.0);
+  if (j < ENG_LOG_N) {
+    const double inv = 1.0 / (1.0 + ((double)j + 0.5) / ENG_LOG_N);
+    t->inv[j] = inv;
+    t->cell[j] = (-log(inv) - XRL_CS_LNE0) * ((double)(XRL_NCS - 1) / (XRL_CS_LNE1 - XRL_CS_LNE0));
+    t->pw[j] = pow(inv, XRL_PHOTO_EXPONENT);
+  }
+}
+
+/* the provider's energy context (xrl_energy) by table: E = 2^k m, r = m inv_j
+ * - 1 with |r| <= 1/256, so that ln E = k ln 2 - ln inv_j + ln(1 + r) and E^-p =
+ * 2^(-11 k / 4) inv_j^p (1 + r)^-p; both series to r^7 (1e-20 and 1e-18).
+ * Table-driven as P. T. P. Tang, "Table-driven implementation of the
+ * logarithm function in IEEE floating-point arithmetic", ACM TOMS 16(4),
+ * 1990.  The logarithm carries 2e-16 absolute, as a correctly rounded one
+ * does in these cells' units. */
+__device__ __forceinline__ xrl_ectx d_energy_tab(double E, const ScatterTab &t) {
+  xrl_ectx c;
+  c.E = E;
+  c.pe = c.cf = 0.0;
+  c.ci = 0;
+  if (!(E > 0.0)) return c;
+  constexpr double inv_h = (double)(XRL_NCS - 1) / (XRL_CS_LNE1 - XRL_CS_LNE0);
+  const long long b = __double_as_longlong(E);
+  const int hi = (int)(b >> 32), k = (hi >> 20) - 1023, j = (hi >> (20 - ENG_LOG_LOG2)) & (ENG_LOG_N - 1);
+  const double m = __longlong_as_double((b & 0x000fffffffffffffll) | 0x3ff0000000000000ll);
+  const double r = fma(m, t.inv[j], -1.0);
+  double q = fma(r, inv_h / 7.0, -inv_h / 6.0);
+  q = fma(r, q, inv_h / 5.0);
+  q = fma(r, q, -inv_h / 4.0);
+  q = fma(r, q, inv_h / 3.0);
+  q = fma(r, q, -inv_h / 2.0);
+  q = fma(r, q, inv_h);
+  const double x = fma(r, q, fma((double)k, 0.6931471805599453 * inv_h, t.cell[j]));
+  int i = (int)x;
+  i = i < 0 ? 0 : (i > XRL_NCS - 2 ? XRL_NCS - 2 : i);
+  c.ci = i;
+  c.cf = x - (double)i;
+  /* binomial series of exponent -11/4 */
+  constexpr double p = XRL_PHOTO_EXPONENT, b1 = -p, b2 = b1 * (-p - 1.0) / 2.0, b3 = b2 * (-p - 2.0) / 3.0,
+                   b4 = b3 * (-p - 3.0) / 4.0, b5 = b4 * (-p - 4.0) / 5.0, b6 = b5 * (-p - 5.0) / 6.0,
+                   b7 = b6 * (-p - 6.0) / 7.0;
+  double w = fma(r, b7, b6);
+  w = fma(r, w, b5);
+  w = fma(r, w, b4);
+  w = fma(r, w, b3);
+  w = fma(r, w, b2);
+  w = fma(r, w, b1);
+  const double s = t.pw[j] * t.exp2t[(k & 3) * 16];
+  c.pe = ldexp(fma(s, w * r, s), (k >> 2) - 3 * k); /* -11 k / 4 = -3 k + k / 4 */
+  return c;
+}
+
+/* e^-m from t = -m ENG_EXP64 (m >= 0), table-driven (P. T. P. Tang, "Table-
+ * driven implementation of the exponential function in IEEE floating-point
+ * arithmetic", ACM TOMS 15(2), 1989): t = 64 k + j + f with |f| <= 1/2, the
+ * value 2^k 2^(j/64) 2^(f/64), the last factor its Taylor polynomial of
+ * degree 5 (4e-17); ldexp underflows to 0 by itself */
+#define ENG_EXP64 92.33248261689366 /* 64 / ln 2 */
+__device__ __forceinline__ double d_exp64(double t, const ScatterTab &tab) {
+  constexpr double h = 0.6931471805599453 / 64.0;
+  const double n = rint(t), f = t - n;
+  const int ni = (int)n;
+  double q = fma(f, h * h * h * h * h / 120.0, h * h * h * h / 24.0);
+  q = fma(f, q, h * h * h / 6.0);
+  q = fma(f, q, h * h / 2.0);
+  q = fma(f, q, h);
+  const double T = tab.exp2t[ni & 63];
+  return ldexp(fma(T, q * f, T), ni >> 6);
+}
 
 /* e^-m from t = -m ENG_EXP_UNIT, for a factor that tables and coefficients
  * hold in these units: t = 512 k + j + f with |f| <= 1/2, so the value is
@@ -1224,70 +1315,39 @@ __device__ __forceinline__ bool d_chunk_next(const EngineParams &P, LayerChunks 
   return c < w.c_end;
 }
 
-/* 32-bit words of a lane's Philox stream, two blocks deep: the current
- * block (a, na words left) and the next one (b, when hasb).  Refills are
- * wave-collective: when an active lane is about to need a block it has not
- * computed, every active lane without a next block computes its next one.
- * Lanes empty their blocks at different trials, so a refill per lane would
- * run the Philox rounds at nearly every trial of a wavefront; this way a
- * wavefront runs them about once per four trials.  The words come out in
- * the stream's order (blocks ctr, ctr + 1, ...; each block's words first to
- * last), as phx_word gives them. */
-struct WaveWords {
-  uint32_t a[4], b[4];
-  uint32_t ctr[4], key[2];
-  int na, hasb;
-};
-
-__device__ __forceinline__ uint32_t d_ww_word(WaveWords &w) {
-  if (__ballot(w.na == 0 && !w.hasb)) {
-    if (!w.hasb) {
-      phx_4x32_10(w.ctr, w.key, w.b);
-      w.ctr[0]++;
-      w.hasb = 1;
-    }
-  }
-  if (w.na == 0) {
-    w.a[0] = w.b[0];
-    w.a[1] = w.b[1];
-    w.a[2] = w.b[2];
-    w.a[3] = w.b[3];
-    w.na = 4;
-    w.hasb = 0;
-  }
-  const uint32_t x = w.a[0];
-  w.a[0] = w.a[1];
-  w.a[1] = w.a[2];
-  w.a[2] = w.a[3];
-  w.na--;
-  return x;
+/* row[] at x >= 0 of a grid whose cells start near x * inv: on the uniform
+ * grids of the generator cell and fraction come from x itself (d_table) */
+__device__ __forceinline__ double d_grid_lookup(int uniform, const double *grid, const double *row, int len, double inv,
+                                               double x) {
+  const double t = x * inv;
+  int pos = (int)t;
+  if (pos > len - 2) pos = len - 2;
+  const double f = uniform ? t - (double)pos : (x - grid[pos]) * d_rcp(grid[pos + 1] - grid[pos]);
+  return fma(row[pos + 1] - row[pos], f, row[pos]);
 }
 
 /* the Compton profile's CDF at momentum pz from its grid (the
  * xmi_profile_cdf_grid table of the element; gs grid points per unit
  * momentum), clamped to the grid's last point, 0 for pz <= 0; in two parts,
  * so that the grid values of one element can be loaded while the previous
- * element is scored: the two grid values the lookup interpolates between,
- * then the linear interpolation */
-__device__ __forceinline__ void d_profile_cdf_load(const double *g, double gs, double pz, double v[2]) {
-  v[0] = v[1] = 0.0;
+ * element is scored: the two grid values and the fraction of the lookup, then
+ * the interpolation */
+struct CdfPair {
+  double v0, v1, f;
+};
+
+__device__ __forceinline__ void d_profile_cdf_load(const double *g, double gs, double pz, CdfPair *p) {
+  p->v0 = p->v1 = p->f = 0.0;
   if (!(pz > 0.0)) return;
-  const double x = pz * gs;
-  if (x >= (double)(XMI_CP_GRID - 1)) {
-    v[0] = v[1] = g[XMI_CP_GRID - 1];
-    return;
-  }
-  const int j = (int)x;
-  v[0] = g[j];
-  v[1] = g[j + 1];
+  const double x = fmin(pz * gs, (double)(XMI_CP_GRID - 1));
+  int j = (int)x;
+  j = j > XMI_CP_GRID - 2 ? XMI_CP_GRID - 2 : j;
+  p->v0 = g[j];
+  p->v1 = g[j + 1];
+  p->f = x - (double)j;
 }
 
-__device__ __forceinline__ double d_profile_cdf_eval(const double v[2], double gs, double pz) {
-  if (!(pz > 0.0)) return 0.0;
-  const double x = pz * gs;
-  if (x >= (double)(XMI_CP_GRID - 1)) return v[0];
-  return v[0] + (v[1] - v[0]) * (x - (double)(int)x);
-}
+__device__ __forceinline__ double d_profile_cdf_eval(const CdfPair &p) { return fma(p.v1 - p.v0, p.f, p.v0); }
 
 /* ---- the advanced Compton model (use_advanced_compton) ------------------
  * src/xmi_main.F90:4785-4983 (transport) and src/xmi_variance_reduction.F90:
@@ -1298,13 +1358,18 @@ __device__ __forceinline__ double d_profile_cdf_eval(const double v[2], double g
 __device__ __forceinline__ double d_qimax(double energy, double Ii, double ct) {
   if (Ii != 0.0 && energy < Ii) return 0.0;
   const double EminIi = energy - Ii;
-  const double Q = 137.0 * (EminIi * energy * (1.0 - ct) / ENG_MEC2 - Ii);
-  return Q / sqrt(EminIi * EminIi + energy * energy - 2.0 * EminIi * energy * ct);
+  const double Q = 137.0 * (EminIi * energy * (1.0 - ct) * (1.0 / ENG_MEC2) - Ii);
+  return Q * d_rsqrt_pos(EminIi * EminIi + energy * energy - 2.0 * EminIi * energy * ct);
 }
 
+/* the projected momentum of an energy E1, without its positive denominator
+ * (xmi_get_q_from_energy's sign) */
 __device__ __forceinline__ double d_q_from_energy(double E0, double E1, double ct) {
-  const double Q = 137.0 * (E1 - E0 + (1.0 - ct) * E0 * E1 / ENG_MEC2);
-  return Q / sqrt(E1 * E1 + E0 * E0 - 2.0 * E0 * E1 * ct);
+  return 137.0 * (E1 - E0 + (1.0 - ct) * E0 * E1 * (1.0 / ENG_MEC2));
+}
+
+__device__ __forceinline__ double d_q_denom(double E0, double E1, double ct) {
+  return sqrt(E1 * E1 + E0 * E0 - 2.0 * E0 * E1 * ct);
 }
 
 /* xmi_get_energy_from_q: the root of the quadratic whose momentum has Q's
@@ -1312,8 +1377,8 @@ __device__ __forceinline__ double d_q_from_energy(double E0, double E1, double c
  * reference stops there) */
 __device__ double d_energy_from_q(double E0, double Q, double c) {
   if (fabs(c - 1.0) < 1e-8) return 0.0;
-  if (fabs(Q) < 1e-4) return E0 / (1.0 + E0 * (1.0 - c) / ENG_MEC2);
-  const double d = 1.0 + E0 / ENG_MEC2 - E0 * c / ENG_MEC2;
+  if (fabs(Q) < 1e-4) return E0 * d_rcp(1.0 + E0 * (1.0 - c) * (1.0 / ENG_MEC2));
+  const double d = 1.0 + E0 * (1.0 / ENG_MEC2) - E0 * c * (1.0 / ENG_MEC2);
   const double aq = 137.0 * 137.0 * d * d - Q * Q;
   const double bq = -2.0 * 137.0 * 137.0 * E0 * d + 2.0 * E0 * c * Q * Q;
   const double cq = 137.0 * 137.0 * E0 * E0 - E0 * E0 * Q * Q;
@@ -1324,58 +1389,105 @@ __device__ double d_energy_from_q(double E0, double Q, double c) {
   } else {
     const double delta = bq * bq - 4.0 * aq * cq;
     if (delta < 0.0) return 0.0;
+    const double ia = 0.5 * d_rcp(aq);
     if (delta == 0.0) {
-      E1 = E2 = -bq / 2.0 / aq;
+      E1 = E2 = -bq * ia;
     } else {
-      const double sd = sqrt(delta);
-      const double t1 = (-bq + sd) / 2.0 / aq, t2 = (-bq - sd) / 2.0 / aq;
+      const double sd = d_sqrt_pos(delta);
+      const double t1 = (-bq + sd) * ia, t2 = (-bq - sd) * ia;
       E1 = t1 < t2 ? t1 : t2;
       E2 = t1 < t2 ? t2 : t1;
     }
   }
-  const double Q1 = d_q_from_energy(E0, E1, c), Q2 = d_q_from_energy(E0, E2, c);
-  if (Q * Q1 > 0.0) return E1;
-  if (Q * Q2 > 0.0) return E2;
-  if (fabs(E1 - E2) < 1e-10 || fabs(Q1 - Q2) < 1e-10) return E1;
+  const double N1 = d_q_from_energy(E0, E1, c), N2 = d_q_from_energy(E0, E2, c);
+  if (Q * N1 > 0.0) return E1;
+  if (Q * N2 > 0.0) return E2;
+  if (fabs(E1 - E2) < 1e-10 || fabs(N1 / d_q_denom(E0, E1, c) - N2 / d_q_denom(E0, E2, c)) < 1e-10) return E1;
   return -1.0;
 }
 
-/* subshell g's two-sided partial-profile CDF at its Qimax */
-__device__ __forceinline__ double d_adv_cdf(const EngineParams &P, const xrl_atom *a, int g, double energy,
-                                            double ct) {
-  const double q = d_qimax(energy, a->edge[P.cp_sh_idx[g]], ct);
+/* subshell g's two-sided partial-profile CDF at its Qimax (binding energy Ii) */
+__device__ __forceinline__ double d_adv_cdf(const EngineParams &P, double Ii, int g, double energy, double ct) {
+  const double q = d_qimax(energy, Ii, ct);
   if (q < -100.0) return 0.0;
   if (q > 100.0) return 1.0;
-  const double qp = fabs(q);
-  const double *Qs = P.cp_Qs, *pc = P.cp_pcdf + (size_t)g * P.cp_len;
-  int pos = (int)(qp / (Qs[1] - Qs[0]));
-  if (pos > P.cp_len - 2) pos = P.cp_len - 2;
-  const double v = d_interp(Qs[pos], pc[pos], Qs[pos + 1], pc[pos + 1], qp);
+  const double v = d_grid_lookup(P.cp_adv_uniform, P.cp_Qs, P.cp_pcdf + (size_t)g * P.cp_len, P.cp_len, P.cp_Qs_rcp, fabs(q));
   return q < 0.0 ? 1.0 - (0.5 + v) : 0.5 + v;
 }
 
 /* the projected momentum at a value cdf of subshell g's two-sided profile */
 __device__ __forceinline__ double d_adv_q(const EngineParams &P, int g, double cdf) {
-  const double *inv = P.cp_inv, *qi = P.cp_qinv + (size_t)g * P.cp_len;
   const double cp = cdf < 0.5 ? 0.5 - cdf : cdf - 0.5;
-  int pos = (int)(cp / (inv[1] - inv[0]));
-  if (pos > P.cp_len - 2) pos = P.cp_len - 2;
-  const double Q = d_interp(inv[pos], qi[pos], inv[pos + 1], qi[pos + 1], cp);
+  const double Q = d_grid_lookup(P.cp_adv_uniform, P.cp_inv, P.cp_qinv + (size_t)g * P.cp_len, P.cp_len, P.cp_inv_rcp, cp);
   return cdf < 0.5 ? -Q : Q;
 }
 
+/* - ENG_EXP64 times the mass path of a photon of the given energy to the
+ * detector from layer L, the records of several crossed layers loaded before
+ * the first is used.  Up to five layers rd holds the layers' factors; beyond
+ * (register budget) the wave's layers lo .. hi are walked four at a time, a
+ * lane taking those on its side of L (up or down) from slot i's record. */
+template <int NL>
+__device__ __forceinline__ double d_mass_path(const EngineParams &P, const VrSoA &V, double energy, int L, int up, int lo,
+                                              int hi, int i, const double *rd, const ScatterTab &tab) {
+  const xrl_ectx ce = d_energy_tab(energy, tab);
+  if (!(energy > 0.0)) return 0.0;
+  const LayCell *cell = P.lay_cell + (size_t)ce.ci * P.n_layers;
+  double t = 0.0;
+  if constexpr (NL <= 5) {
+    LayCell r[NL];
+#pragma unroll
+    for (int l = 0; l < NL; l++)
+      if (rd[l] < 0.0) r[l] = cell[l];
+#pragma unroll
+    for (int l = 0; l < NL; l++)
+      if (rd[l] < 0.0) t = fma(d_cell_mu(P, l, r[l], ce), rd[l], t);
+  } else {
+    for (int l0 = lo; l0 <= hi; l0 += 4) {
+      LayCell r[4];
+      double d[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int l = l0 + k;
+        if (l <= hi && (up ? l >= L - 1 : l <= L - 1)) {
+          r[k] = cell[l];
+          d[k] = V.dist[(size_t)l * P.cap + i];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int l = l0 + k;
+        if (l <= hi && (up ? l >= L - 1 : l <= L - 1)) t = fma(d_cell_mu(P, l, r[k], ce) * P.layer_density[l], d[k], t);
+      }
+    }
+    t *= -ENG_EXP64;
+  }
+  return t;
+}
+
+/* Bound by vector issue (50 % of the cycles) and the address unit's work on
+ * per-lane table reads (66 %): per photon and element one profile CDF, one
+ * inverse CDF and one record per crossed layer.  Hence uniform grids are not
+ * read, an energy's layer records lie side by side and are loaded together,
+ * and logarithm, power, exponential and quotients are the short forms above.
+ * 1e8 histories of the three-layer tube run: 43.6 -> 33.0 ms; the advanced
+ * model on 3e5 photons in seven layers 559 -> 449 us an order (38 % issue;
+ * bound by the last round of its 4700 chunks on 3072 resident waves).
+ * Occupancy: four waves per SIMD (128 VGPRs) measured 2 % faster than three
+ * up to three layers, where few registers spill; three elsewhere. */
 template <int NL, bool use_lds, bool ADV>
-__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(3))) k_vr_scatter(EngineParams P, PhotonSoA S, VrSoA V, int n) {
+__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(!ADV && NL <= 3 ? 4 : 3)))
+k_vr_scatter(EngineParams P, PhotonSoA S, VrSoA V, int n) {
   /* LDS tallies (when they fit): channels [nch][2], Rayleigh/Compton rows
    * [nZ][2][2]; flushed once per workgroup */
   extern __shared__ unsigned long long lds[];
-  __shared__ double exp_tab[64];
+  __shared__ ScatterTab tab;
   const size_t n_ch2 = (size_t)P.nch * 2, n_rc2 = (size_t)P.nZ * 4;
   const size_t cap = (size_t)P.cap;
   unsigned long long *gch = P.t_ch + (size_t)(n - 1) * n_ch2;
   unsigned long long *grc = P.t_rc + (size_t)(n - 1) * n_rc2;
   unsigned long long *tch = gch, *trc = grc;
-  if (threadIdx.x < 64) exp_tab[threadIdx.x] = exp2((double)threadIdx.x / 64.0);
+  d_scatter_tab(&tab);
   if (use_lds) {
     tch = lds;
     trc = lds + n_ch2;
@@ -1385,8 +1497,7 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
   const int shift = P.tally_shift;
   const int lane = __lane_id();
   const double inv_gain = 1.0 / P.gain;
-  /* the Compton profile's random-number grid is uniform */
-  const double inv_drn = 1.0 / (P.cp_rn[1] - P.cp_rn[0]);
+  const double r_end = d_const(P.cp_rn)[P.cp_len - 2];
   /* single-precision literals of src/xmi_variance_reduction.F90:949-1008 */
   const double cc = (double)1.2399e-6f, c0 = (double)4.85e-12f, c1 = (double)1.456e-2f;
   /* wave index through readfirstlane: wave-uniform for the compiler too,
@@ -1403,13 +1514,14 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
     /* per-photon factors, shared by every element of the layer */
     double E = 0.0, wo = 0.0, pesc = 0.0, inv_mu = 0.0, c_lamb0 = 1.0, A0 = 0.0, A1 = 0.0, ct_e = 0.0;
     phx_stream sd; /* advanced model: uniforms from the same stream position */
-    /* rho * path by layer (0 where not crossed): in registers for up to five
-     * layers, read from the records beyond (register budget) */
+    /* - rho * path * ENG_EXP64 by layer (0 where not crossed): in registers for
+     * up to five layers, read from the records beyond (register budget) */
     constexpr int NR = NL <= 5 ? NL : 1;
     double rd[NR];
     xrl_dcsp_ctx dc = {0.0, 0.0, 0.0};
-    int dir = 1, nc = 0, ch_r = -1;
-    WaveWords s = {};
+    int ch_r = -1;
+    uint32_t ww[4] = {0u, 0u, 0u, 0u}; /* the current block's words */
+    uint32_t ctr0 = 0u, hid_lo = 0u, hid_hi = 0u;
 #pragma unroll
     for (int k = 0; k < NR; k++) rd[k] = 0.0;
     if (mine) {
@@ -1417,43 +1529,36 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
       const double ct = V.ct[i], q = V.q[i], mct = 1.0 - ct;
       wo = V.omega[i] * S.weight[i];
       pesc = V.pesc[i];
-      inv_mu = 1.0 / S.mus[(size_t)(L - 1) * cap + i];
-      dir = (info & VR_UP) ? 1 : -1;
-      nc = info >> VR_NC_SHIFT;
+      inv_mu = d_rcp(S.mus[(size_t)(L - 1) * cap + i]);
       if (NL <= 5) {
 #pragma unroll
         for (int l = 0; l < NR; l++)
-          if (l < P.n_layers) rd[l] = P.layer_density[l] * V.dist[(size_t)l * cap + i];
+          if (l < P.n_layers) rd[l] = (-ENG_EXP64 * P.layer_density[l]) * V.dist[(size_t)l * cap + i];
       }
       /* the estimator stream from the block after the geometry and cone
-       * draws, as words */
+       * draws, as words: element k takes word k */
+      ctr0 = V.blk[i];
       {
-        phx_stream s0;
-        phx_stream_init(&s0, P.seed, P.sample, (uint32_t)n, PHX_SUB_VARRED, S.hid[i]);
-        s.key[0] = s0.key[0];
-        s.key[1] = s0.key[1];
-        s.ctr[0] = V.blk[i];
-        s.ctr[1] = s0.ctr[1];
-        s.ctr[2] = s0.ctr[2];
-        s.ctr[3] = s0.ctr[3];
-        s.na = 0;
-        s.hasb = 0;
-        if (ADV) {
-          sd = s0;
-          sd.ctr[0] = V.blk[i];
-        }
+        const unsigned long long hid = S.hid[i];
+        hid_lo = (uint32_t)hid;
+        hid_hi = (uint32_t)(hid >> 32);
+      }
+      if (ADV) {
+        phx_stream_init(&sd, P.seed, P.sample, (uint32_t)n, PHX_SUB_VARRED, S.hid[i]);
+        sd.ctr[0] = ctr0;
       }
       ct_e = ct;
       /* xrl_dcsp_setup from cos theta and sin^2 theta cos^2 phi */
-      const double sth2 = sqrt(0.5 * mct), kk = 1.0 / (1.0 + E / XRL_MEC2 * mct);
-      dc.x = E / XRL_KEV_ANGSTROM * sth2;
+      const double sth2 = mct > 0.0 ? d_sqrt_pos(0.5 * mct) : 0.0, k1 = 1.0 + E * (1.0 / XRL_MEC2) * mct, kk = d_rcp(k1);
+      dc.x = E * (1.0 / XRL_KEV_ANGSTROM) * sth2;
       dc.thomson = XRL_RE2 * (1.0 - q);
-      dc.kn = XRL_RE2 * 0.5 * kk * kk * (kk + 1.0 / kk - 2.0 * q);
-      c_lamb0 = cc / (E * 1000.0);
+      dc.kn = XRL_RE2 * 0.5 * kk * kk * (kk + k1 - 2.0 * q);
+      c_lamb0 = cc * d_rcp(E * 1000.0);
       A0 = c0 * sth2 * sth2;
       A1 = c1 * c_lamb0 * sth2;
       ch_r = E >= 1.0 ? (int)((E - P.zero) * inv_gain) : -1;
     }
+    const int lo = __ballot(mine && !(info & VR_UP)) ? 0 : L - 1, hi = __ballot(mine && (info & VR_UP)) ? P.n_layers - 1 : L - 1;
     const int off = __builtin_amdgcn_readfirstlane(P.layer_off[L - 1]);
     const int nel = __builtin_amdgcn_readfirstlane(P.layer_nel[L - 1]);
     double twr_sum = 0.0; /* Rayleigh keeps the energy: one channel per photon */
@@ -1461,32 +1566,41 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
     /* the accepted momenta's bounds of the Doppler draw (per photon), and
      * the profile-CDF values at them of the next element, loaded one
      * element ahead */
-    const double pz_max = A1 > 0.0 ? A0 / A1 : 0.0, pz_neg = A1 > 0.0 ? (c_lamb0 + A0) / A1 : 0.0;
-    double cdf_max[2] = {0.0, 0.0}, cdf_neg[2] = {0.0, 0.0};
+    const double iA1 = A1 > 0.0 ? d_rcp(A1) : 0.0, pz_max = A0 * iA1, pz_neg = (c_lamb0 + A0) * iA1;
+    CdfPair cdf_max = {0.0, 0.0, 0.0}, cdf_neg = {0.0, 0.0, 0.0};
     if (!ADV && mine && A1 > 0.0 && nel > 0) {
       const int u0 = d_const(P.el_u)[off];
-      d_profile_cdf_load(P.cp_cdfg + (size_t)u0 * XMI_CP_GRID, P.cp_gscale[u0], pz_max, cdf_max);
-      d_profile_cdf_load(P.cp_cdfg + (size_t)u0 * XMI_CP_GRID, P.cp_gscale[u0], pz_neg, cdf_neg);
+      const double *gr = P.cp_cdfg + (size_t)u0 * XMI_CP_GRID;
+      const double gs = d_const(P.cp_gscale)[u0];
+      d_profile_cdf_load(gr, gs, pz_max, &cdf_max);
+      d_profile_cdf_load(gr, gs, pz_neg, &cdf_neg);
     }
     for (int k = 0; k < nel; k++) {
       const int u = d_const(P.el_u)[off + k];
-      const xrl_atom *a = &P.atoms[u];
+      const auto *a = d_const(P.atoms) + u;
       const double Pconv = d_const(P.el_w)[off + k] * inv_mu;
       double f_max = 0.0, f_neg = 0.0;
       if (!ADV && mine && A1 > 0.0) {
-        const double gs = P.cp_gscale[u];
-        f_max = d_profile_cdf_eval(cdf_max, gs, pz_max);
-        f_neg = d_profile_cdf_eval(cdf_neg, gs, pz_neg);
+        f_max = d_profile_cdf_eval(cdf_max);
+        f_neg = d_profile_cdf_eval(cdf_neg);
         if (k + 1 < nel) {
           const int u1 = d_const(P.el_u)[off + k + 1];
-          d_profile_cdf_load(P.cp_cdfg + (size_t)u1 * XMI_CP_GRID, P.cp_gscale[u1], pz_max, cdf_max);
-          d_profile_cdf_load(P.cp_cdfg + (size_t)u1 * XMI_CP_GRID, P.cp_gscale[u1], pz_neg, cdf_neg);
+          const double *gr = P.cp_cdfg + (size_t)u1 * XMI_CP_GRID;
+          const double gs = d_const(P.cp_gscale)[u1];
+          d_profile_cdf_load(gr, gs, pz_max, &cdf_max);
+          d_profile_cdf_load(gr, gs, pz_neg, &cdf_neg);
         }
       }
-      /* Rayleigh */
-      double twr = 0.0;
+      /* Rayleigh, and the element's factor of its Compton terms
+       * (xrl_dcsp_rayl_c and xrl_dcsp_compt_c: 1 / d1^4 and 1 - 1 / d2^2 =
+       * v (2 + v) / d2^2 from one reciprocal) */
+      double twr = 0.0, dcw = 0.0;
       if (mine) {
-        twr = Pconv * (xrl_dcsp_rayl_c(a, &dc) * wo) * pesc;
+        const double u1 = dc.x * a->inv_ff_x0, u2 = dc.x * a->inv_sf_x0, v = u2 * u2;
+        const double d1 = fma(3.0 * u1, u1, 1.0), d2 = 1.0 + v, d12 = d1 * d1, d14 = d12 * d12, d22 = d2 * d2;
+        const double t = d_rcp(d14 * d22), Z = (double)a->Z, pw = Pconv * wo * a->barn_per_A;
+        twr = (pw * dc.thomson) * (Z * Z) * (t * d22) * pesc;
+        dcw = (pw * dc.kn) * Z * (v * (2.0 + v)) * (t * d14);
         twr_sum += twr;
       }
       /* Compton, xmi_compton_varred2: Doppler-broadened energy from the
@@ -1495,30 +1609,21 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
       if (ADV && mine) {
         /* every occupied subshell with weight count * CDF(Qimax) / sum, one
          * uniform each (xmi_compton_varred) */
-        const int g0 = P.cp_sh_off[u], g1 = P.cp_sh_off[u + 1];
+        const int g0 = d_const(P.cp_sh_off)[u], g1 = d_const(P.cp_sh_off)[u + 1];
         double csum = 0.0;
-        for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct_e);
-        const double dcw = Pconv * (xrl_dcsp_compt_c(a, &dc) * wo);
+        for (int g = g0; g < g1; g++) {
+          const int sh = d_const(P.cp_sh_idx)[g];
+          csum += a->occupancy[sh] * d_adv_cdf(P, a->edge[sh], g, E, ct_e);
+        }
+        const double icsum = csum != 0.0 ? d_rcp(csum) : 0.0;
         for (int g = g0; csum != 0.0 && g < g1; g++) {
-          const double cdf = d_adv_cdf(P, a, g, E, ct_e);
-          const double sw = a->occupancy[P.cp_sh_idx[g]] * cdf / csum;
+          const int sh = d_const(P.cp_sh_idx)[g];
+          const double cdf = d_adv_cdf(P, a->edge[sh], g, E, ct_e);
+          const double sw = a->occupancy[sh] * cdf * icsum;
           if (sw == 0.0) continue;
           const double energy = d_energy_from_q(E, d_adv_q(P, g, phx_uniform(&sd) * cdf), ct_e);
           if (!(energy > 0.0)) continue;
-          const xrl_ectx ce = xrl_energy(energy);
-          double m2 = 0.0;
-          if (NL <= 5) {
-#pragma unroll
-            for (int l = 0; l < NR; l++)
-              if (rd[l] > 0.0) m2 += d_layer_mu_tab(P, l, &ce) * rd[l];
-          } else {
-#pragma unroll 1
-            for (int kk = 0; kk < nc; kk++) {
-              const int l0 = L - 1 + kk * dir;
-              m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)l0 * cap + i]);
-            }
-          }
-          const double tw = dcw * d_exp_neg(-m2, exp_tab) * sw;
+          const double tw = dcw * d_exp64(d_mass_path<NL>(P, V, energy, L, info & VR_UP, lo, hi, i, rd, tab), tab) * sw;
           twc += tw;
           const int ch = energy >= 1.0 ? (int)((energy - P.zero) * inv_gain) : -1;
           if (ch >= 0 && ch <= P.nch - 1 && tw > 0.0) fx_add_global(&tch[2 * ch], tw, shift);
@@ -1532,12 +1637,19 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
          * each (the same distribution, and no wavefront waits on its lanes'
          * longest rejection run); r ranges over [0, r_end), the inverse
          * table without its last interval */
-        const double *rn = P.cp_rn;
         const double *icdf = P.cp_icdf + (size_t)u * P.cp_len;
-        const double r_end = rn[P.cp_len - 2];
         if (!(A1 > 0.0)) f_max = f_neg = r_end; /* the profile CDFs at A0 / A1 were loaded ahead */
         const double m_pos = f_max + (r_end - f_neg);
-        const uint32_t wd = d_ww_word(s);
+        if ((k & 3) == 0) {
+          uint32_t c4[4] = {ctr0 + (uint32_t)(k >> 2), (P.sample << 12) | (((uint32_t)n & 0xFFu) << 4) | PHX_SUB_VARRED, hid_lo,
+                            hid_hi};
+          const uint32_t key[2] = {(uint32_t)P.seed, (uint32_t)(P.seed >> 32)};
+          phx_4x32_10(c4, key, ww);
+        }
+        const uint32_t wd = ww[0];
+        ww[0] = ww[1];
+        ww[1] = ww[2];
+        ww[2] = ww[3];
         const double uu = (double)wd * 0x1.0p-32 * (r_end + m_pos);
         double r, sgn;
         if (uu < r_end) {
@@ -1548,31 +1660,15 @@ __global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(
           r = v < f_max ? v : v - f_max + f_neg;
           sgn = 1.0;
         }
-        int pos = (int)(r * inv_drn);
-        if (pos > P.cp_len - 3) pos = P.cp_len - 3;
-        const double pz = sgn * (icdf[pos] + (icdf[pos + 1] - icdf[pos]) * ((r - rn[pos]) * inv_drn));
-        const double energy = (cc / 1000.0) / (c_lamb0 + (A0 - A1 * pz));
-        {
-          const xrl_ectx ce = xrl_energy(energy);
-          double m2 = 0.0;
-          if (NL <= 5) {
-#pragma unroll
-            for (int l = 0; l < NR; l++)
-              if (rd[l] > 0.0) m2 += d_layer_mu_tab(P, l, &ce) * rd[l];
-          } else {
-#pragma unroll 1
-            for (int kk = 0; kk < nc; kk++) {
-              const int l0 = L - 1 + kk * dir;
-              m2 += d_layer_mu_tab(P, l0, &ce) * (P.layer_density[l0] * V.dist[(size_t)l0 * cap + i]);
-            }
-          }
-          twc = Pconv * (xrl_dcsp_compt_c(a, &dc) * wo) * d_exp_neg(-m2, exp_tab);
-          const int ch = energy >= 1.0 ? (int)((energy - P.zero) * inv_gain) : -1;
-          if (ch >= 0 && ch <= P.nch - 1 && twc > 0.0) fx_add_global(&tch[2 * ch], twc, shift);
-        }
+        const double pz = sgn * d_grid_lookup(P.cp_rn_uniform, P.cp_rn, icdf, P.cp_len - 1, P.cp_rn_inv, r);
+        const double energy = (cc / 1000.0) * d_rcp(c_lamb0 + (A0 - A1 * pz));
+        twc = dcw * d_exp64(d_mass_path<NL>(P, V, energy, L, info & VR_UP, lo, hi, i, rd, tab), tab);
+        const int ch = energy >= 1.0 ? (int)((energy - P.zero) * inv_gain) : -1;
+        if (ch >= 0 && ch <= P.nch - 1 && twc > 0.0) fx_add_global(&tch[2 * ch], twc, shift);
       }
       /* history rows: wave totals collected in lanes, 32 elements a group */
-      const double tr = d_wave_total(twr), tc = d_wave_total(twc);
+      double tr, tc;
+      d_wave_total2(twr, twc, &tr, &tc);
       const int j = k & 31;
       if (lane == 2 * j) rsum = tr;
       if (lane == 2 * j + 1) rsum = tc;
@@ -1872,7 +1968,8 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
     const xrl_atom *a = &P.atoms[u];
     const int g0 = P.cp_sh_off[u], g1 = P.cp_sh_off[u + 1];
     double csum = 0.0;
-    for (int g = g0; g < g1; g++) csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct);
+    for (int g = g0; g < g1; g++)
+      csum += a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a->edge[P.cp_sh_idx[g]], g, E, ct);
     if (csum == 0.0) {
       S.energy[i] = 0.0;
       return;
@@ -1881,7 +1978,7 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
     double ts = 0.0, cdf_sel = 0.0;
     int sel = -1, last = g0;
     for (int g = g0; g < g1; g++) {
-      const double w = a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a, g, E, ct);
+      const double w = a->occupancy[P.cp_sh_idx[g]] * d_adv_cdf(P, a->edge[P.cp_sh_idx[g]], g, E, ct);
       if (w > 0.0) last = g;
       ts += w / csum;
       if (r <= ts) {
@@ -1890,7 +1987,7 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
       }
     }
     if (sel < 0) sel = last; /* rounding left the running sum just below r */
-    cdf_sel = d_adv_cdf(P, a, sel, E, ct);
+    cdf_sel = d_adv_cdf(P, a->edge[P.cp_sh_idx[sel]], sel, E, ct);
     const double e = d_energy_from_q(E, d_adv_q(P, sel, phx_uniform(&s) * cdf_sel), ct);
     if (!(e > 0.0)) {
       S.energy[i] = 0.0;
@@ -1904,17 +2001,14 @@ __device__ __forceinline__ void d_compton_one(const EngineParams &P, const Photo
   const double cc = (double)1.2399e-6f, c0 = (double)4.85e-12f, c1 = (double)1.456e-2f;
   double energy = E * 1000.0;
   double c_lamb0 = cc / energy;
-  const double *rn = P.cp_rn;
   const double *icdf = P.cp_icdf + (size_t)u * P.cp_len;
-  const double drn = rn[1] - rn[0], inv_drn = 1.0 / drn;
   /* the reference loops until acceptance; every draw with pz <= 0 is accepted,
    * so the bound below is never reached by valid data and only turns a
    * corrupted table into a counted error instead of a hung wave */
   int accepted = 0;
   for (int it = 0; it < 4096; it++) {
     double r = phx_uniform(&s);
-    int pos = (int)(r / drn);
-    double pz = fma((icdf[pos + 1] - icdf[pos]) * inv_drn, r - rn[pos], icdf[pos]);
+    double pz = d_grid_lookup(P.cp_rn_uniform, P.cp_rn, icdf, P.cp_len, P.cp_rn_inv, r);
     if (phx_uniform(&s) < 0.5) pz = -pz;
     double dlamb = c0 * sth2 * sth2 - c1 * c_lamb0 * sth2 * pz;
     energy = cc / (c_lamb0 + dlamb) / 1000.0;
@@ -2320,10 +2414,11 @@ __device__ __forceinline__ int d_interact_entry(const EngineParams &P, const Pho
  * photons that interact at this order, and a wavefront straddles two queues
  * at two places at most.  Each photon is one thread's, with its own random
  * stream, so results do not depend on the assignment. */
-/* 72 VGPRs leave seven waves per SIMD.  ADV: the advanced Compton model,
- * compiled apart */
+/* bound by the latency of its gathers (78 % of the wave cycles wait, 31 % of
+ * the vector issue): eight waves per SIMD, 63 VGPRs without spills, measured
+ * 2 % faster than seven.  ADV: the advanced Compton model, compiled apart */
 template <bool ADV>
-__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
 k_interact(EngineParams P, PhotonSoA S, int n) {
   __shared__ unsigned int off[3 * ENG_SPREAD + 1];
   d_queue_offsets(P.qcount, off);
