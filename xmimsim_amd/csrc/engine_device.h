@@ -104,17 +104,14 @@ struct EngineParams {
   double layer_ze[ENG_MAX_LAYERS];
   int layer_nel[ENG_MAX_LAYERS];
   int layer_off[ENG_MAX_LAYERS];
-  const int *el_Z;              /* flattened per layer */
-  const double *el_w;
+  const double *el_w;           /* flattened per layer */
   const int *el_u;              /* hdf5 index */
   /* attenuation of each layer as one lookup: mu_l(E) = E^-p * pb[K] + rc(E),
    * K = number of the layer's edges above E (edges sorted descending), rc the
    * weighted sum of the elements' Rayleigh+Compton tables on the shared ln E
-   * grid; kstart[ci] = edges certainly above any E of ln E cell ci */
-  const double *lay_rc;         /* [n_layers][XRL_NCS] */
+   * grid, all in the records of lay_cell */
   const double *lay_edge;       /* [lay_eoff[l] .. lay_eoff[l+1]) */
   const double *lay_pb;         /* [lay_eoff[l] + l .. lay_eoff[l+1] + l] */
-  const int *lay_kstart;        /* [n_layers][XRL_NCS] */
   const struct LayCell *lay_cell; /* [XRL_NCS][n_layers]: an energy's layers side by side */
   const struct LayCell *el_cell;  /* [XRL_NCS][n_lay_el], elements of the layers in layer_off order: each element's
                                      own total cross section (K counts its own edges) */
@@ -147,7 +144,7 @@ struct EngineParams {
    * subshells of element u are g = cp_sh_off[u] .. cp_sh_off[u+1]-1, with
    * the provider subshell cp_sh_idx[g], the partial-profile CDF
    * cp_pcdf[g][cp_len] on the Q grid cp_Qs and its inverse cp_qinv[g][cp_len]
-   * on the CDF grid cp_inv (both grids uniform and shared) */
+   * on the CDF grid cp_inv (both grids shared) */
   int adv_compton;
   const int *cp_sh_off, *cp_sh_idx;
   const double *cp_pcdf, *cp_qinv, *cp_Qs, *cp_inv;
@@ -157,15 +154,7 @@ struct EngineParams {
   const double *line_E;         /* [nZ][219] */
   const double *rate_cum;       /* [nZ][220] radiative rates summed along each shell's lines, index |line| */
   const double *precalc_mu;     /* [n_layers][nZ][219] */
-  /* detection tables */
-  const int *act_n;             /* [nZ] */
-  const int *act_line;          /* [nZ][ENG_MAX_ACT] */
-  const int *act_shell;
-  const double *act_factor;     /* fluor_yield(shell) * rad_rate(line) */
-  const double *act_E;
-  const int *act_ch;
-  const double *act_murho;      /* [n_layers][nZ][ENG_MAX_ACT] */
-  /* the same lines flattened per layer: entry t of layer l (fl_off[l] <= t <
+  /* the estimator's active lines flattened per layer: entry t of layer l (fl_off[l] <= t <
    * fl_off[l+1]) is active line q of element u of that layer */
   int fl_off[ENG_MAX_LAYERS + 1];
   const int4 *fl_info;          /* {u, q, shell, compact bin} */

@@ -191,37 +191,34 @@ static hipError_t copy_d2h(void *dst, const void *src, size_t bytes, hipStream_t
   return e;
 }
 
-/* many uploads through one staging fill: every array copied into its own
- * 256-byte aligned part of the staging memory, one asynchronous copy each,
- * and one synchronisation at the end */
+/* one run's tables: arrays at 256-byte aligned offsets of one device
+ * allocation, filled by a single copy (28 copies cost about 10 us each, a
+ * third of a small run).  Asynchronous: the staging memory is the caller's
+ * own and is not refilled before the stream has passed the copy. */
 struct UploadSet {
   struct Item {
-    DevBuf *b;
+    void **dst;
     const void *src;
     size_t bytes;
   };
   std::vector<Item> items;
   template <typename T>
-  void add(DevBuf &b, const T *src, size_t count) {
-    items.push_back({&b, src, sizeof(T) * count});
+  void add(const T **dst, const std::vector<T> &src) {
+    items.push_back({(void **)dst, src.data(), sizeof(T) * src.size()});
   }
-  hipError_t run(hipStream_t st, Staging &sg) {
+  hipError_t run(DevBuf &arena, hipStream_t st, Staging &sg) {
     size_t total = 0;
     for (const Item &it : items) total += (it.bytes + 255) & ~(size_t)255;
     hipError_t e = sg.ensure(total);
+    if (e == hipSuccess) e = arena.ensure(total);
+    if (e != hipSuccess) return e;
     size_t off = 0;
     for (const Item &it : items) {
-      if (e == hipSuccess) e = it.b->ensure(it.bytes);
-      if (e != hipSuccess) break;
-      if (it.bytes) {
-        memcpy((char *)sg.p + off, it.src, it.bytes);
-        e = hipMemcpyAsync(it.b->p, (char *)sg.p + off, it.bytes, hipMemcpyHostToDevice, st);
-        off += (it.bytes + 255) & ~(size_t)255;
-      }
+      if (it.bytes) memcpy((char *)sg.p + off, it.src, it.bytes);
+      *it.dst = arena.as<char>() + off;
+      off += (it.bytes + 255) & ~(size_t)255;
     }
-    /* the staging memory is reused after this */
-    hipError_t e2 = hipStreamSynchronize(st);
-    return e != hipSuccess ? e : e2;
+    return total ? hipMemcpyAsync(arena.p, sg.p, total, hipMemcpyHostToDevice, st) : hipSuccess;
   }
 };
 
@@ -274,11 +271,9 @@ struct Engine {
   DevBuf sa_grid, sa_r, sa_t;
   int sa_nr = 0, sa_nt = 0;
   /* per-call buffers (grow only) */
-  DevBuf el_Z, el_w, el_u, precalc_mu, act_n, act_line, act_shell, act_factor, act_E, act_ch, act_murho;
-  DevBuf fl_info, fl_wf, fl_ent, lbin_g;
-  DevBuf lay_rc, lay_edge, lay_pb, lay_kstart, lay_cell, el_cell;
-  DevBuf src_desc, src_run0, src_line_mus, exc_layers, exc_atoms;
-  DevBuf state, vr, tallies, counters, queue, lay_list, lay_woff, lay_total, lay_segbase, cone_acc, esc_tally;
+  DevBuf tables;     /* one run's tables (UploadSet) */
+  Staging run_stage; /* and their staging memory */
+  DevBuf state, vr, tallies, queue, lay_list, lay_woff, lay_total, lay_segbase, cone_acc, esc_tally;
   DevBuf queue2, qcount2, olist;
   DevBuf batch_queue;
 };
@@ -482,36 +477,85 @@ extern "C" void xmi_engine_forget_tables(const void *h) {
 /* hash of every cell and both axes of a grid: a grid edited in place, or a new
  * grid at a reused address, is uploaded again unless its contents are the same
  * (four independent multiply-xorshift chains over the 64-bit words) */
-static uint64_t grid_hash(const xmi_solid_angle *sa) {
+/* hash of n doubles, copied to out as they are read unless out is NULL */
+static uint64_t hash_doubles(const double *p, size_t n, double *out) {
   uint64_t h[4] = {0x9E3779B97F4A7C15ull, 0xC2B2AE3D27D4EB4Full, 0x165667B19E3779F9ull, 0x27D4EB2F165667C5ull};
-  auto mix = [&](const double *p, size_t n) {
-    size_t i = 0;
-    for (; i + 4 <= n; i += 4)
-      for (int k = 0; k < 4; k++) {
-        uint64_t w;
-        memcpy(&w, p + i + k, 8);
-        h[k] = (h[k] ^ w) * 0xff51afd7ed558ccdull;
-        h[k] ^= h[k] >> 29;
-      }
-    for (; i < n; i++) {
-      uint64_t w;
-      memcpy(&w, p + i, 8);
-      h[0] = (h[0] ^ w) * 0xff51afd7ed558ccdull;
-      h[0] ^= h[0] >> 29;
+  size_t i = 0;
+  for (; i + 4 <= n; i += 4) {
+    uint64_t w[4];
+    memcpy(w, p + i, 32);
+    if (out) memcpy(out + i, w, 32);
+    for (int k = 0; k < 4; k++) {
+      h[k] = (h[k] ^ w[k]) * 0xff51afd7ed558ccdull;
+      h[k] ^= h[k] >> 29;
     }
-  };
-  size_t tot = (size_t)sa->grid_dims_r_n * sa->grid_dims_theta_n;
-  mix(sa->grid_dims_r_vals, (size_t)sa->grid_dims_r_n);
-  mix(sa->grid_dims_theta_vals, (size_t)sa->grid_dims_theta_n);
-  mix(sa->solid_angles, tot);
-  return (h[0] ^ (h[1] * 3) ^ (h[2] * 5) ^ (h[3] * 7)) + tot;
+  }
+  for (; i < n; i++) {
+    uint64_t w;
+    memcpy(&w, p + i, 8);
+    if (out) memcpy(out + i, &w, 8);
+    h[0] = (h[0] ^ w) * 0xff51afd7ed558ccdull;
+    h[0] ^= h[0] >> 29;
+  }
+  return h[0] ^ (h[1] * 3) ^ (h[2] * 5) ^ (h[3] * 7);
 }
 
+/* the hash of a solid-angle grid, over pieces of GRID_PIECE values that up to
+ * GRID_THREADS threads share (the caller's one of them), so that the 8 MB of
+ * a default grid are read at more than one core's bandwidth: 340 us with one
+ * thread.  The pieces' hashes are combined in order, whoever formed them.
+ * out: the grid's copy (NULL: none), written on the way. */
+#define GRID_PIECE ((size_t)65536)
+#define GRID_THREADS 4
+static uint64_t grid_hash(const xmi_solid_angle *sa, double *out) {
+  const size_t tot = (size_t)sa->grid_dims_r_n * sa->grid_dims_theta_n, np = (tot + GRID_PIECE - 1) / GRID_PIECE;
+  std::vector<uint64_t> part(np);
+  std::atomic<size_t> next(0);
+  auto work = [&]() {
+    for (size_t k; (k = next.fetch_add(1)) < np;) {
+      const size_t o = k * GRID_PIECE, n = tot - o < GRID_PIECE ? tot - o : GRID_PIECE;
+      part[k] = hash_doubles(sa->solid_angles + o, n, out ? out + o : nullptr);
+    }
+  };
+  std::thread helper[GRID_THREADS - 1];
+  /* a piece takes about 20 us, a thread's start about as long: helpers from
+   * four pieces on.  Without a helper (no thread to be had) the caller does
+   * their share */
+  for (size_t k = 0; k + 1 < GRID_THREADS && 4 * (k + 1) <= np; k++) {
+    try {
+      helper[k] = std::thread(work);
+    } catch (...) {
+      break;
+    }
+  }
+  work();
+  for (std::thread &t : helper)
+    if (t.joinable()) t.join();
+  uint64_t h = hash_doubles(sa->grid_dims_r_vals, (size_t)sa->grid_dims_r_n, nullptr) * 0x9E3779B97F4A7C15ull;
+  h = (h ^ (h >> 29) ^ hash_doubles(sa->grid_dims_theta_vals, (size_t)sa->grid_dims_theta_n, nullptr)) * 0xff51afd7ed558ccdull;
+  for (size_t k = 0; k < np; k++) h = ((h ^ (h >> 29)) ^ part[k]) * 0xff51afd7ed558ccdull;
+  return h + tot;
+}
+
+/* the grid on the device, uploaded unless the same handle holds the same
+ * values as at the last run.  A new handle's grid is hashed and staged in one
+ * pass. */
 static int ensure_grid(Engine &E, const xmi_solid_angle *sa) {
-  uint64_t hsh = grid_hash(sa);
-  if (E.sa_key == sa && E.sa_hash == hsh) return 1;
-  size_t tot = (size_t)sa->grid_dims_r_n * sa->grid_dims_theta_n;
-  if (upload(E.sa_grid, sa->solid_angles, tot, E.stream, E.stage) != hipSuccess ||
+  const size_t tot = (size_t)sa->grid_dims_r_n * sa->grid_dims_theta_n;
+  uint64_t hsh = 0;
+  const bool same = E.sa_key == sa;
+  if (same && (hsh = grid_hash(sa, nullptr)) == E.sa_hash) return 1;
+  hipError_t e = E.stage.ensure(tot * sizeof(double));
+  if (e == hipSuccess) e = E.sa_grid.ensure(tot * sizeof(double));
+  E.sa_key = nullptr;
+  if (e == hipSuccess) {
+    if (same) memcpy(E.stage.p, sa->solid_angles, tot * sizeof(double));
+    else hsh = grid_hash(sa, (double *)E.stage.p);
+    e = hipMemcpyAsync(E.sa_grid.p, E.stage.p, tot * sizeof(double), hipMemcpyHostToDevice, E.stream);
+    const hipError_t e2 = hipStreamSynchronize(E.stream); /* the staging memory is reused after this */
+    if (e == hipSuccess) e = e2;
+  }
+  if (e != hipSuccess ||
       upload(E.sa_r, sa->grid_dims_r_vals, (size_t)sa->grid_dims_r_n, E.stream, E.stage) != hipSuccess ||
       upload(E.sa_t, sa->grid_dims_theta_vals, (size_t)sa->grid_dims_theta_n, E.stream, E.stage) != hipSuccess) {
     xmi_set_error("solid-angle grid upload failed");
@@ -938,20 +982,18 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
   }
   /* history ids are laid out with the full per-source budget; batches only run
    * the first `count` of each source */
-  std::vector<double> exc_flat;
+  std::vector<double> exc_flat; /* elements by their place in exc_atoms */
+  std::vector<xrl_atom> exc_atoms;
   for (int k = 0; k < in->n_exc_layers; k++) {
     const xmi_layerF *L = &in->exc_layers[k];
     exc_flat.push_back(L->density);
     exc_flat.push_back(L->thickness);
     exc_flat.push_back((double)L->n_elements);
-    for (int j = 0; j < L->n_elements; j++) exc_flat.push_back((double)L->Z[j]);
+    for (int j = 0; j < L->n_elements; j++) {
+      exc_flat.push_back((double)exc_atoms.size());
+      exc_atoms.push_back(*xrl_atom_get(L->Z[j]));
+    }
     for (int j = 0; j < L->n_elements; j++) exc_flat.push_back(L->weight[j]);
-  }
-  std::vector<xrl_atom> exc_atoms;
-  if (in->n_exc_layers > 0) {
-    exc_atoms.resize(XMI_MAXZ + 1);
-    for (int k = 0; k < in->n_exc_layers; k++)
-      for (int j = 0; j < in->exc_layers[k].n_elements; j++) exc_atoms[in->exc_layers[k].Z[j]] = *xrl_atom_get(in->exc_layers[k].Z[j]);
   }
   /* fixed-point scale: the total source intensity maps to 2^100, leaving a
    * factor 2^27 of headroom below 2^127 and a resolution of 2^-100 of it */
@@ -992,7 +1034,9 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     size_t tally_words = n_ch2 + n_line2 + n_rc2 + n_bch2 + n_bh2;
     HIP_TRY(G.state.ensure(state_bytes));
     HIP_TRY(G.vr.ensure(vr_bytes));
-    HIP_TRY(G.tallies.ensure(tally_words * sizeof(unsigned long long)));
+    /* the counters follow the tallies: one clear and one copy back for both */
+    const size_t cnt_words = (size_t)ENG_NCOUNTERS * ENG_SPREAD;
+    HIP_TRY(G.tallies.ensure((tally_words + cnt_words) * sizeof(unsigned long long)));
     int dev = 0, n_cu = 256;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1011,7 +1055,6 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       const long need = ((W + ENG_SPREAD - 1) / ENG_SPREAD) * 64 * trips;
       if (need > P.qreg) P.qreg = (int)need;
     }
-    HIP_TRY(G.counters.ensure((size_t)ENG_NCOUNTERS * ENG_SPREAD * sizeof(unsigned long long)));
     HIP_TRY(G.queue.ensure((size_t)ENG_NQUEUES * ENG_SPREAD * P.qreg * sizeof(int)));
     /* brute force: a second queue set (the interactions of order n - 1 while
      * order n's step fills the first), and two offspring lists */
@@ -1040,42 +1083,29 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       HIP_TRY(G.cone_acc.ensure(cone_bytes));
       if (fresh) HIP_TRY(hipMemsetAsync(G.cone_acc.p, 0, cone_bytes, st));
     }
+    SourceTable ST;
     {
       UploadSet up;
-      up.add(G.el_Z, elZ.data(), elZ.size());
-      up.add(G.el_w, elW.data(), elW.size());
-      up.add(G.el_u, elU.data(), elU.size());
-      up.add(G.precalc_mu, pmu.data(), pmu.size());
-      up.add(G.act_n, actn.data(), actn.size());
-      up.add(G.act_line, actl.data(), actl.size());
-      up.add(G.act_shell, acts.data(), acts.size());
-      up.add(G.act_factor, actf.data(), actf.size());
-      up.add(G.act_E, actE.data(), actE.size());
-      up.add(G.act_ch, actc.data(), actc.size());
-      up.add(G.act_murho, actm.data(), actm.size());
-      up.add(G.fl_info, fl_info.data(), fl_info.size());
-      up.add(G.fl_wf, fl_wf.data(), fl_wf.size());
-      up.add(G.fl_ent, fl_ent.data(), fl_ent.size());
-      up.add(G.lbin_g, lbin_g.data(), lbin_g.size());
-      up.add(G.lay_rc, lay_rc.data(), lay_rc.size());
-      up.add(G.lay_edge, lay_edge.data(), lay_edge.size());
-      up.add(G.lay_pb, lay_pb.data(), lay_pb.size());
-      up.add(G.lay_kstart, lay_kstart.data(), lay_kstart.size());
-      up.add(G.lay_cell, lay_cell.data(), lay_cell.size());
-      up.add(G.el_cell, el_cell.data(), el_cell.size());
-      up.add(G.src_desc, src.data(), src.size());
-      up.add(G.src_run0, run0.data(), run0.size());
-      up.add(G.src_line_mus, src_mus.data(), src_mus.size());
-      up.add(G.exc_layers, exc_flat.data(), exc_flat.size());
-      up.add(G.exc_atoms, exc_atoms.data(), exc_atoms.size());
-      HIP_TRY(up.run(st, G.stage));
+      up.add(&P.el_w, elW);
+      up.add(&P.el_u, elU);
+      up.add(&P.precalc_mu, pmu);
+      up.add(&P.fl_info, fl_info);
+      up.add(&P.fl_wf, fl_wf);
+      up.add(&P.fl_ent, fl_ent);
+      up.add(&P.lbin_g, lbin_g);
+      up.add(&P.lay_edge, lay_edge);
+      up.add(&P.lay_pb, lay_pb);
+      up.add(&P.lay_cell, lay_cell);
+      up.add(&P.el_cell, el_cell);
+      up.add(&ST.d, src);
+      up.add(&ST.run0, run0);
+      up.add(&ST.line_mus, src_mus);
+      up.add(&ST.exc_layers, exc_flat);
+      up.add(&ST.exc_atoms, exc_atoms);
+      HIP_TRY(up.run(G.tables, st, G.run_stage));
     }
-    HIP_TRY(hipMemsetAsync(G.tallies.p, 0, tally_words * sizeof(unsigned long long), st));
-    HIP_TRY(hipMemsetAsync(G.counters.p, 0, (size_t)ENG_NCOUNTERS * ENG_SPREAD * sizeof(unsigned long long), st));
+    HIP_TRY(hipMemsetAsync(G.tallies.p, 0, (tally_words + cnt_words) * sizeof(unsigned long long), st));
 
-    P.el_Z = G.el_Z.as<int>();
-    P.el_w = G.el_w.as<double>();
-    P.el_u = G.el_u.as<int>();
     P.atoms = T->atoms.as<xrl_atom>();
     P.ray_icdf = T->ray.as<double>();
     P.comp_icdf = T->comp.as<double>();
@@ -1118,24 +1148,6 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.line_E = T->lineE.as<double>();
     P.rate_cum = T->rate_cum.as<double>();
     P.tab_uniform = T->tab_uniform;
-    P.precalc_mu = G.precalc_mu.as<double>();
-    P.act_n = G.act_n.as<int>();
-    P.act_line = G.act_line.as<int>();
-    P.act_shell = G.act_shell.as<int>();
-    P.act_factor = G.act_factor.as<double>();
-    P.act_E = G.act_E.as<double>();
-    P.act_ch = G.act_ch.as<int>();
-    P.act_murho = G.act_murho.as<double>();
-    P.fl_info = G.fl_info.as<int4>();
-    P.fl_wf = G.fl_wf.as<double>();
-    P.fl_ent = G.fl_ent.as<double>();
-    P.lbin_g = G.lbin_g.as<int>();
-    P.lay_rc = G.lay_rc.as<double>();
-    P.lay_edge = G.lay_edge.as<double>();
-    P.lay_pb = G.lay_pb.as<double>();
-    P.lay_kstart = G.lay_kstart.as<int>();
-    P.lay_cell = G.lay_cell.as<LayCell>();
-    P.el_cell = G.el_cell.as<LayCell>();
     P.n_lay_el = (int)elZ.size();
     P.phi_icdf = T->phi.as<double>();
     P.phi_T = T->phiT.as<double>();
@@ -1183,7 +1195,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.t_rc = tw + n_ch2 + n_line2;
     P.t_bch = brute ? tw + n_ch2 + n_line2 + n_rc2 : nullptr;
     P.t_bhist = brute ? P.t_bch + n_bch2 : nullptr;
-    P.counters = G.counters.as<unsigned long long>();
+    P.counters = tw + tally_words;
     P.queue = G.queue.as<int>();
     P.qcount = P.counters;
     P.pqueue = nullptr;
@@ -1232,14 +1244,8 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     vp += per * sizeof(int);
     V.blk = (unsigned int *)vp;
 
-    SourceTable ST;
-    ST.d = G.src_desc.as<SourceDesc>();
-    ST.run0 = G.src_run0.as<uint64_t>();
     ST.n = (int)src.size();
-    ST.line_mus = G.src_line_mus.as<double>();
-    ST.exc_layers = G.exc_layers.as<double>();
     ST.n_exc = in->n_exc_layers;
-    ST.exc_atoms = G.exc_atoms.as<xrl_atom>();
 
 
     HIP_TRY(hipEventCreate(&evs[0]));
@@ -1256,7 +1262,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
        * batch's primaries, or the capacity in a captured graph, whose
        * source kernel marks the slots beyond the batch empty) */
       int *qs[2] = {G.queue.as<int>(), G.queue2.as<int>()};
-      unsigned long long *qc[2] = {G.counters.as<unsigned long long>(), G.qcount2.as<unsigned long long>()};
+      unsigned long long *qc[2] = {P.counters, G.qcount2.as<unsigned long long>()};
       unsigned int *oc = brute ? (unsigned int *)(qc[1] + ENG_NQUEUES * ENG_SPREAD) : nullptr;
       int *ol[2] = {G.olist.as<int>(), brute ? G.olist.as<int>() + (P.off_half ? P.off_half : 1) : nullptr};
       auto orders = [&](int count) -> hipError_t {
@@ -1349,11 +1355,10 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
       }
     }
     HIP_TRY(hipEventRecord(evs[1], st));
-    std::vector<unsigned long long> th(tally_words);
-    std::vector<unsigned long long> cnt_sub((size_t)ENG_NCOUNTERS * ENG_SPREAD);
+    std::vector<unsigned long long> th(tally_words + cnt_words);
     unsigned long long cnt[ENG_NCOUNTERS];
-    HIP_TRY(copy_d2h(th.data(), G.tallies.p, tally_words * sizeof(unsigned long long), st, G.stage));
-    HIP_TRY(copy_d2h(cnt_sub.data(), G.counters.p, cnt_sub.size() * sizeof(unsigned long long), st, G.stage));
+    HIP_TRY(copy_d2h(th.data(), G.tallies.p, th.size() * sizeof(unsigned long long), st, G.stage));
+    const unsigned long long *cnt_sub = th.data() + tally_words;
     for (int c = 0; c < ENG_NCOUNTERS; c++) {
       cnt[c] = 0ull;
       for (int j = 0; j < ENG_SPREAD; j++) cnt[c] += cnt_sub[(size_t)c * ENG_SPREAD + j];
@@ -1471,8 +1476,10 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     ok = 1;
   }
 fail:
+  /* copies from the staging memory, kernels and replays may still run when a
+   * later step failed */
+  if (!ok) (void)hipStreamSynchronize(E.stream);
   if (graph_exec || graph) {
-    /* replays may still run when a later step failed */
     (void)hipStreamSynchronize(E.stream);
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -1815,7 +1822,7 @@ extern "C" int xmi_solid_angle_calculation_cl(xmi_inputFPtr inputFPtr, xmi_solid
   }
   /* the device copy is the grid just returned: remember it */
   g_engine.sa_key = sa;
-  g_engine.sa_hash = grid_hash(sa);
+  g_engine.sa_hash = grid_hash(sa, nullptr);
   g_engine.sa_nr = (int)n;
   g_engine.sa_nt = (int)n;
   *out = sa;
