@@ -133,3 +133,37 @@ def test_resident_training_equals_step_by_step():
         b.train_resident(np.full((1, B), n, np.int32), lr[:1])
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("nets,dims,B", [
+    (1, (7, 64, 64), 64),             # one tile, one part of the contraction
+    (3, (70, 192, 320, 64), 192),     # widths and rows that 128 does not divide: 64 x 64 tiles, three-step parts
+    (2, (85, 128, 64, 128), 320),
+    (16, (130, 256, 256, 64), 2048),  # 128 x 128 tiles, grouped by XCD, in exactly two workgroups a compute unit
+])
+def test_tile_shapes_match_reference(nets, dims, B):
+    """Forward pass and gradients where tiles and parts of the contraction
+    change shape; the tolerances of the tests above (same bf16 operands, f32
+    sums of another order against f64)."""
+    import surrogate_ref as R
+    from xmimsim_amd.surrogate import Surrogate
+    rng = np.random.default_rng(B)
+    s = Surrogate(n_nets=nets, dims=dims, max_batch=B, seed=2)
+    X = rng.normal(0, 1, (B, dims[0])).astype(np.float32)
+    T = rng.normal(0, 1, (B, dims[-1])).astype(np.float32)
+    M = (rng.random((B, dims[-1])) > 0.3).astype(np.float32)
+    print("tiles", nets, dims, B, flush=True)
+    Y = s.predict(X)
+    loss, g = s.gradients(X, T, M)
+    P = s.get_params()
+    for e in sorted({0, nets - 1}):
+        layers = s.unpack(P[e])
+        ref, _ = R.forward(layers, X, use_bf16=True)
+        assert np.abs(Y[e] - ref).max() <= 2e-3 * np.abs(ref).max()
+        rl, rg = R.loss_and_grads(layers, X, T, M, use_bf16=True)
+        assert loss[e] == pytest.approx(rl, rel=1e-3)
+        for dW, db in zip([x[0] for x in rg], [x[1] for x in rg]):
+            assert np.isfinite(dW).all() and np.isfinite(db).all()
+        flat = np.concatenate([np.concatenate([dW.ravel(), db]) for dW, db in rg])
+        assert np.linalg.norm(g[e] - flat) / np.linalg.norm(flat) < 1e-2
+    s.close()

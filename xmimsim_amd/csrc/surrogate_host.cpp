@@ -51,8 +51,10 @@ struct Buf {
 struct Layer {
   int K, N;     /* padded input and output widths */
   Buf W, Wb, WT, b, gW, gb, mW, vW, mb, vb;
-  Buf Z, H, HT; /* hidden layers: pre-activation f32, activation bf16 and its transpose */
-  Buf G, Gb, GT; /* gradient of the loss with respect to this layer's pre-activation */
+  Buf D, H, HT; /* hidden layers: activation gradient f32, activation bf16 and its transpose */
+  Buf Gb, GT;   /* gradient of the loss with respect to this layer's pre-activation */
+  Buf cs;       /* its column sums, in parts of rows */
+  int splits = 1, chunks = 1; /* parts of gW and cs of the last backward pass */
 };
 
 }  // namespace
@@ -60,7 +62,7 @@ struct Layer {
 struct xmi_surrogate {
   int nets = 0, n_layers = 0, max_batch = 0, in_features = 0, out_features = 0, steps = 0;
   std::vector<Layer> L;
-  Buf Xf, X0b, X0T, T, Mk, Y, partial, colsum;
+  Buf Xf, X0b, X0T, T, Mk, Y, partial;
   /* resident training data (xmi_surrogate_set_data) and the per-call
    * buffers of xmi_surrogate_train_resident */
   Buf Xall, Tall, Mall, idx, counts, losses;
@@ -77,7 +79,7 @@ struct xmi_surrogate {
     }                                                                                    \
   } while (0)
 
-static const int SG_LOSS_BLOCKS = 120;
+static const int SG_LOSS_BLOCKS = 512;
 
 static int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
@@ -114,13 +116,16 @@ xmi_surrogate *xmi_surrogate_create(int n_nets, int n_layers, const int *dims, i
     y.N = dims[l + 1];
     const size_t nw = (size_t)n_nets * y.N * y.K, nb = (size_t)n_nets * y.N;
     ok = y.W.alloc(nw * 4) == hipSuccess && y.Wb.alloc(nw * 2) == hipSuccess && y.WT.alloc(nw * 2) == hipSuccess &&
-         y.b.alloc(nb * 4) == hipSuccess && y.gW.alloc(nw * 4) == hipSuccess && y.gb.alloc(nb * 4) == hipSuccess &&
+         y.b.alloc(nb * 4) == hipSuccess && y.gW.alloc(nw * 4 * (size_t)sg_dw_splits(n_nets, y.N, y.K, 0)) == hipSuccess && y.gb.alloc(nb * 4) == hipSuccess &&
          y.mW.alloc(nw * 4) == hipSuccess && y.vW.alloc(nw * 4) == hipSuccess && y.mb.alloc(nb * 4) == hipSuccess &&
          y.vb.alloc(nb * 4) == hipSuccess;
     const size_t na = (size_t)n_nets * B * y.N;
     if (ok && l + 1 < n_layers)
-      ok = y.Z.alloc(na * 4) == hipSuccess && y.H.alloc(na * 2) == hipSuccess && y.HT.alloc(na * 2) == hipSuccess;
-    if (ok) ok = y.G.alloc(na * 4) == hipSuccess && y.Gb.alloc(na * 2) == hipSuccess && y.GT.alloc(na * 2) == hipSuccess;
+      ok = y.D.alloc(na * 4) == hipSuccess && y.H.alloc(na * 2) == hipSuccess && y.HT.alloc(na * 2) == hipSuccess;
+    /* column sums of at least 32 rows each */
+    if (ok)
+      ok = y.cs.alloc((size_t)n_nets * (B / 32) * y.N * 4) == hipSuccess && y.Gb.alloc(na * 2) == hipSuccess &&
+           y.GT.alloc(na * 2) == hipSuccess;
     if (!ok) break;
     /* He-normal weights (zero on the padded input columns), zero biases */
     std::vector<float> w(nw, 0.0f);
@@ -137,12 +142,6 @@ xmi_surrogate *xmi_surrogate_create(int n_nets, int n_layers, const int *dims, i
          s->X0T.alloc(B * K0 * 2) == hipSuccess && s->T.alloc(B * No * 4) == hipSuccess &&
          s->Mk.alloc(B * No * 4) == hipSuccess && s->Y.alloc((size_t)n_nets * B * No * 4) == hipSuccess &&
          s->partial.alloc((size_t)n_nets * SG_LOSS_BLOCKS * 4) == hipSuccess;
-    size_t cs = 0;
-    for (int l = 0; l < n_layers; l++) {
-      const size_t c = sg_colsum_scratch(n_nets, max_batch, s->L[l].N);
-      cs = c > cs ? c : cs;
-    }
-    if (ok) ok = s->colsum.alloc(cs * 4) == hipSuccess;
   }
   /* bf16 copies of the initial weights */
   for (int l = 0; l < n_layers && ok; l++) {
@@ -181,8 +180,9 @@ int xmi_surrogate_padded_width(const xmi_surrogate *s, int layer) {
 
 }  // extern "C"
 
-/* forward pass of every net on `batch` rows already packed in X0b/X0T */
-static int forward(xmi_surrogate *s, int batch) {
+/* forward pass of every net on `batch` rows already packed in X0b/X0T; with
+ * `train`, what the backward pass reads is stored too */
+static int forward(xmi_surrogate *s, int batch, int train) {
   const size_t B = (size_t)batch;
   for (int l = 0; l < s->n_layers; l++) {
     Layer &y = s->L[l];
@@ -202,12 +202,14 @@ static int forward(xmi_surrogate *s, int batch) {
     e.bias = y.b.as<float>();
     e.s_bias = y.N;
     if (l + 1 < s->n_layers) {
-      e.cf = y.Z.as<float>();
-      e.s_cf = (long)(B * y.N);
       e.cb = y.H.as<uint16_t>();
       e.s_cb = (long)(B * y.N);
-      e.ct = y.HT.as<uint16_t>();
-      e.s_ct = (long)(B * y.N);
+      if (train) {
+        e.cf = y.D.as<float>();
+        e.s_cf = (long)(B * y.N);
+        e.ct = y.HT.as<uint16_t>();
+        e.s_ct = (long)(B * y.N);
+      }
       SG_TRY(sg_launch_gemm(SG_EPI_HIDDEN, s->nets, batch, y.N, y.K, A, lda, sa, y.Wb.as<uint16_t>(), y.K,
                             (long)y.N * y.K, &e, s->st));
     } else {
@@ -227,8 +229,9 @@ static int backward_launch(xmi_surrogate *s, int batch, float inv, const unsigne
   const size_t B = (size_t)batch, No = (size_t)s->out_features;
   Layer &out = s->L[s->n_layers - 1];
   SG_TRY(sg_launch_loss(batch, (int)No, s->nets, s->Y.as<float>(), s->T.as<float>(), s->Mk.as<float>(), inv, count,
-                        out.G.as<float>(), out.Gb.as<uint16_t>(), out.GT.as<uint16_t>(), partial, SG_LOSS_BLOCKS,
+                        out.Gb.as<uint16_t>(), out.GT.as<uint16_t>(), out.cs.as<float>(), partial, SG_LOSS_BLOCKS,
                         s->st));
+  out.chunks = batch / 64;
   for (int l = s->n_layers - 1; l >= 0; l--) {
     Layer &y = s->L[l];
     /* dW = G^T X: [N x B] . [K x B]^T */
@@ -238,23 +241,23 @@ static int backward_launch(xmi_surrogate *s, int batch, float inv, const unsigne
     memset(&e, 0, sizeof(e));
     e.cf = y.gW.as<float>();
     e.s_cf = (long)y.N * y.K;
+    e.splits = y.splits = sg_dw_splits(s->nets, y.N, y.K, batch);
+    e.s_split = (long)s->nets * y.N * y.K;
     SG_TRY(sg_launch_gemm(SG_EPI_DW, s->nets, y.N, y.K, batch, y.GT.as<uint16_t>(), batch, (long)(B * y.N), XT, batch,
                           sxt, &e, s->st));
-    SG_TRY(sg_launch_colsum(s->nets, batch, y.N, y.G.as<float>(), (long)(B * y.N), s->colsum.as<float>(),
-                            y.gb.as<float>(), y.N, s->st));
     if (l > 0) {
-      /* gradient at the previous pre-activation: (G W) * gelu'(Z_prev): [B x N] . [K x N]^T */
+      /* gradient at the previous pre-activation: (G W) * the activation gradient: [B x N] . [K x N]^T */
       Layer &p = s->L[l - 1];
       SgEpiArgs d;
       memset(&d, 0, sizeof(d));
-      d.cf = p.G.as<float>();
-      d.s_cf = (long)(B * p.N);
       d.cb = p.Gb.as<uint16_t>();
       d.s_cb = (long)(B * p.N);
       d.ct = p.GT.as<uint16_t>();
       d.s_ct = (long)(B * p.N);
-      d.zprev = p.Z.as<float>();
-      d.s_zprev = (long)(B * p.N);
+      d.dprev = p.D.as<float>();
+      d.s_dprev = (long)(B * p.N);
+      d.cs = p.cs.as<float>();
+      p.chunks = batch / sg_dx_chunk(s->nets, batch, y.K);
       SG_TRY(sg_launch_gemm(SG_EPI_DX, s->nets, batch, y.K, y.N, y.Gb.as<uint16_t>(), y.N, (long)(B * y.N),
                             y.WT.as<uint16_t>(), y.N, (long)y.N * y.K, &d, s->st));
     }
@@ -302,12 +305,37 @@ static int adam_launch(xmi_surrogate *s, float lr) {
   s->steps++;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - powf(b1, (float)s->steps), c2 = 1.0f - powf(b2, (float)s->steps);
-  for (Layer &y : s->L) {
-    const size_t nw = (size_t)s->nets * y.N * y.K, nb = (size_t)s->nets * y.N;
-    SG_TRY(sg_launch_adam(nw, y.N, y.K, y.W.as<float>(), y.gW.as<float>(), y.mW.as<float>(), y.vW.as<float>(), lr, b1,
-                          b2, eps, c1, c2, y.Wb.as<uint16_t>(), y.WT.as<uint16_t>(), s->st));
-    SG_TRY(sg_launch_adam(nb, 1, 1, y.b.as<float>(), y.gb.as<float>(), y.mb.as<float>(), y.vb.as<float>(), lr, b1, b2,
-                          eps, c1, c2, nullptr, nullptr, s->st));
+  SgAdamArgs a;
+  memset(&a, 0, sizeof(a));
+  a.nets = s->nets;
+  a.lr = lr;
+  a.b1 = b1;
+  a.b2 = b2;
+  a.eps = eps;
+  a.c1 = c1;
+  a.c2 = c2;
+  for (int l0 = 0; l0 < s->n_layers; l0 += SG_ADAM_LAYERS) {
+    const int n = s->n_layers - l0 < SG_ADAM_LAYERS ? s->n_layers - l0 : SG_ADAM_LAYERS;
+    for (int l = 0; l < n; l++) {
+      const Layer &y = s->L[l0 + l];
+      SgAdamLayer &o = a.layer[l];
+      o.N = y.N;
+      o.K = y.K;
+      o.splits = y.splits;
+      o.chunks = y.chunks;
+      o.s_split = (size_t)s->nets * y.N * y.K;
+      o.gW = y.gW.as<float>();
+      o.cs = y.cs.as<float>();
+      o.W = y.W.as<float>();
+      o.mW = y.mW.as<float>();
+      o.vW = y.vW.as<float>();
+      o.b = y.b.as<float>();
+      o.mb = y.mb.as<float>();
+      o.vb = y.vb.as<float>();
+      o.Wb = y.Wb.as<uint16_t>();
+      o.WT = y.WT.as<uint16_t>();
+    }
+    SG_TRY(sg_launch_adam(&a, n, s->st));
   }
   return 1;
 }
@@ -319,7 +347,7 @@ extern "C" {
 int xmi_surrogate_train_step(xmi_surrogate *s, const float *X, const float *T, const float *mask, int batch, float lr,
                              float *loss) {
   if (!s || !check_batch(s, batch)) return 0;
-  if (!pack_inputs(s, X, batch) || !forward(s, batch) || !backward(s, batch, T, mask, loss)) return 0;
+  if (!pack_inputs(s, X, batch) || !forward(s, batch, 1) || !backward(s, batch, T, mask, loss)) return 0;
   if (!adam_launch(s, lr)) return 0;
   SG_TRY(hipStreamSynchronize(s->st));
   return 1;
@@ -366,7 +394,7 @@ int xmi_surrogate_train_resident(xmi_surrogate *s, const int32_t *idx, int steps
     SG_TRY(sg_launch_gather(batch, s->in_features, ld, s->out_features, s->idx.as<int>() + (size_t)k * batch,
                             s->Xall.as<float>(), s->Tall.as<float>(), s->Mall.as<float>(), s->X0b.as<uint16_t>(),
                             s->X0T.as<uint16_t>(), s->T.as<float>(), s->Mk.as<float>(), cnt, s->st));
-    if (!forward(s, batch) ||
+    if (!forward(s, batch, 1) ||
         !backward_launch(s, batch, 0.0f, cnt, s->losses.as<float>() + (size_t)k * s->nets * SG_LOSS_BLOCKS) ||
         !adam_launch(s, lr[k]))
       return 0;
@@ -392,7 +420,13 @@ int xmi_surrogate_train_resident(xmi_surrogate *s, const int32_t *idx, int steps
 int xmi_surrogate_gradients(xmi_surrogate *s, const float *X, const float *T, const float *mask, int batch,
                             float *loss, float *grad) {
   if (!s || !check_batch(s, batch)) return 0;
-  if (!pack_inputs(s, X, batch) || !forward(s, batch) || !backward(s, batch, T, mask, loss)) return 0;
+  if (!pack_inputs(s, X, batch) || !forward(s, batch, 1) || !backward(s, batch, T, mask, loss)) return 0;
+  for (Layer &y : s->L) {
+    const size_t nw = (size_t)s->nets * y.N * y.K;
+    if (y.splits > 1) SG_TRY(sg_launch_sum(nw, y.splits, nw, y.gW.as<float>(), s->st));
+    SG_TRY(sg_launch_bias_grad(s->nets, y.N, y.chunks, y.cs.as<float>(), y.gb.as<float>(), s->st));
+  }
+  SG_TRY(hipStreamSynchronize(s->st));
   const long per = xmi_surrogate_param_count(s);
   for (int e = 0; e < s->nets; e++) {
     float *g = grad + (size_t)e * per;
@@ -409,7 +443,7 @@ int xmi_surrogate_gradients(xmi_surrogate *s, const float *X, const float *T, co
 /* outputs of every net: Y[n_nets][batch][out_features] */
 int xmi_surrogate_predict(xmi_surrogate *s, const float *X, int batch, float *Y) {
   if (!s || !check_batch(s, batch)) return 0;
-  if (!pack_inputs(s, X, batch) || !forward(s, batch)) return 0;
+  if (!pack_inputs(s, X, batch) || !forward(s, batch, 0)) return 0;
   const size_t No = (size_t)s->out_features, B = (size_t)batch;
   for (int e = 0; e < s->nets; e++)
     SG_TRY(hipMemcpyAsync(Y + (size_t)e * B * No, s->Y.as<float>() + (size_t)e * B * No, B * No * 4,
