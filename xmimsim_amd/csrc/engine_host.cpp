@@ -1048,7 +1048,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
      * live photons: each of its waves takes at most ceil(slots / (64 W))
      * trips of 64 entries, and a sub-queue serves ceil(W / ENG_SPREAD) of
      * its W waves */
-    const int bblocks = brute ? eng_brute_blocks(n_cu) : 0;
+    const int bblocks = brute ? eng_brute_blocks(n_cu, P.coll_present) : 0;
     if (brute) {
       const long W = (long)bblocks * (ENG_BLOCK / 64);
       const long trips = ((long)slots + 64 * W - 1) / (64 * W);

@@ -128,7 +128,7 @@ hipError_t eng_launch_source_queued(const EngineParams *P, const PhotonSoA *S, c
 hipError_t eng_launch_order_brute(const EngineParams *P, const PhotonSoA *S, int n, int count, int blocks,
                                   hipStream_t st, hipEvent_t *ev /* 3 events (before, between, after) or NULL */);
 /* workgroups of the brute-force grid: one resident round of the step kernel */
-int eng_brute_blocks(int n_cu);
+int eng_brute_blocks(int n_cu, int coll);
 hipError_t eng_launch_order(const EngineParams *P, const PhotonSoA *S, const VrSoA *V, int n, int count, int n_cu,
                             hipStream_t st, hipEvent_t *ev);
 #ifdef __cplusplus

@@ -686,13 +686,6 @@ __device__ __forceinline__ void d_enqueue(const EngineParams &P, int type, int i
   for (int t = 0; t < 3; t++) d_append(P, t, type == t, idx);
 }
 
-/* photon of queue entry q (0 <= q < ENG_SPREAD * qreg) of type t, or -1 */
-__device__ __forceinline__ int d_dequeue(const EngineParams &P, int t, unsigned int q) {
-  const unsigned int j = q / (unsigned int)P.qreg, r = q - j * (unsigned int)P.qreg;
-  if (j >= ENG_SPREAD || r >= P.qcount[(size_t)t * ENG_SPREAD + j]) return -1;
-  return P.queue[((size_t)t * ENG_SPREAD + j) * P.qreg + r];
-}
-
 /* layer lists: k_step stores each wave's number of events per layer (0 = no
  * event), k_layer_scan turns them into offsets, k_vr_list writes the slots.
  * Both launches run one thread per slot with the same workgroups, so a slot
@@ -2388,23 +2381,25 @@ __device__ __forceinline__ void d_list_append(int *list, unsigned int *cnt, int 
 }
 
 /* entry q of the concatenated interaction queues (Rayleigh, Compton, photo;
- * each queue's ENG_SPREAD sub-queues in order; off: their prefix sums):
- * the photon's interaction.  Returns 1 when a cascade started an offspring */
-template <bool BRUTE, bool ADV>
-__device__ __forceinline__ int d_interact_entry(const EngineParams &P, const PhotonSoA &S, int n,
-                                                const unsigned int *off, unsigned int q, int *slot) {
-  constexpr int NS = 3 * ENG_SPREAD;
-  int lo = 0, hi = NS;
+ * each queue's ENG_SPREAD sub-queues in order; off: their prefix sums): the
+ * photon's slot, and the queue in *type */
+__device__ __forceinline__ int d_queue_entry(const EngineParams &P, const unsigned int *off, unsigned int q, int *type) {
+  int lo = 0, hi = 3 * ENG_SPREAD;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (off[mid] <= q) lo = mid;
     else hi = mid;
   }
-  const int t = lo / ENG_SPREAD;
-  const int i = P.queue[(size_t)lo * P.qreg + (q - off[lo])];
-  *slot = i;
-  if (t == 0) d_rayleigh_one<BRUTE>(P, S, n, i);
-  else if (t == 1) d_compton_one<BRUTE, ADV>(P, S, n, i);
+  *type = lo / ENG_SPREAD;
+  return P.queue[(size_t)lo * P.qreg + (q - off[lo])];
+}
+
+/* the interaction of the photon in slot i from queue `type`; returns 1 when a
+ * cascade started an offspring */
+template <bool BRUTE, bool ADV>
+__device__ __forceinline__ int d_interact_one(const EngineParams &P, const PhotonSoA &S, int n, int type, int i) {
+  if (type == 0) d_rayleigh_one<BRUTE>(P, S, n, i);
+  else if (type == 1) d_compton_one<BRUTE, ADV>(P, S, n, i);
   else return d_photo_one<BRUTE>(P, S, n, i);
   return 0;
 }
@@ -2425,8 +2420,9 @@ k_interact(EngineParams P, PhotonSoA S, int n) {
   __syncthreads();
   const unsigned int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= off[3 * ENG_SPREAD]) return;
-  int i;
-  (void)d_interact_entry<false, ADV>(P, S, n, off, q, &i);
+  int type;
+  const int i = d_queue_entry(P, off, q, &type);
+  (void)d_interact_one<false, ADV>(P, S, n, type, i);
 }
 
 /* the brute-force interactions (analogue yields, cascades), one thread per
@@ -2444,7 +2440,11 @@ k_interact_brute(EngineParams P, PhotonSoA S, int n) {
   const unsigned int total = off[3 * ENG_SPREAD], q = blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x * blockDim.x >= total) return;
   int i = -1, spawned = 0;
-  if (q < total) spawned = d_interact_entry<true, ADV>(P, S, n, off, q, &i);
+  if (q < total) {
+    int type;
+    i = d_queue_entry(P, off, q, &type);
+    spawned = d_interact_one<true, ADV>(P, S, n, type, i);
+  }
   d_list_append(P.olist_out, P.ocount_out, spawned, i + P.off_half);
 }
 
@@ -2457,54 +2457,89 @@ k_interact_brute(EngineParams P, PhotonSoA S, int n) {
  * element and line (weight times fluorescence yield), and the weight after
  * the forced step of every interacted photon normalises its input energy.
  * One thread per queue entry of the three interaction queues. */
+
+/* integer sum of v over the wavefront, wave-uniform (the steps of
+ * d_wave_total) */
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ unsigned long long d_dpp0_u64(unsigned long long v) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROW_MASK, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), CTRL, ROW_MASK, 0xf, true);
+  return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long d_wave_total_u64(unsigned long long v) {
+  v += d_dpp0_u64<0x111, 0xf>(v);
+  v += d_dpp0_u64<0x112, 0xf>(v);
+  v += d_dpp0_u64<0x114, 0xf>(v);
+  v += d_dpp0_u64<0x118, 0xf>(v);
+  v += d_dpp0_u64<0x142, 0xa>(v);
+  v += d_dpp0_u64<0x143, 0xc>(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, 63);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), 63);
+  return ((unsigned long long)hi << 32) | lo;
+}
+
 /* exact wave-aggregated fixed-point add: every lane with key >= 0 adds
  * value to bin key of tally; the lanes of one key are summed as integers
  * (three 42-bit limbs, which 64 lanes cannot overflow) and added once, so
  * that thousands of photons of one bin do not serialise on its address and
- * the sum does not depend on which photons share a wavefront.  Call from
- * converged code. */
+ * the sum does not depend on which photons share a wavefront.  From the first
+ * key with fewer than FEW lanes on, the remaining lanes add for themselves
+ * (Compton energies: nearly every lane its own bin).  Call from converged
+ * code. */
+template <int FEW>
 __device__ __forceinline__ void d_fx_add_keyed(unsigned long long *tally, long key, double value, int shift) {
+  unsigned long long pending = __ballot(key >= 0);
+  if (!pending) return;
   unsigned long long lo = 0ull, hi = 0ull;
   if (key >= 0) fx_split(value, shift, &lo, &hi);
   const unsigned long long M42 = (1ull << 42) - 1ull;
   const unsigned long long l0 = lo & M42, l1 = (lo >> 42) | ((hi & ((1ull << 20) - 1ull)) << 22), l2 = hi >> 20;
-  unsigned long long pending = __ballot(key >= 0);
   while (pending) {
     const int leader = __ffsll((long long)pending) - 1;
-    const long k = __shfl(key, leader);
+    const long k = (long)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(key >> 32), leader) << 32) |
+                          (unsigned)__builtin_amdgcn_readlane((int)key, leader));
     const int mine = key == k;
-    unsigned long long a0 = mine ? l0 : 0ull, a1 = mine ? l1 : 0ull, a2 = mine ? l2 : 0ull;
-    for (int off = 32; off > 0; off >>= 1) {
-      a0 += __shfl_xor(a0, off);
-      a1 += __shfl_xor(a1, off);
-      a2 += __shfl_xor(a2, off);
+    const unsigned long long group = __ballot(mine);
+    if (FEW > 1 && __popcll(group) < FEW) {
+      if ((pending >> __lane_id()) & 1ull) fx_merge_global(&tally[(size_t)key * 2], lo, hi);
+      return;
     }
+    const unsigned long long a0 = d_wave_total_u64(mine ? l0 : 0ull), a1 = d_wave_total_u64(mine ? l1 : 0ull),
+                             a2 = d_wave_total_u64(mine ? l2 : 0ull);
     if (__lane_id() == leader) {
       const unsigned __int128 t = (unsigned __int128)a0 + ((unsigned __int128)a1 << 42) + ((unsigned __int128)a2 << 84);
       fx_merge_global(&tally[(size_t)k * 2], (unsigned long long)t, (unsigned long long)(t >> 64));
     }
-    pending &= ~__ballot(mine);
+    pending &= ~group;
   }
 }
 
-__global__ void __launch_bounds__(ENG_BLOCK) k_escape(EngineParams P, PhotonSoA S, VrSoA V, EscParams Q) {
-  const unsigned int per = (unsigned int)ENG_SPREAD * (unsigned int)P.qreg;
-  const unsigned int q = blockIdx.x * blockDim.x + threadIdx.x;
-  const int type = (int)(q / per);
-  const int i = type <= 2 ? d_dequeue(P, type, q - (unsigned int)type * per) : -1;
+/* interaction and way out in one thread, so that the photon's record stays in
+ * the caches between them: a launch of its own over the record of 8e6 photons
+ * took 555 us after the interactions' 520 and a copy of the weights; together
+ * 831 (four waves per SIMD; six spill and take 879) */
+__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(4)))
+k_interact_escape(EngineParams P, PhotonSoA S, EscParams Q) {
+  __shared__ unsigned int off[3 * ENG_SPREAD + 1];
+  d_queue_offsets(P.qcount, off);
+  __syncthreads();
+  const unsigned int total = off[3 * ENG_SPREAD], q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x * blockDim.x >= total) return;
   const int shift = P.tally_shift;
   long key_n = -1, key_c = -1, key_f = -1;
   double w_n = 0.0, w = 0.0;
-  if (i >= 0) {
+  if (q < total) {
+    int type;
+    const int i = d_queue_entry(P, off, q, &type);
+    w_n = S.weight[i];
+    (void)d_interact_one<false, false>(P, S, 1, type, i);
     const int iE = (int)(S.hid[i] / (uint64_t)Q.n_photons);
     if (iE >= 0 && iE < Q.nE) {
-      /* the photon's weight after the forced step (V.pesc) normalises;
-       * the photo-absorption step has multiplied S.weight by the
-       * fluorescence yield, which an
-       * escape-ratio run applies to the escape tally only
+      /* the photon's weight after the forced step (w_n) normalises; the
+       * photo-absorption step has multiplied S.weight by the fluorescence
+       * yield, which an escape-ratio run applies to the escape tally only
        * (src/xmi_variance_reduction.F90:742-746) */
       key_n = iE;
-      w_n = V.pesc[i];
       w = S.weight[i];
       const double E = S.energy[i];
       const int cur = S.layer[i];
@@ -2544,9 +2579,9 @@ __global__ void __launch_bounds__(ENG_BLOCK) k_escape(EngineParams P, PhotonSoA 
       }
     }
   }
-  d_fx_add_keyed(Q.interacted, key_n, w_n, shift);
-  d_fx_add_keyed(Q.compton, key_c, w, shift);
-  d_fx_add_keyed(Q.fluo, key_f, w, shift);
+  d_fx_add_keyed<1>(Q.interacted, key_n, w_n, shift);
+  d_fx_add_keyed<4>(Q.compton, key_c, w, shift);
+  d_fx_add_keyed<1>(Q.fluo, key_f, w, shift);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -2594,12 +2629,13 @@ __device__ __forceinline__ void d_det_frame(const EngineParams &P, const double 
  * (L, L, L) crosses x = 0 at (0, e_y - e_x, e_z - e_x), always as a crossing
  * from behind.  Kept as computed there.  A line parallel to the window,
  * where the reference stops the program, counts as no crossing. */
-__device__ int d_detector_segment(const EngineParams &P, const double *b, const double *e) {
+template <bool COLL>
+__device__ __forceinline__ int d_detector_segment(const EngineParams &P, const double *b, const double *e) {
   double bd[3], ed[3], ip[3];
   d_det_frame(P, b, bd);
   d_det_frame(P, e, ed);
   const double o[3] = {0.0, 0.0, 0.0}, nx[3] = {1.0, 0.0, 0.0};
-  if (!P.coll_present) {
+  if (!COLL) {
     if (bd[0] * ed[0] > 0.0) return 0;
     const double L = d_distance(ed, bd);
     const double ld[3] = {L, L, L};
@@ -2641,7 +2677,8 @@ __device__ int d_detector_segment(const EngineParams &P, const double *b, const 
  * left the sample reaches the detector when it moves against the detector
  * normal and crosses the window (and the collimator's top) within their
  * radii */
-__device__ int d_escape_hits_detector(const EngineParams &P, const double *coords, const double *dirv) {
+template <bool COLL>
+__device__ __forceinline__ int d_escape_hits_detector(const EngineParams &P, const double *coords, const double *dirv) {
   if (d_dot(dirv, P.n_det) >= 0.0) return 0;
   double dd[3], cd[3], ip[3];
   d_matvec(P.det_inv, dirv, dd);
@@ -2649,7 +2686,7 @@ __device__ int d_escape_hits_detector(const EngineParams &P, const double *coord
   const double o[3] = {0.0, 0.0, 0.0}, nx[3] = {1.0, 0.0, 0.0};
   if (!d_intersect(o, nx, cd, dd, ip)) return 0;
   if (d_norm(ip) > P.det_radius) return 0;
-  if (!P.coll_present) return 1;
+  if (!COLL) return 1;
   const double pc[3] = {P.coll_height, 0.0, 0.0};
   if (!d_intersect(pc, nx, cd, dd, ip)) return 0;
   ip[0] = 0.0;
@@ -2660,6 +2697,7 @@ __device__ int d_escape_hits_detector(const EngineParams &P, const double *coord
  * interactions takes its step; one that stays in the sample with fewer than
  * n_int interactions gets its atom and interaction type (*type), the others
  * end, those that reach the detector tallied (*key_ch, *key_h, *w_hit) */
+template <bool COLL>
 __device__ __forceinline__ void d_brute_step(const EngineParams &P, const PhotonSoA &S, int n, int i, int *type,
                                              int *stepped, int *reached, long *key_ch, long *key_h, double *w_hit) {
   const size_t cap = (size_t)P.cap;
@@ -2687,13 +2725,13 @@ __device__ __forceinline__ void d_brute_step(const EngineParams &P, const Photon
     const double mu = S.mus[(size_t)l0 * cap + i];
     double dist = d_distance(c, ip);
     const double temp_prod = -1.0 * dist * P.layer_density[l0] * mu;
-    const double tempexp = exp(temp_prod);
+    const double em = expm1(temp_prod); /* e^t = 1 + em to the rounding that max_r carries */
     min_r = max_r;
-    max_r = max_r - blbs * expm1(temp_prod);
+    max_r = max_r - blbs * em;
     if (R <= max_r) {
       dist = -1.0 * log1p(-1.0 * (R - min_r) / blbs) / mu / P.layer_density[l0];
       const double to[3] = {c[0] + dist * dirv[0], c[1] + dist * dirv[1], c[2] + dist * dirv[2]};
-      const int rc = d_detector_segment(P, c, to);
+      const int rc = d_detector_segment<COLL>(P, c, to);
       c[0] = to[0];
       c[1] = to[1];
       c[2] = to[2];
@@ -2705,7 +2743,7 @@ __device__ __forceinline__ void d_brute_step(const EngineParams &P, const Photon
       }
       break;
     }
-    const int rc = d_detector_segment(P, c, ip);
+    const int rc = d_detector_segment<COLL>(P, c, ip);
     if (rc) {
       ended = 1;
       hit = rc == 2;
@@ -2714,9 +2752,9 @@ __device__ __forceinline__ void d_brute_step(const EngineParams &P, const Photon
     c[0] = ip[0];
     c[1] = ip[1];
     c[2] = ip[2];
-    blbs = blbs * tempexp;
+    blbs = fma(blbs, em, blbs);
   }
-  if (!inside && !ended) hit = d_escape_hits_detector(P, c, dirv);
+  if (!inside && !ended) hit = d_escape_hits_detector<COLL>(P, c, dirv);
   if (hit) {
     /* channels(n_interactions:, channel) and the history row of the last
      * interaction; the host sums the orders into the cumulative rows */
@@ -2743,9 +2781,13 @@ __device__ __forceinline__ void d_brute_step(const EngineParams &P, const Photon
  * interaction queues (those that interacted) followed by the offspring that
  * its cascades started.  A fixed grid strides over them, every lane of a
  * wave taking the same trips, so that the queue appends, counters and
- * tallies see converged waves.  Three waves per SIMD (166 VGPRs, 8 spilled)
- * run 17 % faster than the two that 183 unconstrained VGPRs allow. */
-__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(3)))
+ * tallies see converged waves.  COLL: with a detector collimator, whose cone
+ * test takes the registers (163 VGPRs, three waves per SIMD); without one four
+ * waves (128 VGPRs) run 7 % faster than three and 10 % than five, whose spills
+ * cost more: 371 us a launch over the orders of 8e6 photons, 414 with the cone
+ * test compiled in and two exponentials a layer. */
+template <bool COLL>
+__global__ void __launch_bounds__(ENG_BLOCK) __attribute__((amdgpu_waves_per_eu(COLL ? 3 : 4)))
 k_step_brute(EngineParams P, PhotonSoA S, int n, int count) {
   constexpr int NS = 3 * ENG_SPREAD;
   __shared__ unsigned int off[NS + 1];
@@ -2776,13 +2818,13 @@ k_step_brute(EngineParams P, PhotonSoA S, int n, int count) {
       } else {
         i = P.olist_in[q - nq];
       }
-      if (S.layer[i] > 0) d_brute_step(P, S, n, i, &type, &stepped, &reached, &key_ch, &key_h, &w_hit);
+      if (S.layer[i] > 0) d_brute_step<COLL>(P, S, n, i, &type, &stepped, &reached, &key_ch, &key_h, &w_hit);
     }
     d_enqueue(P, type, i);
     d_wave_count(d_ctr(P, ENG_CNT_STEPS), stepped);
     d_wave_count(d_ctr(P, ENG_CNT_HITS), reached);
-    d_fx_add_keyed(P.t_bch, key_ch, w_hit, P.tally_shift);
-    d_fx_add_keyed(P.t_bhist, key_h, w_hit, P.tally_shift);
+    d_fx_add_keyed<4>(P.t_bch, key_ch, w_hit, P.tally_shift);
+    d_fx_add_keyed<4>(P.t_bhist, key_h, w_hit, P.tally_shift);
   }
 }
 
@@ -2921,9 +2963,8 @@ hipError_t eng_launch_source_queued(const EngineParams *P, const PhotonSoA *S, c
   return hipGetLastError();
 }
 
-/* one escape-ratio batch: the forced first interaction, the weight after it
- * kept in V.pesc (the weight of the escape tallies), the interaction, the
- * escape test and tallies */
+/* one escape-ratio batch: the forced step, then the interaction with the
+ * escape test and its tallies */
 hipError_t eng_launch_escape(const EngineParams *P, const PhotonSoA *S, const VrSoA *V, const EscParams *Q,
                              int count, hipStream_t st) {
   int blocks = (count + ENG_BLOCK - 1) / ENG_BLOCK;
@@ -2936,11 +2977,7 @@ hipError_t eng_launch_escape(const EngineParams *P, const PhotonSoA *S, const Vr
     else if (nl <= 8) hipLaunchKernelGGL((k_step<8, false>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, 1, count);
     else hipLaunchKernelGGL((k_step<16, false>), dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, 1, count);
   }
-  hipError_t e = hipMemcpyAsync(V->pesc, S->weight, sizeof(double) * (size_t)count, hipMemcpyDeviceToDevice, st);
-  if (e != hipSuccess) return e;
-  launch_interact(P, S, 1, (count + ENG_BLOCK - 1) / ENG_BLOCK, st);
-  const int eblocks = (int)((3 * (size_t)ENG_SPREAD * P->qreg + ENG_BLOCK - 1) / ENG_BLOCK);
-  hipLaunchKernelGGL(k_escape, dim3(eblocks), dim3(ENG_BLOCK), 0, st, *P, *S, *V, *Q);
+  hipLaunchKernelGGL(k_interact_escape, dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, *Q);
   return hipGetLastError();
 }
 
@@ -2948,7 +2985,8 @@ hipError_t eng_launch_order_brute(const EngineParams *P, const PhotonSoA *S, int
                                   hipStream_t st, hipEvent_t *ev) {
   hipLaunchKernelGGL(k_reset_queues, dim3(1), dim3(ENG_NQUEUES * ENG_SPREAD), 0, st, *P);
   if (ev) (void)hipEventRecord(ev[0], st);
-  hipLaunchKernelGGL(k_step_brute, dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, n, count);
+  if (P->coll_present) hipLaunchKernelGGL(k_step_brute<true>, dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, n, count);
+  else hipLaunchKernelGGL(k_step_brute<false>, dim3(blocks), dim3(ENG_BLOCK), 0, st, *P, *S, n, count);
   if (ev) (void)hipEventRecord(ev[1], st);
   /* the interactions: one thread per photon that may be alive */
   const int alive = (n == 1 || !P->off_half) ? count : 2 * count;
@@ -2957,9 +2995,10 @@ hipError_t eng_launch_order_brute(const EngineParams *P, const PhotonSoA *S, int
   return hipGetLastError();
 }
 
-int eng_brute_blocks(int n_cu) {
+int eng_brute_blocks(int n_cu, int coll) {
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_step_brute, ENG_BLOCK, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, coll ? (const void *)k_step_brute<true> : (const void *)k_step_brute<false>,
+                                                   ENG_BLOCK, 0) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
   return n_cu * per_cu;

@@ -335,6 +335,7 @@ XRL_FN double xrl_total_profile_cdf(const xrl_atom *a, double pz) {
 XRL_FN double xrl_bisect_G3(double target, double p, double lo, double hi) {
   for (int it = 0; it < 100; it++) {
     double mid = 0.5 * (lo + hi);
+    if (mid == lo || mid == hi) break; /* further steps keep the interval */
     if (xrl_profile_G3(mid / p) < target) lo = mid;
     else hi = mid;
   }
@@ -345,6 +346,7 @@ XRL_FN double xrl_bisect_G3(double target, double p, double lo, double hi) {
 XRL_FN double xrl_bisect_total_profile(const xrl_atom *a, double target, double lo, double hi) {
   for (int it = 0; it < 100; it++) {
     double mid = 0.5 * (lo + hi);
+    if (mid == lo || mid == hi) break; /* further steps keep the interval */
     if (xrl_total_profile_cdf(a, mid) < target) lo = mid;
     else hi = mid;
   }
@@ -357,6 +359,7 @@ XRL_FN double xrl_bisect_phi(double t, double target) {
   double lo = 0.0, hi = 2.0 * 3.14159265358979323846;
   for (int it = 0; it < 100; it++) {
     double mid = 0.5 * (lo + hi);
+    if (mid == lo || mid == hi) break;
     if (mid - t * sin(2.0 * mid) < target) lo = mid;
     else hi = mid;
   }
