@@ -42,7 +42,8 @@ def _nl_bound(n_layers: int) -> int:
 
 def lines_kp_candidates(n_layers: int) -> Tuple[int, ...]:
     """Photons per lane, besides the default, that the line kernel is built
-    for at this layer count (default 3 up to four layers, 2 up to eight, 1)."""
+    for at this layer count (default 4 up to three layers, 3 up to five, 2 up
+    to eight, 1 beyond)."""
     nl = _nl_bound(n_layers)
     return (2, 4) if nl <= 4 else ((1,) if nl <= 8 else ())
 

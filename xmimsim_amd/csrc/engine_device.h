@@ -153,6 +153,7 @@ struct EngineParams {
   const double *precalc_xrf;    /* [nZ][9][nZ][219] */
   const double *line_E;         /* [nZ][219] */
   const double *rate_cum;       /* [nZ][220] radiative rates summed along each shell's lines, index |line| */
+  const double *auger_cum;      /* [nZ][XRL_AUGER_N] Auger rates summed along each shell's transitions */
   const double *precalc_mu;     /* [n_layers][nZ][219] */
   /* the estimator's active lines flattened per layer: entry t of layer l (fl_off[l] <= t <
    * fl_off[l+1]) is active line q of element u of that layer */

@@ -234,7 +234,7 @@ struct DeviceTables {
   const xmi_hdf5F *owner = nullptr;
   int nZ = 0;
   int Zs[XMI_MAXZ + 1];
-  DevBuf atoms, ray, comp, tabE, tabR, fycorr, ipE, ipr, iprc, ipoff, ipacc, cp_icdf, cp_rn, precalc_xrf, lineE, rate_cum;
+  DevBuf atoms, ray, comp, tabE, tabR, fycorr, ipE, ipr, iprc, ipoff, ipacc, cp_icdf, cp_rn, precalc_xrf, lineE, rate_cum, auger_cum;
   DevBuf cp_cdfg, cp_gscale;
   DevBuf phi, phiT, phiR;
   /* the advanced Compton model's subshell profiles, uploaded on first use */
@@ -335,7 +335,7 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
   std::vector<double> ipE, ipr, iprc;
   std::vector<int> ipoff(nZ + 1), ipacc((size_t)nZ * ENG_IP_ACC);
   std::vector<double> pxrf((size_t)nZ * 9 * nZ * XMI_NLINES_VR, 0.0), lineE((size_t)nZ * XMI_NLINES_VR, 0.0),
-      rcum((size_t)nZ * (XMI_NLINES_VR + 1), 0.0);
+      rcum((size_t)nZ * (XMI_NLINES_VR + 1), 0.0), acum((size_t)nZ * XRL_AUGER_N, 0.0);
   t->ip_acc_E0 = z0->ip_energies[0];
   double Emax = z0->ip_energies[z0->ip_len - 1];
   t->ip_acc_inv = (double)ENG_IP_ACC / (Emax - t->ip_acc_E0);
@@ -376,6 +376,9 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
       xrl_shell_lines(sh, &first, &last);
       double sum = 0.0;
       for (int l = first; l <= last; l++) rcum[(size_t)i * (XMI_NLINES_VR + 1) + l] = sum += atoms[i].rad_rate[l];
+      sum = 0.0;
+      if (xrl_auger_range(sh, &first, &last))
+        for (int k = first; k <= last; k++) acum[(size_t)i * XRL_AUGER_N + k] = sum += xrl_auger_rate(&atoms[i], k);
     }
   }
   ipoff[nZ] = (int)ipE.size();
@@ -397,6 +400,7 @@ static DeviceTables *get_tables(const xmi_hdf5F *h, hipStream_t st, Staging &sg)
   hipError_t e = hipSuccess;
   e = upload(t->atoms, atoms.data(), atoms.size(), st, sg);
   if (e == hipSuccess) e = upload(t->rate_cum, rcum.data(), rcum.size(), st, sg);
+  if (e == hipSuccess) e = upload(t->auger_cum, acum.data(), acum.size(), st, sg);
   if (e == hipSuccess) e = upload(t->ray, ray.data(), ray.size(), st, sg);
   if (e == hipSuccess) e = upload(t->comp, comp.data(), comp.size(), st, sg);
   if (e == hipSuccess) e = upload(t->tabE, z0->Energies, (size_t)t->n_e, st, sg);
@@ -1147,6 +1151,7 @@ static int msim_run(Engine &E, xmi_inputFPtr inputFPtr, xmi_hdf5FPtr hdf5FPtr, i
     P.precalc_xrf = T->precalc_xrf.as<double>();
     P.line_E = T->lineE.as<double>();
     P.rate_cum = T->rate_cum.as<double>();
+    P.auger_cum = T->auger_cum.as<double>();
     P.tab_uniform = T->tab_uniform;
     P.n_lay_el = (int)elZ.size();
     P.phi_icdf = T->phi.as<double>();

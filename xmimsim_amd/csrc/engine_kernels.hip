@@ -2221,16 +2221,18 @@ __device__ int d_cascade_auger(const EngineParams &P, const PhotonSoA &S, int i,
   int first, last, spawned = 0;
   if (!xrl_auger_range(shell, &first, &last)) return 0;
   const double r = phx_uniform(s);
-  double sumz = 0.0;
-  int t = -1;
-  for (int k = first; k <= last; k++) {
-    sumz += xrl_auger_rate(a, k);
-    if (r < sumz) {
-      t = k;
-      break;
-    }
+  /* the first transition whose running sum exceeds r; five or six probes of
+   * the table replace up to 64 rates of several divisions each, formed by the
+   * few lanes of a wave whose vacancies decay so: the brute-force interactions
+  XX
+  const double *cum = P.auger_cum + (size_t)u * XRL_AUGER_N;
+  int t = first, hi = last + 1;
+  while (t < hi) {
+    const int mid = (t + hi) >> 1;
+    if (r < cum[mid]) hi = mid;
+    else t = mid + 1;
   }
-  if (t < 0) return 0;
+  if (t > last) return 0;
   int sh[2];
   xrl_auger_shells(t, &sh[0], &sh[1]);
   for (int k = 0; k < 2; k++) {
