@@ -133,6 +133,36 @@ def test_axes_that_do_not_increase_take_the_host_routine(orc):
     prep.close()
 
 
+@pytest.mark.parametrize("respond", [api.detector_response, api.detector_response_noalloc])
+def test_no_order_leaves_nothing_under_way(respond):
+    """Calls without an order (only the net-line histories get the detector's
+    absorption) between calls with orders: another detector's tables of a call
+    that has returned must not reach the next one's."""
+    rng = np.random.default_rng(8)
+    preps = []
+    for k, thick in enumerate((0.002, 0.2)):
+        inp = workloads.single_layer_steel(n_photons_line=10, n_interactions=2)
+        inp.nchannels, inp.gain = 128, 0.2
+        inp.det_absorbers = [api.Layer([4 + 9 * k], [1.0], 1.85, thick)]
+        preps.append(api.Prepared(inp))
+    ch = np.zeros((3, 128))
+    ch[1:] = rng.uniform(0.0, 100.0, (2, 128))
+    vr = np.zeros((100, 385, 2))
+    vr[25, 2] = vr[28, 1] = (1e4, 1e3)
+    opts = api.default_options(use_escape_peaks=0, use_sum_peaks=0, use_poisson=0, use_default_seeds=1)
+    v_ref = [vr.copy(), vr.copy()]
+    ref = [respond(p, ch, v, options=opts) for p, v in zip(preps, v_ref)]
+    assert np.abs(ref[0] - ref[1]).max() > 1e-3 * ref[0].max()
+    for k in (0, 1, 1, 0):
+        v = vr.copy()
+        none = respond(preps[1 - k], np.full((1, 128), 7.0), v, options=opts)
+        assert none.shape == (1, 128) and not none.any()
+        assert np.array_equal(v, v_ref[1 - k])
+        assert np.array_equal(respond(preps[k], ch, options=opts), ref[k])
+    for p in preps:
+        p.close()
+
+
 @pytest.mark.parametrize("nch", [200, 4096, 5000])
 def test_pileup_keeps_the_spectrum_without_pulses_in_time(nch):
     """A pulse width of 1e-12 s: every pulse is its own train, so the counts

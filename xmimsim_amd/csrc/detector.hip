@@ -832,8 +832,11 @@ static int det_convolute(const xmi_inputF *in, double **channels_noconv, double 
   d.type = (int)in->detector.detector_type;
   const uint64_t seed = xmi_engine_current_seed(options);
   const int escape = er && !q.host_front;
+  /* without an order the device has nothing to do, and no copy may be under
+   * way when the staging memory goes back to its owner */
+  const int first = zero_interaction ? 0 : 1, any_order = first <= n_interactions_all;
   std::vector<double> eff;
-  if (q.host_front) {
+  if (q.host_front && any_order) {
     eff.resize(nch);
     for (int i = 0; i < nch; i++) eff[i] = det_efficiency(in, i * d.gain + d.zero);
   }
@@ -844,9 +847,9 @@ static int det_convolute(const xmi_inputF *in, double **channels_noconv, double 
   (void)det_carve(block, nch, group, q, &dv);
   const size_t n_const = (size_t)((char *)dv.tab - (char *)dv.lay), n_spec = up((size_t)group * nch * sizeof(double));
   const size_t n_tab = escape ? DET_ESC_WORDS * sizeof(double) : 0;
-  DET_TRY(stage.ensure(n_const + n_spec + n_tab + n_spec + up(group * sizeof(DetTrains))));
+  if (any_order) DET_TRY(stage.ensure(n_const + n_spec + n_tab + n_spec + up(group * sizeof(DetTrains))));
   char *s_spec = stage.p + n_const, *s_tab = s_spec + n_spec, *s_out = s_tab + n_tab, *s_tr = s_out + n_spec;
-  {
+  if (any_order) {
     auto put = [&](const void *dst, const void *src, size_t bytes) {
       if (bytes) memcpy(stage.p + ((const char *)dst - (const char *)dv.lay), src, bytes);
     };
@@ -878,7 +881,7 @@ static int det_convolute(const xmi_inputF *in, double **channels_noconv, double 
     rows_done = true;
   };
   const int nb = (nch + 255) / 256;
-  for (int n0 = zero_interaction ? 0 : 1; n0 <= n_interactions_all; n0 += group) {
+  for (int n0 = first; n0 <= n_interactions_all; n0 += group) {
     const int n_ord = std::min(group, n_interactions_all - n0 + 1);
     for (int n = 0; n < n_ord; n++) {
       double *t = (double *)s_spec + (size_t)n * nch;
