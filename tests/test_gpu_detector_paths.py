@@ -133,6 +133,31 @@ def test_axes_that_do_not_increase_take_the_host_routine(orc):
     prep.close()
 
 
+@pytest.mark.parametrize("ne", [618, 619])
+def test_many_escape_elements(ne):
+    """Escape ratios of as many elements as the device's line buffer holds,
+    and of one more (the host routine): only the first element's ratios are
+    not zero, so both give what it gives alone."""
+    rng = np.random.default_rng(6)
+    inp = workloads.single_layer_steel(n_photons_line=10, n_interactions=1)
+    inp.nchannels, inp.gain, inp.det_absorbers, inp.crystal = 64, 0.375, [], []
+    prep = api.Prepared(inp)
+    ax = np.array([1.0, 12.0, 24.0])
+    one, keep1 = _ratios([14], ax, ax, ax, rng, False)
+    many, keep = _ratios([14] * ne, ax, ax, ax, rng, False)
+    keep[0][:] = 0.0
+    keep[0][:, :, 0] = keep1[0][:, :, 0]
+    keep[2][:] = keep1[2]
+    ch = np.zeros((2, 64))
+    ch[1] = rng.uniform(1.0, 100.0, 64)
+    ref = api.detector_response(prep, ch, escape_ratios=one, options=_opts())
+    for respond in (api.detector_response, api.detector_response_noalloc):
+        out = respond(prep, ch, escape_ratios=many, options=_opts())
+        # sums of the same terms in another order
+        assert np.abs(out - ref).max() <= 1e-12 * ref.max()
+    prep.close()
+
+
 @pytest.mark.parametrize("respond", [api.detector_response, api.detector_response_noalloc])
 def test_no_order_leaves_nothing_under_way(respond):
     """Calls without an order (only the net-line histories get the detector's

@@ -554,11 +554,16 @@ static int det_findpos(const double *a, int n, double x) {
 /* lines of the K, L1, L2 and L3 vacancies that the reference's escape peaks
  * loop over */
 static const int esc_shell_first[4] = {1, 32, 60, 86}, esc_shell_last[4] = {29, 58, 85, 109};
+static int esc_line_count() {
+  int n = 0;
+  for (int sh = 0; sh < 4; sh++) n += esc_shell_last[sh] - esc_shell_first[sh] + 1;
+  return n;
+}
 
 /* escape peaks with given escape ratios, src/xmi_detector_f.F90:582-809, on
- * the host: for axes that are not increasing, a gain that is not positive
- * or a Compton table of over DET_ESC_WORDS / 4 output energies, which the
- * device routine does not take.  fluo_escape_ratios holds the Fortran array (element, line 1..109, input
+ * the host: for axes that are not increasing, a gain that is not positive, a
+ * Compton table of over DET_ESC_WORDS / 4 output energies or more lines than
+ * DET_ESC_LINES, which the device routine does not take.  fluo_escape_ratios holds the Fortran array (element, line 1..109, input
  * energy) in column-major order; compton_escape_ratios (input, output). */
 static void det_escape(std::vector<double> &ch, const xmi_inputF *in, const xmi_escape_ratios *er) {
   const int nch = (int)ch.size();
@@ -629,6 +634,7 @@ extern "C" uint64_t xmi_engine_current_seed(const xmi_main_options *options);
 #define DET_ESC_WORDS (1l << 20)  /* doubles of the escape tables of one launch */
 #define DET_ESC_AXES (1l << 18)   /* doubles of their axes */
 #define DET_LAYER_BYTES (64 << 10) /* detector layers and their elements */
+#define DET_ESC_LINES (64 << 10)   /* lines of the escape ratios' elements */
 
 /* what one call uploads once: the detector's layers and elements with their
  * atoms, the escape axes and lines */
@@ -670,7 +676,7 @@ static void det_input(const xmi_inputF *in, const xmi_escape_ratios *er, DetInpu
   const double *fe = er->fluo_escape_input_energies, *ci = er->compton_escape_input_energies,
                *co = er->compton_escape_output_energies;
   if (!(gain > 0.0) || !det_increasing(fe, nfe) || !det_increasing(ci, nce) || !det_increasing(co, nco) ||
-      (long)nfe + nce + nco > DET_ESC_AXES) {
+      (long)nfe + nce + nco > DET_ESC_AXES || er->n_elements > DET_ESC_LINES / esc_line_count()) {
     q.host_front = 1;
     return;
   }
@@ -1043,6 +1049,14 @@ extern "C" void xmi_detector_convolute_all(xmi_inputFPtr inputFPtr, double **cha
 #define DET_NOALLOC_MAX_CHANNELS 65536
 #define DET_SCRATCH_BYTES ((size_t)32 << 20)
 static __device__ __align__(256) unsigned char scratch[DET_SCRATCH_BYTES];
+/* one order of the largest spectrum with the largest tables fits (det_carve:
+ * 24 arrays, each rounded up to 256 bytes; its bounds are det_input's) */
+static_assert((size_t)DET_NOALLOC_MAX_CHANNELS * (13 * sizeof(double) + 2 * sizeof(int)) + DET_LAYER_BYTES +
+                      94 * sizeof(xrl_atom) + DET_ESC_LINES * sizeof(DetEscLine) +
+                      (DET_ESC_AXES + DET_ESC_WORDS) * sizeof(double) + (DET_GUIDE + 1) * sizeof(int) +
+                      sizeof(DetTrains) + 24 * 256 <=
+                  DET_SCRATCH_BYTES,
+              "the allocation-free response's buffers fit its array");
 
 #define DET_MAX_DEVICES 64
 static void *g_scratch_ptr[DET_MAX_DEVICES];
