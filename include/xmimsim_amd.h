@@ -443,6 +443,12 @@ void xmi_detector_convolute_all_custom(xmi_inputFPtr inputFPtr, double **channel
                                        xmi_escape_ratios *escape_ratios, int n_interactions_all,
                                        int zero_interaction);
 
+/* xmi_detector_convolute_all keeps the workspaces of its last calls (up to
+ * four, each of at most 64 MB on the device and 64 MB page-locked); this gives
+ * back those that no call is using and returns their bytes (device and
+ * page-locked).  The next call allocates again. */
+int64_t xmi_detector_release_workspaces(void);
+
 /* The same detector response without any device allocation.  No counterpart
  * in the reference: it is for callers that cannot allocate device memory
  * (harnesses that forbid hipMalloc, tight serving loops).  The caller owns

@@ -133,6 +133,28 @@ def test_axes_that_do_not_increase_take_the_host_routine(orc):
     prep.close()
 
 
+def test_workspaces_are_given_back():
+    """What a response keeps for the next call goes with the release, whose
+    repetition finds nothing; a response after it gives the same."""
+    rng = np.random.default_rng(12)
+    inp = workloads.single_layer_steel(n_photons_line=10, n_interactions=4)
+    inp.nchannels, inp.gain = 4096, 0.01
+    prep = api.Prepared(inp)
+    ch = np.zeros((5, 4096))
+    ch[1:] = rng.uniform(0.0, 100.0, (4, 4096))
+    opts = api.default_options(use_escape_peaks=0, use_sum_peaks=1, use_poisson=1, use_default_seeds=1)
+    er, keep = _ratios([14], *(np.linspace(0.1, 24.0, 200) for _ in range(3)), rng, False)
+    api.release_detector_workspaces()
+    a = api.detector_response(prep, ch, escape_ratios=er, options=_opts())  # 8 MB of tables
+    b = api.detector_response(prep, ch, options=opts)
+    # one workspace (the calls came one after another): the tables on both sides, and the spectra
+    assert 2 * (8 << 20) < api.release_detector_workspaces() <= 128 << 20
+    assert api.release_detector_workspaces() == 0
+    assert np.array_equal(api.detector_response(prep, ch, escape_ratios=er, options=_opts()), a)
+    assert np.array_equal(api.detector_response(prep, ch, options=opts), b)
+    prep.close()
+
+
 @pytest.mark.parametrize("ne", [618, 619])
 def test_many_escape_elements(ne):
     """Escape ratios of as many elements as the device's line buffer holds,

@@ -146,6 +146,7 @@ EXPORTED_SYMBOLS = [
     "xmi_solid_angle_calculation_cl", "xmi_free_solid_angle", "xmi_hits_per_single", "xmi_main_msim",
     "xmi_free", "xmi_set_seed", "xmi_msim_get_stats", "xmi_msim_last_error", "xmi_msim_set_profiling",
     "xmi_msim_get_layer_events", "xmi_msim_set_launch", "xmi_msim_get_launch", "xmi_provider_active_lines", "xmi_detector_convolute_all",
+    "xmi_detector_release_workspaces",
     "xmi_detector_convolute_all_custom", "xmi_surrogate_create", "xmi_surrogate_train_step", "xmi_main_msim_batch",
     "xmi_tables_set_device", "xmi_tables_copy", "xmi_escape_ratios_calculation", "xmi_free_escape_ratios",
     "xmi_get_default_escape_ratios_options", "xmi_input_read_from_xml_file", "xmi_input_read_from_xml_string",
@@ -613,6 +614,14 @@ def detector_response(prep: "Prepared", channels: np.ndarray, var_red: Optional[
         out[k] = np.ctypeslib.as_array(conv[k], shape=(nch,))
         lib.xmi_free(conv[k])
     return out
+
+
+def release_detector_workspaces() -> int:
+    """Gives back the device and page-locked memory that detector_response
+    keeps for its next calls; returns the bytes."""
+    lib = load_library()
+    lib.xmi_detector_release_workspaces.restype = C.c_int64
+    return lib.xmi_detector_release_workspaces()
 
 
 def detector_response_noalloc(prep: "Prepared", channels: np.ndarray, var_red: Optional[np.ndarray] = None,

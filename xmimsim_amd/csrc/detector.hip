@@ -940,7 +940,11 @@ static int det_convolute(const xmi_inputF *in, double **channels_noconv, double 
 /* workspaces of xmi_detector_convolute_all: a stream, device memory and
  * page-locked staging, each taken by one call at a time.  At most
  * DET_POOL wait for the next call, with at most DET_KEEP bytes each; the
- * others are released when their call ends. */
+ * others are released when their call ends, the waiting ones by
+ * xmi_detector_release_workspaces.  A workspace's memory is used on its own
+ * stream only, which therefore need not be ordered with the null stream: it
+ * is created non-blocking, so that a waiting workspace does not take part in
+ * other work's synchronisations. */
 #define DET_POOL 4
 #define DET_KEEP ((size_t)64 << 20)
 struct DetWork {
@@ -975,7 +979,7 @@ static DetWork *det_take_work(size_t bytes, hipError_t *e) {
     w = new DetWork();
     w->dev = dev;
     w->stage.locked = true;
-    *e = hipStreamCreate(&w->st);
+    *e = hipStreamCreateWithFlags(&w->st, hipStreamNonBlocking);
   }
   if (*e == hipSuccess && w->n < bytes) {
     if (w->block) (void)hipFree(w->block);
@@ -1000,6 +1004,20 @@ static void det_give_work(DetWork *w, bool ok) {
   }
   (void)hipStreamSynchronize(w->st);
   delete w;
+}
+
+extern "C" int64_t xmi_detector_release_workspaces(void) {
+  std::vector<DetWork *> idle;
+  int64_t bytes = 0;
+  {
+    std::lock_guard<std::mutex> g(g_pool_mutex);
+    idle.swap(*g_det_pool);
+  }
+  for (DetWork *w : idle) {
+    bytes += (int64_t)(w->n + w->stage.n);
+    delete w; /* their calls have synchronised */
+  }
+  return bytes;
 }
 
 /* orders of one group: as many as `bytes` of device memory hold, at least one */
