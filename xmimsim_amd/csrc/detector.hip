@@ -733,25 +733,29 @@ static size_t det_carve(void *base, size_t nch, size_t n_ord, const DetInput &q,
   return c.n;
 }
 
-/* host memory of the copies: page-locked in a workspace, else a vector */
+/* host memory of the copies: page-locked in a workspace, else the heap's,
+ * not cleared (a call writes what it copies; clearing the 8 MB of the escape
+ * tables' part took the allocation-free response of 1024 channels from 0.25 to
+ * 0.30 ms, its first call from 0.6 to 2.2 ms) */
 struct DetStage {
-  std::vector<char> v;
   char *p = nullptr;
   size_t n = 0;
   bool locked = false;
-  hipError_t ensure(size_t bytes) {
-    if (bytes <= n) return hipSuccess;
-    if (!locked) {
-      v.resize(bytes);
-      p = v.data();
-      n = bytes;
-      return hipSuccess;
-    }
-    if (p) (void)hipHostFree(p);
+  ~DetStage() { release(); }
+  void release() {
+    if (p && locked) (void)hipHostFree(p);
+    else free(p);
     p = nullptr;
     n = 0;
-    const hipError_t e = hipHostMalloc((void **)&p, bytes, hipHostMallocDefault);
+  }
+  hipError_t ensure(size_t bytes) {
+    if (bytes <= n) return hipSuccess;
+    release();
+    hipError_t e = hipSuccess;
+    if (locked) e = hipHostMalloc((void **)&p, bytes, hipHostMallocDefault);
+    else if (!(p = (char *)malloc(bytes))) e = hipErrorOutOfMemory;
     if (e == hipSuccess) n = bytes;
+    else p = nullptr;
     return e;
   }
 };
@@ -955,7 +959,7 @@ struct DetWork {
   DetStage stage;
   ~DetWork() {
     if (block) (void)hipFree(block);
-    if (stage.p) (void)hipHostFree(stage.p);
+    stage.release();
     if (st) (void)hipStreamDestroy(st);
   }
 };
