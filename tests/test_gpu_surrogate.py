@@ -40,6 +40,53 @@ def test_forward_matches_reference():
     s.close()
 
 
+def _mt64(seed):
+    """Words of the 64-bit Mersenne Twister (T. Nishimura, "Tables of 64-bit
+    Mersenne Twisters", ACM TOMACS 10 (2000) 348-357)."""
+    M = (1 << 64) - 1
+    x = [seed & M]
+    for i in range(1, 312):
+        x.append((6364136223846793005 * (x[-1] ^ (x[-1] >> 62)) + i) & M)
+    while True:
+        for i in range(312):
+            y = (x[i] & (M << 31) & M) | (x[(i + 1) % 312] & 0x7FFFFFFF)
+            x[i] = x[(i + 156) % 312] ^ (y >> 1) ^ (0xB5026F5AA96619E9 if y & 1 else 0)
+        for y in list(x):
+            y ^= (y >> 29) & 0x5555555555555555
+            y ^= (y << 17) & 0x71D67FFFEDA60000 & M
+            y ^= (y << 37) & 0xFFF7EEE000000000 & M
+            yield y ^ (y >> 43)
+
+
+def test_initial_weights_are_the_polar_method_on_the_seed():
+    """He-normal weights, drawn layer by layer in pairs from one engine; a
+    pair's second value is dropped at the end of a layer of odd count."""
+    f = np.float32
+    dims, nets, seed = (3, 64, 192), 3, 77
+    from xmimsim_amd.surrogate import Surrogate
+    s = Surrogate(n_nets=nets, dims=dims, max_batch=64, seed=seed)
+    P = s.get_params()
+    words = _mt64(seed)
+    for l in range(2):
+        n = nets * dims[l + 1] * dims[l]
+        ref = np.zeros(n + 1, np.float64)
+        for k in range(0, n, 2):
+            while True:
+                x, y = (2.0 * float(f(next(words)) * f(2.0 ** -64)) - 1.0 for _ in range(2))
+                r2 = float(f(f(x) * f(x)) + f(f(y) * f(y)))
+                if 0.0 < r2 <= 1.0:
+                    break
+            m = np.sqrt(-2.0 * np.log(r2) / r2)
+            ref[k], ref[k + 1] = y * m, x * m
+        ref = (ref[:n] * np.sqrt(2.0 / dims[l])).reshape(nets, dims[l + 1], dims[l])
+        for e in range(nets):
+            W, b = s.unpack(P[e])[l]
+            # a handful of f32 roundings
+            assert np.allclose(W[:, :dims[l]], ref[e], rtol=1e-6, atol=0.0)
+            assert not W[:, dims[l]:].any() and not b.any()
+    s.close()
+
+
 def test_gradients_match_reference():
     import surrogate_ref as R
     rng = np.random.default_rng(11)
