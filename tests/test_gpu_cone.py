@@ -32,3 +32,32 @@ def test_cone_hits_equal_the_oracle(orc, hits, coll, y):
     assert np.abs(g - og).max() <= (1e-9 if coll else 1e-12) * og.max()
     assert g.max() > 0
     prep.close()
+
+
+@pytest.mark.parametrize("y,area", [(2.0, 0.2), (2.0, 0.05), (5.0, 0.3)])
+def test_cone_size_rounds_as_the_cosine_of_the_angle(y, area):
+    """Hits divide the cone's size, 2 pi (1 - cos) with the rounded cosine of
+    the larger half angle, into equal parts: a cell is a whole number of them
+    to the last bits.  Far from the window an ulp of the cosine is 1e-14 of the
+    size and more."""
+    hits = 3
+    inp = workloads.single_layer_steel(n_photons_line=10)
+    inp.area_detector, inp.p_detector_window = area, (0.0, y, 100.0)
+    prep = api.Prepared(inp)
+    print("cone size", y, area, flush=True)
+    g, r, t = prep.compute_solid_angle(hits_per_single=hits, seed=5)
+    L = np.longdouble
+    R, rr, tt = L(math.sqrt(area / math.pi)), L(r)[None, :], L(t)[:, None]
+    a1 = np.arctan(R * np.sin(tt) / (rr - R * np.cos(tt)))
+    apex = np.maximum(np.arctan(R / rr), np.where(a1 <= 0, a1 + 4 * np.arctan(L(1)), a1))
+    om = 1.0 - np.cos(apex).astype(np.float64)
+    on = (g > 0) & (om < 0.05)
+    n = g[on] * hits / (2.0 * np.pi * om[on])
+    # six roundings are 7e-16, half an ulp of the cosine at least 2e-15.  In
+    # double, cos(atan()) rounds the other way in 0.6 to 1.6 % of these cells,
+    # a quotient of two roundings in 40 %: a tenth of
+    # that is the line
+    off = np.abs(n - np.rint(n)) > 1.5e-15 * n
+    print("cells", on.mean(), "rounded otherwise", off.mean(), flush=True)
+    assert on.mean() > 0.3 and off.mean() < 0.04
+    prep.close()

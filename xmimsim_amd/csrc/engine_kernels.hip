@@ -279,7 +279,7 @@ __device__ __forceinline__ double d_table(int uniform, const double *arr, const 
  * root and one sine per trial, no division.  q = l1 v2 - h v1 is linear in c1
  * and x; its two factors are formed once per cone.  Bound by vector issue,
  * about 40 % of it the Philox multiplies: 1024 x 1024 cells of 5000 trials
- * take 13.9 ms (25.7 ms with the general sine and cosine, two divisions and
+ * take 14.0 ms (25.7 ms with the general sine and cosine, two divisions and
  * two square roots per trial), the off-grid points of a batch 31 us (54). */
 struct SaCone {
   double cone_sa;
@@ -332,14 +332,17 @@ __device__ __forceinline__ int d_sa_setup(const SaGeom g, double r1, double thet
     st = s1;
     fcbr = R;
   }
-  /* the larger of the cone's two half angles, by its cosine: atan(fcbr / r)
-   * and atan(fcbr sin / (r - fcbr cos)), the latter in (0, pi] */
-  const double cb = r / sqrt(r * r + fcbr * fcbr);
-  const double ay = fcbr * st, ax = r - fcbr * ct;
-  const double ca = ay > 0.0 ? ax / sqrt(ax * ax + ay * ay) : -1.0;
-  const double cos_apex = cb < ca ? cb : ca;
-  c->cone_sa = 2.0 * ENG_PI * (1.0 - cos_apex);
-  c->k = (1.0 - cos_apex) * (1.0 / 4294967296.0);
+  /* the larger of the cone's two half angles, as the reference takes it: the
+   * cone's size is one minus the rounded cosine, an ulp of which is 1e-14 of
+   * the size in cells far from the window.  (A quotient for the cosine would save
+   * 1 % of the grid's time; its roundings fall to the other side in 40 % of
+   * those cells.) */
+  const double beta = atan(fcbr / r);
+  double alpha = atan(fcbr * st / (r - fcbr * ct));
+  if (alpha <= 0.0) alpha += ENG_PI;
+  const double om = 1.0 - cos(beta > alpha ? beta : alpha);
+  c->cone_sa = 2.0 * ENG_PI * om;
+  c->k = om * (1.0 / 4294967296.0);
   c->k2 = 0.5 * c->k;
   c->st = st;
   c->ct = ct;
