@@ -325,7 +325,7 @@ void xmi_msim_set_profiling(int on);
  * take the defaults.  Applies to the calls that start after it; not to be
  * changed while a call runs. */
 typedef struct _xmi_msim_launch {
-  int batch_log2; /* histories per batch 2^batch_log2, 12..21 (default: 2^23) */
+  int batch_log2; /* histories per batch 2^batch_log2, 12..23 (default: 23) */
   int use_graph;  /* 1: capture one batch's launches in a HIP graph, replayed per batch; each replay pops its
                      batch from a device batch queue */
   int lines_kp;   /* photons per lane of the estimator's line kernel: 2..4 up to 4 layers (default 4 up to 3

@@ -10,10 +10,13 @@ def test_set_launch_ranges(lib):
     try:
         api.set_launch(batch_log2=18, use_graph=1, lines_kp=4, wg_per_cu=3)
         assert api.get_launch() == {"batch_log2": 18, "use_graph": 1, "lines_kp": 4, "wg_per_cu": 3}
-        for bad in ({"batch_log2": 11}, {"batch_log2": 22}, {"lines_kp": 5}, {"use_graph": 2}, {"wg_per_cu": -1}):
+        for bad in ({"batch_log2": 11}, {"batch_log2": 24}, {"lines_kp": 5}, {"use_graph": 2}, {"wg_per_cu": -1}):
             with pytest.raises(ValueError):
                 api.set_launch(**bad)
         assert api.get_launch()["batch_log2"] == 18  # a refused shape leaves the last one
+        for batch in (12, 21, 22, 23):  # the largest is the default, by its name
+            api.set_launch(batch_log2=batch)
+            assert api.get_launch()["batch_log2"] == batch
     finally:
         api.set_launch()
     assert api.get_launch() == autotune.DEFAULT

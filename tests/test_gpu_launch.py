@@ -107,6 +107,39 @@ def test_launch_shapes_agree(launch):
     prep.close()
 
 
+@pytest.mark.parametrize("n_layers", [1, 3])
+def test_default_batches_equal_small_ones(n_layers):
+    """One full batch of 2^23 histories, whose layer scan spans 128 segments
+    (two waves of k_layer_base), and one of an odd rest: the events of every
+    layer are those of 2^18 batches (at most 4 segments), the sums agree as
+    between other shapes, and the default's name gives the default's bits."""
+    inp = _steel(2 ** 23 + 600001)
+    inp.n_interactions_trajectory = 2
+    if n_layers == 3:  # thin, so that photons reach the last
+        steel = inp.layers[0]
+        inp.layers = [api.Layer([13], [1.0], 2.7, 1e-3), api.Layer(steel.Z, steel.weight, steel.density, 1e-3),
+                      api.Layer([22, 29], [0.5, 0.5], 5.0, 1e-3)]
+        inp.reference_layer = 2
+    prep = api.Prepared(inp)
+    prep.compute_solid_angle(hits_per_single=200, seed=3)
+
+    def run(**launch):
+        print("batches", n_layers, launch, flush=True)
+        (ch, vr, _, s), st = _run(prep, 17, **launch)
+        return ch, vr, s.histories, st.batches, prep.layer_events
+
+    ch0, vr0, h0, b0, ev0 = run()
+    ch1, vr1, h1, b1, ev1 = run(batch_log2=18)
+    ch2, vr2, _, b2, ev2 = run(batch_log2=23)
+    assert h0 == h1 == inp.n_photons_line and (b0, b1, b2) == (2, 35, 2)
+    assert ev0 == ev1 == ev2 and all(e > 0 for e in ev0)
+    assert np.array_equal(ch0, ch2) and np.array_equal(vr0, vr2)
+    for a, b in ((ch1, ch0), (vr1, vr0)):
+        scale = np.abs(b).max()
+        assert np.all(np.abs(a - b) <= 1e-12 * np.maximum(np.abs(b), 1e-3 * scale))
+    prep.close()
+
+
 def test_autotune_picks_a_shape_of_its_space(tmp_path):
     prep = api.Prepared(_steel(20000))
     prep.compute_solid_angle(hits_per_single=200, seed=3)

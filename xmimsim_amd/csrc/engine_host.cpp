@@ -45,8 +45,8 @@ extern "C" int xmi_msim_set_launch(const xmi_msim_launch *l) {
     xmi_set_error("xmi_msim_set_launch: NULL argument");
     return 0;
   }
-  if (l->batch_log2 && (l->batch_log2 < 12 || l->batch_log2 > 21)) {
-    xmi_set_error("xmi_msim_set_launch: batch_log2 %d outside 12..21", l->batch_log2);
+  if (l->batch_log2 && (l->batch_log2 < 12 || l->batch_log2 > ENG_BATCH_LOG2)) {
+    xmi_set_error("xmi_msim_set_launch: batch_log2 %d outside 12..%d", l->batch_log2, ENG_BATCH_LOG2);
     return 0;
   }
   if (l->lines_kp < 0 || l->lines_kp > 4 || l->wg_per_cu < 0 || l->wg_per_cu > 32 || l->use_graph < 0 ||
