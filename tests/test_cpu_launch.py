@@ -34,8 +34,13 @@ def test_sample_input_scales_budgets():
 
 
 def test_lines_kp_candidates():
-    assert autotune.lines_kp_candidates(1) == autotune.lines_kp_candidates(4) == (2, 4)
-    assert autotune.lines_kp_candidates(5) == (1,)
+    """Every instance of the line kernel but the default, which is timed first
+    anyway (4 photons per lane up to three layers, 3 up to five, 2 up to
+    eight, 1 beyond)."""
+    assert autotune.lines_kp_candidates(1) == autotune.lines_kp_candidates(3) == (2, 3)
+    assert autotune.lines_kp_candidates(4) == (2, 4)
+    assert autotune.lines_kp_candidates(5) == (1, 2)
+    assert autotune.lines_kp_candidates(6) == autotune.lines_kp_candidates(8) == (1,)
     assert autotune.lines_kp_candidates(12) == ()
 
 
@@ -56,7 +61,7 @@ def test_descent_finds_the_separable_optimum():
     assert len(calls) == 4 + 2 + 2 + 2 + 1
 
 
-def test_tune_caches_by_signature(lib, tmp_path):
+def test_tune_caches_by_signature(lib, tmp_path, monkeypatch):
     prep = api.Prepared(workloads.single_layer_steel(n_photons_line=1000))
     path = str(tmp_path / "launch.json")
     seen = []
@@ -66,10 +71,14 @@ def test_tune_caches_by_signature(lib, tmp_path):
         return 10.0 - shape["lines_kp"] - (shape["batch_log2"] == 19)
 
     best, table = autotune.tune(prep, cache=path, timer=timer)
-    assert best == {"batch_log2": 19, "use_graph": 0, "lines_kp": 4, "wg_per_cu": 0}
+    assert best == {"batch_log2": 19, "use_graph": 0, "lines_kp": 3, "wg_per_cu": 0}
+    assert {r["launch"]["batch_log2"] for r in table} == {0, 22, 21, 20, 19}
     assert len(table) == len(seen) and best in [r["launch"] for r in table]
     again, rows = autotune.tune(prep, cache=path, timer=timer)
     assert again == best and rows == [] and len(seen) == len(table)
+    with monkeypatch.context() as m:  # shapes of another library are timed again
+        m.setattr(autotune, "build_id", lambda: "another")
+        assert len(autotune.tune(prep, cache=path, timer=timer)[1]) == len(table)
     brute = api.Prepared(workloads.single_layer_steel(n_photons_line=1000),
                          options=api.default_options(use_variance_reduction=0))
     b, t = autotune.tune(brute, cache=path, timer=timer)

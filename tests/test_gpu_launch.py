@@ -91,7 +91,7 @@ def test_graph_batch_engines():
     grid.close()
 
 
-@pytest.mark.parametrize("launch", [{"batch_log2": 15}, {"lines_kp": 2}, {"lines_kp": 4}, {"wg_per_cu": 2},
+@pytest.mark.parametrize("launch", [{"batch_log2": 15}, {"lines_kp": 2}, {"lines_kp": 3}, {"lines_kp": 4}, {"wg_per_cu": 2},
                                     {"batch_log2": 16, "lines_kp": 4, "wg_per_cu": 3, "use_graph": 1}])
 def test_launch_shapes_agree(launch):
     """Other shapes regroup the estimator's per-wave sums: every channel and
@@ -104,6 +104,24 @@ def test_launch_shapes_agree(launch):
     for a, b in ((ch1, ch0), (vr1, vr0)):
         scale = np.abs(b).max()
         assert np.all(np.abs(a - b) <= 1e-12 * np.maximum(np.abs(b), 1e-3 * scale)), launch
+    prep.close()
+
+
+@pytest.mark.parametrize("n_layers,kp", [(3, 2), (3, 3), (4, 2), (4, 4), (5, 1), (5, 2), (7, 1)])
+def test_photons_per_lane_agree(n_layers, kp):
+    """Every other instance of the line kernel at its layer counts: within
+    1e-12 of the default's."""
+    inp = _steel(100000)
+    Zs = ([13], [26, 24], [22, 29], [30], [14, 20], [28], [25, 40])
+    inp.layers = [api.Layer(list(Z), [1.0 / len(Z)] * len(Z), 2.0 + k, 1e-3) for k, Z in enumerate(Zs[:n_layers])]
+    inp.reference_layer = 1
+    prep = api.Prepared(inp)
+    assert kp in autotune.lines_kp_candidates(n_layers)
+    prep.compute_solid_angle(hits_per_single=200, seed=3)
+    print("photons per lane", n_layers, kp, flush=True)
+    (_, vr0, _, _), _ = _run(prep, 13)
+    (_, vr1, _, _), _ = _run(prep, 13, lines_kp=kp)
+    assert vr0.sum() > 0 and np.all(np.abs(vr1 - vr0) <= 1e-12 * np.maximum(np.abs(vr0), 1e-3 * np.abs(vr0).max()))
     prep.close()
 
 

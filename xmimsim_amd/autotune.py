@@ -18,11 +18,12 @@ The search is a coordinate descent from the default shape in that order, each
 parameter over its candidates with the others fixed, every candidate timed
 twice (device time of the transport, the minimum kept).  The choice is cached
 per workload signature (layers, elements per layer, lines and intervals,
-interactions, options) in a JSON file.  Shapes change the estimator's sums
+interactions, options) and library build in a JSON file.  Shapes change the estimator's sums
 only in their last bits (the order of the per-wave sums), so a tuned run
 agrees with the default shape's to about 1e-12 relative.
 """
 import copy
+import hashlib
 import json
 import os
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -33,19 +34,24 @@ DEFAULT = {"batch_log2": 0, "use_graph": 0, "lines_kp": 0, "wg_per_cu": 0}
 CACHE = os.path.join(os.path.expanduser("~"), ".cache", "xmimsim_amd", "launch.json")
 
 
-def _nl_bound(n_layers: int) -> int:
-    for b in (1, 2, 4, 8):
-        if n_layers <= b:
-            return b
-    return 16
-
-
 def lines_kp_candidates(n_layers: int) -> Tuple[int, ...]:
     """Photons per lane, besides the default, that the line kernel is built
     for at this layer count (default 4 up to three layers, 3 up to five, 2 up
     to eight, 1 beyond)."""
-    nl = _nl_bound(n_layers)
-    return (2, 4) if nl <= 4 else ((1,) if nl <= 8 else ())
+    if n_layers <= 3:
+        return (2, 3)
+    if n_layers <= 4:
+        return (2, 4)
+    if n_layers <= 5:
+        return (1, 2)
+    return (1,) if n_layers <= 8 else ()
+
+
+def build_id() -> str:
+    """Content of the library the shapes were timed with: other kernels or
+    defaults are another library."""
+    with open(api.load_library()._name, "rb") as f:
+        return hashlib.sha1(f.read()).hexdigest()[:16]
 
 
 def signature(prep: "api.Prepared") -> str:
@@ -111,17 +117,17 @@ def descend(measure, steps) -> Dict[str, int]:
 
 
 def tune(prep: "api.Prepared", sample_histories: int = 1 << 23, seed: int = 1,
-         batch_sizes: Sequence[int] = (20, 19), wg_per_cu: Sequence[int] = (2, 3),
+         batch_sizes: Sequence[int] = (22, 21, 20, 19), wg_per_cu: Sequence[int] = (2, 3),
          cache: Optional[str] = CACHE, repeats: int = 2, timer=None) -> Tuple[Dict[str, int], List[Dict]]:
     """The fastest launch shape for prep's workload and the table of timed
     shapes ({"launch": shape, "ms": device time}); (shape, []) when the
-    cache holds the signature.  Candidates are tried besides the defaults
+    cache holds the signature for this library.  Candidates are tried besides the defaults
     (2^23 histories per batch, kernel by kernel, the default photons per lane
     and the occupancy's workgroups).  The engine's launch shape in force
     before the call is restored; apply the result with
     api.set_launch(**shape).  timer(shape) -> ms replaces the timed runs
     (tests of the search)."""
-    key = f"{signature(prep)};sample={sample_histories}"
+    key = f"{signature(prep)};sample={sample_histories};build={build_id()}"
     data = _load_cache(cache)
     if key in data:
         return data[key]["launch"], []
