@@ -245,16 +245,6 @@ __device__ __forceinline__ void fx_add_global(unsigned long long *bin, double v,
   if (hi) atomicAdd(bin + 1, hi);
 }
 
-__device__ __forceinline__ void fx_add_shared(unsigned long long *bin, double v, int shift) {
-  unsigned long long lo, hi;
-  fx_split(v, shift, &lo, &hi);
-  if (lo) {
-    unsigned long long old = atomicAdd(bin, lo);
-    if (old + lo < old) hi += 1ull;
-  }
-  if (hi) atomicAdd(bin + 1, hi);
-}
-
 /* adds a 128-bit (lo,hi) pair held elsewhere into a global bin */
 __device__ __forceinline__ void fx_merge_global(unsigned long long *bin, unsigned long long lo, unsigned long long hi) {
   if (lo) {

@@ -36,7 +36,8 @@
 /* histories per batch unless the launch shape says otherwise: every kernel of
  * an order ends with a part-filled round of workgroups, and the scan, list
  * and reset launches cost the same for any size, so the batch is as large as
- * 2.3 GB of photon records (three layers) make it */
+ * 1.85 GB of records make it (three layers: 140 bytes of photon state and 80
+ * of the estimator a slot) */
 #define ENG_BATCH_LOG2 23
 /* segments of the per-wave layer-count scan (k_layer_scan, d_layer_list):
  * the waves of the largest batch, one thread per slot */
@@ -83,7 +84,7 @@ struct SourceTable {
   const uint64_t *run0;       /* [n] the descriptors' run0, for the search */
   int n;
   const double *line_mus;     /* [n_sources][n_layers] mus at the line energy */
-  const double *exc_layers;   /* per absorber: density, thickness, n_el, Z[n_el], w[n_el] */
+  const double *exc_layers;   /* per absorber: density, thickness, n_el, place in exc_atoms[n_el], w[n_el] */
   int n_exc;
   const xrl_atom *exc_atoms;  /* [95] indexed by Z */
 };

@@ -1076,16 +1076,6 @@ __global__ void __launch_bounds__(ENG_SCAN_NSEG) k_layer_base(EngineParams P, in
  * register arrays have compile-time indices only (NL bounds the layer count).  Tallies are 128-bit fixed point, privatised in LDS when they fit;
  * integer adds commute, so totals do not depend on the order of the adds. */
 
-__device__ __forceinline__ double d_wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
-
-__device__ __forceinline__ void d_tally_wave(unsigned long long *bin, double v, int shift) {
-  double s = d_wave_sum(v);
-  if (__lane_id() == 0 && s > 0.0) fx_add_global(bin, s, shift);
-}
-
 __device__ __forceinline__ double d_readlane(double v, int lane) {
   long long b = __double_as_longlong(v);
   unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
@@ -1103,22 +1093,11 @@ __device__ __forceinline__ double d_dpp0(double v) {
   return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
 }
 
-/* sum of v over the wavefront, in a fixed order (row prefix sums, then the
- * row totals), returned wave-uniform: DPP moves keep the reduction in the
- * VALU, without the LDS round trips of a shuffle butterfly */
-__device__ __forceinline__ double d_wave_total(double v) {
-  v += d_dpp0<0x111, 0xf>(v); /* row_shr:1 */
-  v += d_dpp0<0x112, 0xf>(v); /* row_shr:2 */
-  v += d_dpp0<0x114, 0xf>(v); /* row_shr:4 */
-  v += d_dpp0<0x118, 0xf>(v); /* row_shr:8: lane 15 of a row holds its sum */
-  v += d_dpp0<0x142, 0xa>(v); /* row_bcast:15 into rows 1 and 3 */
-  v += d_dpp0<0x143, 0xc>(v); /* row_bcast:31 into rows 2 and 3: lane 63 holds the total */
-  return d_readlane(v, 63);
-}
-
-/* the wavefront's sums of a and of b, in a fixed order: the halves exchanged
- * first (a's sums then live in lanes 0 to 31, b's in 32 to 63), so that one
- * row reduction serves both */
+/* the wavefront's sums of a and of b, in a fixed order (row prefix sums, then
+ * the row totals), returned wave-uniform: the halves exchanged first (a's sums
+ * then live in lanes 0 to 31, b's in 32 to 63), so that one row reduction
+ * serves both.  DPP moves keep it in the VALU, without the LDS round trips of a
+ * shuffle butterfly */
 __device__ __forceinline__ void d_wave_total2(double a, double b, double *ta, double *tb) {
   const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
   const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
@@ -2463,8 +2442,8 @@ k_interact_brute(EngineParams P, PhotonSoA S, int n) {
  * the forced step of every interacted photon normalises its input energy.
  * One thread per queue entry of the three interaction queues. */
 
-/* integer sum of v over the wavefront, wave-uniform (the steps of
- * d_wave_total) */
+/* integer sum of v over the wavefront, wave-uniform (the row steps of
+ * d_wave_total2, then row_bcast:31 into rows 2 and 3: lane 63 holds it) */
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ unsigned long long d_dpp0_u64(unsigned long long v) {
   const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, CTRL, ROW_MASK, 0xf, true);
