@@ -117,26 +117,26 @@ def _fp64_weights():
 
 
 def vr_flops_per_event(w):
-    """Algorithmic FP64 flops of the scatter and line phases of one
-    detection-weight evaluation (FMA = 2, add/mul = 1, math routines weighted
-    as in profiles/fp64_op_weights.json):
-      lines    per line: 2L (attenuation sum) + exp + 3 (wf * P_shell * g *
-               e^-mu) + 1 (sum over photons); per event 3 + div (g)
-      scatter  per event: sin, cos (theta), cos (phi), sin (theta/2) and 12 +
-               div (Thomson and Klein-Nishina factors); per element:
-               Rayleigh 5 div + 11 (form factor, cross section, weight,
-               channel); Compton per Doppler draw 3 div + 20 (bounds of the
-               accepted momenta, their CDF values, the draw, the energy),
-               then log + exp + 4 (energy context) + 7L (attenuation) + exp
-               + 4 div + 12 (scattering function, cross section, weight,
-               channel)"""
+    """FP64 flops of the scatter and line kernels for one detection-weight
+    evaluation, counted on what they execute for it (FMA = 2, add/mul = 1,
+    function forms weighted as in profiles/fp64_op_weights.json); L = layers on
+    the path, without the layers of the instance that it does not cross:
+      lines    per line: 2L - 1 (attenuation sum) + exp_unit + 2 (shell and
+               weight factor, sum over photons); per event 2 rsqrt + 2 div + 8
+               (weight factor with E^-11/4)
+      scatter  per event: 3 rcp + sqrt + 35 + 2L (Thomson and Klein-Nishina
+               factors, bounds of the accepted momenta, layers' factors); per
+               element: rcp + 38 (profile CDFs at the bounds, form factor,
+               scattering function, weights); per Compton draw rcp + 17 (the
+               word's place in the inverse table, the energy), then energy +
+               6L (attenuation) + exp64 + 3 (weight, channel)"""
     wt = _fp64_weights()
-    ex, lg, dv, sn, cs = wt["exp"], wt["log"], wt["div"], wt["sin"], wt["cos"]
     E, EL, tr = w["elements"], w["element_layers"], w["doppler_trials"]
     A, AL = w["lines"], w["line_layers"]
-    return {"lines": A * (ex + 4) + 2 * AL + 3 + dv,
-            "scatter": (2 * sn + 2 * cs + 12 + dv + E * (5 * dv + 11) + tr * (3 * dv + 20)
-                        + E * (lg + 2 * ex + 4 * dv + 16) + 7 * EL)}
+    L = AL / A
+    return {"lines": A * (wt["exp_unit"] + 1) + 2 * AL + 2 * wt["rsqrt"] + 2 * wt["div"] + 8,
+            "scatter": (3 * wt["rcp"] + wt["sqrt"] + 35 + 2 * L + E * (wt["rcp"] + 38) + tr * (wt["rcp"] + 17)
+                        + E * (wt["energy"] + wt["exp64"] + 3) + 6 * EL)}
 
 
 def cpu_baseline(args, prep_gpu):
@@ -180,6 +180,16 @@ def _measured_traffic(workload):
         return {}
     with open(path) as f:
         return {k: v["bytes_per_launch"] for k, v in json.load(f)["kernels"].items()}
+
+
+def _measured_issue(workload):
+    """Share of the cycles in which a kernel's vector ALUs issue, from the
+    committed SQ counters of this workload, if there are any."""
+    path = os.path.join(ROOT, "profiles", f"counters_{workload}.json")
+    if not os.path.exists(path):
+        return {}
+    with open(path) as f:
+        return {k: v["valu_busy"] for k, v in json.load(f)["kernels"].items()}
 
 
 def apply_launch(args, prep=None):
@@ -578,9 +588,11 @@ def main():
                  "step": "k_step", "interactions": "k_interact"}
         traffic = _measured_traffic(args.workload)
         # the dominant kernel of the step: the scatter and line kernels are
-        # bound by FP64 vector issue and gather latency (their table reads hit
-        # the caches: the measured HBM traffic is far below the algorithmic
-        # bytes), so their roofline is FP64 at the vector peak
+        # bound by vector issue and gather latency (their table reads hit the
+        # caches: the measured HBM traffic is far below the algorithmic bytes),
+        # so their roofline is FP64 at the vector peak.  The peak counts two
+        # flops an instruction; the kernels' conversions, rounding, table
+        # indices and LDS traffic issue beside their additions and products
         dom = max(("scatter", "lines"), key=lambda k: prof[k])
         sec = prof[dom] * 1e-3 / launches
         achieved = fpe[dom] * ev_launch / sec / 1e12
@@ -606,6 +618,8 @@ def main():
                     "events": events, "events_per_launch": round(ev_launch), "launches": int(launches),
                     "work_per_event": {k: round(v, 4) for k, v in work.items()},
                     "hbm_measured": hbm,
+                    # share of the cycles with vector issue, by the SQ counters of the profile
+                    "valu_busy_measured": _measured_issue(args.workload),
                     # both estimator kernels against the FP64 peak, by their counted flops
                     "fp64_frac_estimator": {names[k]: round(fpe[k] * ev_launch / (prof[k] * 1e-3 / launches)
                                                             / 1e12 / FP64_PEAK_TFLOPS, 4)
